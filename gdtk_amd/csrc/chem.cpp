@@ -153,6 +153,7 @@ void build_chemdev(const gdtk_tpg_gas& g, const gdtk_mechanism& m, ChemDev& cd, 
             }
         }
     }
+    cd.walk = mechanism_walk(cd);
     if (!(m.T_lower < m.T_upper)) throw Error(GDTK_ERR_ARG, "tempLimits lower must be below upper");
     cd.T_lower = m.T_lower;
     cd.T_upper = m.T_upper;

@@ -66,12 +66,81 @@ struct RateRow {
     int pad_[3];
 };
 
+// How the rate code walks a mechanism (chosen on the host, mechanism_walk): its species lists,
+// the rows above, or code in which the structure of the mechanism is known at compile time.
+enum ChemWalk : int { WALK_LIST = 0, WALK_ROWS = 1, WALK_AIR5_PARK = 2, WALK_AIR5_GUPTA = 3, WALK_N2_PAIR = 4 };
+constexpr int NUM_WALKS = 5;
+
+// A species' code word in a row: its exponent as reactant and product, and whether it is in the
+// third-body list.
+constexpr int row_code(int reac, int prod, int third) {
+    return reac | (prod << 2) | (((prod - reac) & 15) << 4) | (third << 8);
+}
+
+// Mechanism structures with rate code of their own: which species react in what order and
+// which act as third bodies, no rates and no efficiencies.  They are the structures of the
+// mechanisms that the package ships: dissociation of 5-species air (N2, O2, NO, N, O) with the
+// two Zeldovich exchanges, the same with N2 + N <=> 3 N apart, and dissociating nitrogen (N2, N).
+// A row walk spends most of its instructions on the selects that the code words steer (of 750
+// a rate evaluation of air, 60 are arithmetic) and waits for each row's scalar loads; with the
+// structure known both go: 1048576 cells of air over 1e-7 s (63e6 step attempts) integrate in
+// 2.6 ms instead of 8.4, 3001 cells with at most 49 attempts each in 0.16 ms instead of 0.77 (with the
+// step algebra of alpha_qss_step).
+template <int WALK>
+struct MechShape {  // the walks without a structure
+    static constexpr int nsp = 0, nr = 0;
+    static __host__ __device__ constexpr int code(int, int) { return 0; }
+    static __host__ __device__ constexpr int flags(int) { return 0; }
+};
+template <>
+struct MechShape<WALK_AIR5_PARK> {
+    static constexpr int nsp = 5, nr = 5;
+    static __host__ __device__ constexpr int code(int ir, int s) {
+        constexpr int none = row_code(0, 0, 0), m = row_code(0, 0, 1), a = row_code(1, 0, 0), b = row_code(0, 1, 0);
+        constexpr int am = row_code(1, 0, 1), bm = row_code(0, 1, 1), b2m = row_code(0, 2, 1);
+        constexpr int t[5][5] = {{am, m, m, b2m, m},       // N2 + M <=> 2 N + M
+                                 {m, am, m, m, b2m},       // O2 + M <=> 2 O + M
+                                 {m, m, am, bm, bm},       // NO + M <=> N + O + M
+                                 {none, b, a, b, a},       // NO + O <=> O2 + N
+                                 {a, none, b, b, a}};      // N2 + O <=> NO + N
+        return t[ir][s];
+    }
+    static __host__ __device__ constexpr int flags(int ir) { return ir < 3 ? 1 : 0; }
+};
+template <>
+struct MechShape<WALK_AIR5_GUPTA> {
+    static constexpr int nsp = 5, nr = 6;
+    static __host__ __device__ constexpr int code(int ir, int s) {
+        constexpr int none = row_code(0, 0, 0), m = row_code(0, 0, 1), a = row_code(1, 0, 0), b = row_code(0, 1, 0);
+        constexpr int am = row_code(1, 0, 1), bm = row_code(0, 1, 1), b2 = row_code(0, 2, 0), b2m = row_code(0, 2, 1);
+        constexpr int t[6][5] = {{m, am, m, m, b2m},                       // O2 + M <=> 2 O + M
+                                 {am, m, m, b2, m},                        // N2 + M <=> 2 N + M, M not N
+                                 {a, none, none, row_code(1, 3, 0), none}, // N2 + N <=> 3 N
+                                 {m, m, am, bm, bm},                       // NO + M <=> N + O + M
+                                 {none, b, a, b, a},                       // NO + O <=> O2 + N
+                                 {a, none, b, b, a}};                      // N2 + O <=> NO + N
+        return t[ir][s];
+    }
+    static __host__ __device__ constexpr int flags(int ir) { return (ir < 2 || ir == 3) ? 1 : 0; }
+};
+template <>
+struct MechShape<WALK_N2_PAIR> {
+    static constexpr int nsp = 2, nr = 2;
+    static __host__ __device__ constexpr int code(int ir, int s) {
+        constexpr int t[2][2] = {{row_code(2, 1, 0), row_code(0, 2, 0)},   // 2 N2 <=> N2 + 2 N
+                                 {row_code(1, 0, 0), row_code(1, 3, 0)}};  // N2 + N <=> 3 N
+        return t[ir][s];
+    }
+    static __host__ __device__ constexpr int flags(int) { return 0; }
+};
+
 struct ChemDev {
     int nsp, nr;
     double M[CH_MAX_SP], R[CH_MAX_SP];
     CEADev cea[CH_MAX_SP];
     ReacDev r[CH_MAX_R];
     int all_sorted;  // every reaction in dense form: rr[] holds the mechanism
+    int walk;        // ChemWalk of the mechanism
     RateRow rr[CH_MAX_R];
     double T_lower, T_upper;
     int method;  // 0 alpha-QSS, 1 RKF
@@ -82,6 +151,27 @@ struct ChemDev {
     double T_frozen;
     int tight;  // tightTempCoupling: T(u) and the rate constants after every subcycle
 };
+
+// The walk of a filled table: a structure of its own code where the rows match it word for
+// word, the rows where every list is in ascending species order, otherwise the lists.
+template <int WALK>
+inline bool shape_matches(const ChemDev& cd) {
+    using S = MechShape<WALK>;
+    if (cd.nsp != S::nsp || cd.nr != S::nr) return false;
+    for (int ir = 0; ir < S::nr; ++ir) {
+        if (cd.rr[ir].flags != S::flags(ir)) return false;
+        for (int s = 0; s < S::nsp; ++s)
+            if (cd.rr[ir].code[s] != S::code(ir, s)) return false;
+    }
+    return true;
+}
+inline int mechanism_walk(const ChemDev& cd) {
+    if (!cd.all_sorted) return WALK_LIST;
+    if (shape_matches<WALK_AIR5_PARK>(cd)) return WALK_AIR5_PARK;
+    if (shape_matches<WALK_AIR5_GUPTA>(cd)) return WALK_AIR5_GUPTA;
+    if (shape_matches<WALK_N2_PAIR>(cd)) return WALK_N2_PAIR;
+    return WALK_ROWS;
+}
 
 constexpr double CH_R_UNIVERSAL = 8.31451;               // gas/physical_constants.d
 constexpr double CH_P_ATM = 101.325e3;
@@ -517,17 +607,23 @@ __device__ __forceinline__ void eval_rate_constants(const ChemDev& cd, double Ti
 
 // The forward and backward rates of one reaction row (dense form) at conc, with c2 = conc^2:
 // reaction.d:289-330 (eval_forward_rate / eval_backward_rate) for lists in ascending order.
-template <int NSP>
-__device__ __forceinline__ void dense_row_rates(const RateRow& rr, double kf, double kb, const double* conc,
+// With the structure in WALK every select below is decided at compile time; the products and
+// sums and their order are the same.
+template <int NSP, int WALK>
+__device__ __forceinline__ void dense_row_rates(const RateRow& rr, int ir, double kf, double kb, const double* conc,
                                                 const double* c2, double& wf_out, double& wb_out) {
+    constexpr bool SHAPED = WALK > WALK_ROWS;
     int code[NSP];
 #pragma unroll
-    for (int s = 0; s < NSP; ++s) code[s] = rr.code[s];
+    for (int s = 0; s < NSP; ++s) code[s] = SHAPED ? MechShape<WALK>::code(ir, s) : rr.code[s];
+    const int flags = SHAPED ? MechShape<WALK>::flags(ir) : rr.flags;
     double collider = 0.0;
+    if (!SHAPED || (flags & 1)) {
 #pragma unroll
-    for (int s = 0; s < NSP; ++s) collider += (code[s] & 256) ? rr.eff[s] * conc[s] : 0.0;
-    double wf = (rr.flags & 1) ? kf * collider : kf;
-    double wb = (rr.flags & 1) ? kb * collider : kb;
+        for (int s = 0; s < NSP; ++s) collider += (code[s] & 256) ? rr.eff[s] * conc[s] : 0.0;
+    }
+    double wf = (flags & 1) ? kf * collider : kf;
+    double wb = (flags & 1) ? kb * collider : kb;
     // c^e for e in 0..3 as (c or 1) * (c^2 or 1): c * (c * c) for e = 3, as ch_ipow
 #pragma unroll
     for (int s = 0; s < NSP; ++s) wf *= ((code[s] & 1) ? conc[s] : 1.0) * ((code[s] & 2) ? c2[s] : 1.0);
@@ -538,37 +634,41 @@ __device__ __forceinline__ void dense_row_rates(const RateRow& rr, double kf, do
 }
 
 // Net coefficient of species s in a dense row (4-bit two's complement in bits 4-7).
-__device__ __forceinline__ int dense_row_nu(const RateRow& rr, int s) { return (int)((unsigned)rr.code[s] << 24) >> 28; }
+template <int WALK>
+__device__ __forceinline__ int dense_row_nu(const RateRow& rr, int ir, int s) {
+    const int code = (WALK > WALK_ROWS) ? MechShape<WALK>::code(ir, s) : rr.code[s];
+    return (int)((unsigned)code << 24) >> 28;
+}
 
 // reaction_mechanism.d:83-96 (eval_split_rates) with reaction.d's forward/backward rates
 // (collider sum over the efficiency list, then the concentration products in list order)
 // and production/loss per participant in reaction order.
 //
-// DENSE (every list of the mechanism in ascending species order, rr[] filled; the host
-// picks the instantiation) takes a branch-free walk over the rows: an absent reactant or
+// WALK_ROWS and the shapes (every list of the mechanism in ascending species order, rr[] filled;
+// the host picks the instantiation) take a branch-free walk over the rows: an absent reactant or
 // product multiplies by exactly 1, a species outside the third-body list or the reaction
 // adds exactly 0 (a selected zero, not a product with zero), and a reaction without third
 // body takes kf as it is, so every result equals the list walk bit for bit while the table
 // words load in bulk instead of one load and branch per entry.
-template <int NSP, int NRM, bool DENSE>
+template <int NSP, int NRM, int WALK>
 __device__ __forceinline__ void eval_split_rates(const ChemDev& cd, const double* kf, const double* kb,
                                                  const double* conc, double* q, double* L) {
 #pragma unroll
     for (int s = 0; s < NSP; ++s) { q[s] = 0.0; L[s] = 0.0; }
-    if constexpr (DENSE) {
+    if constexpr (WALK != WALK_LIST) {
         double c2[NSP];
 #pragma unroll
         for (int s = 0; s < NSP; ++s) c2[s] = conc[s] * conc[s];
         const int nr = cd.nr;
 #pragma unroll
         for (int ir = 0; ir < NRM; ++ir) {
-            if (ir >= nr) break;
+            if (WALK == WALK_ROWS && ir >= nr) break;  // a shape has NRM reactions
             const RateRow& rr = cd.rr[ir];
             double wf, wb;
-            dense_row_rates<NSP>(rr, kf[ir], kb[ir], conc, c2, wf, wb);
+            dense_row_rates<NSP, WALK>(rr, ir, kf[ir], kb[ir], conc, c2, wf, wb);
 #pragma unroll
             for (int s = 0; s < NSP; ++s) {
-                const int nu = dense_row_nu(rr, s);
+                const int nu = dense_row_nu<WALK>(rr, ir, s);
                 const double m = (double)(nu < 0 ? -nu : nu);
                 const bool pos = nu > 0;
                 q[s] += (nu != 0) ? m * (pos ? wf : wb) : 0.0;
@@ -626,11 +726,11 @@ __device__ __forceinline__ void eval_split_rates(const ChemDev& cd, const double
 }
 
 // reaction_mechanism.d:162-203
-template <int NSP, int NRM, bool DENSE>
+template <int NSP, int NRM, int WALK>
 __device__ __forceinline__ double estimate_step_size(const ChemDev& cd, const double* kf, const double* kb, const double* conc) {
     const double MUCH_LARGER_FACTOR = 10000.0, ZERO_EPS = 1.0e-50, ZERO_TOL = 1.0e-30, EPS1 = 1.0e-3;
     double q[NSP], L[NSP];
-    eval_split_rates<NSP, NRM, DENSE>(cd, kf, kb, conc, q, L);
+    eval_split_rates<NSP, NRM, WALK>(cd, kf, kb, conc, q, L);
     double min_dt = 1.0e6, dt;
 #pragma unroll
     for (int s = 0; s < NSP; ++s) {
@@ -647,49 +747,69 @@ __device__ __forceinline__ double estimate_step_size(const ChemDev& cd, const do
     return dt_chem;
 }
 
-// alpha(r) of chemistry_update.d:599-604 for r = 1/(p h + eps)
-__device__ __forceinline__ double qss_alpha(double p, double h) {
-    const double ZERO_EPS = 1.0e-50;
-    double r = 1.0 / (p * h + ZERO_EPS);
-    return (180.0 * r * r * r + 60.0 * r * r + 11.0 * r + 1.0) / (360.0 * r * r * r + 60.0 * r * r + 12.0 * r + 1.0);
+// a / b for normal operands: the hardware reciprocal refined by one cubic step (residual e:
+// y (1 + e + e^2), relative error e^3), the quotient and one remainder correction, which
+// leaves it within an ulp.  7 instructions, where the compiler's division takes 11 to scale
+// operands that none of the quotients here needs scaled.
+__device__ __forceinline__ double quick_rcp(double b) {
+    const double y = __builtin_amdgcn_rcp(b);
+    const double e = fma(-b, y, 1.0);
+    return fma(y, fma(e, e, e), y);
 }
+__device__ __forceinline__ double quick_div(double a, double b) { return div_by(a, b, quick_rcp(b)); }
 
 // AlphaQssStep.opCall, chemistry_update.d:533-655: predictor, up to maxIters correctors
 // with alpha-bar from p_p, convergence against the first predictor, and the step
 // suggestion from three Newton iterations for sqrt(sigma).  yOut is written on success.
 // Trip 0 of the loop is the predictor (rates at y0), trips 1..maxIters the correctors
-// (rates at yp), so the rate code is inlined once; each trip evaluates exactly the
-// reference's expressions for its kind:
+// (rates at yp), so the rate code is inlined once:
 //   predictor  yp = y0 + h (q0 - p0 y0) / (1 + alpha(p0) h p0)
 //   corrector  yc = y0 + h (q~ - p- y0) / (1 + alpha(pp) h p-),
 //              q~ = alpha(pp) qp + (1 - alpha(pp)) q0,  p- = (p0 + pp) / 2
-template <int NSP, int NRM, bool DENSE>
+// The reference's alpha(r), r = 1 / (p h + 1e-50) (:599-604), is N(x) / D(x) in x = p h with
+//   N = x^3 + 11 x^2 + 60 x + 180,  D = x^3 + 12 x^2 + 60 x + 360,  D - N = x^2 + 180,
+// so both forms are taken over the common denominator D,
+//   y = y0 + (h (N q + (D - N) q0) - x- y0 D) / (D + N x-),  x- = h p-,
+// with 2 divisions a species and trip (p, and y) instead of 4, and neither a reciprocal of p h
+// nor alpha itself.  x is bounded at 1e60, where alpha is 1, so that x^3 stays finite.
+// sigma = max n / d over the species is kept as its n and d (compared by cross products), and
+// the three Newton iterations from x = sigma for its root, x <- (x + sigma / x) / 2, give
+// with S = n + d, P = S^2 + 4 n d
+//   1 / x3 = 8 d P S / (P^2 + 16 n d S^2):
+// one division for the step suggestion instead of 8.
+template <int NSP, int NRM, int WALK>
 __device__ __forceinline__ bool alpha_qss_step(const ChemDev& cd, const double* kf, const double* kb, const double* y0,
                                                double h, double* yOut, double& hSuggest, int& iters) {
     const double ZERO_EPS = 1.0e-50;
-    double q0[NSP], p0[NSP], yp[NSP], yp0[NSP], yc[NSP];
+    double q0[NSP], x0[NSP], yp[NSP], yp0[NSP], yc[NSP];
 #pragma unroll
     for (int s = 0; s < NSP; ++s) {
         q0[s] = 0.0;
-        p0[s] = 0.0;
+        x0[s] = 0.0;
         yp[s] = y0[s];
     }
     bool converged = false;
     for (int trip = 0; trip <= cd.maxIters; ++trip) {
         const bool pred = (trip == 0);
         double q[NSP], L[NSP];
-        eval_split_rates<NSP, NRM, DENSE>(cd, kf, kb, yp, q, L);  // yp = y0 on the predictor trip
+        eval_split_rates<NSP, NRM, WALK>(cd, kf, kb, yp, q, L);  // yp = y0 on the predictor trip
         bool passes = true;
 #pragma unroll
         for (int s = 0; s < NSP; ++s) {
-            const double p = L[s] / (yp[s] + ZERO_EPS);
-            const double a = qss_alpha(p, h);
-            const double qx = pred ? q[s] : a * q[s] + (1 - a) * q0[s];
-            const double px = pred ? p : 0.5 * (p0[s] + p);
-            const double ynew = y0[s] + (h * (qx - px * y0[s])) / (1.0 + a * h * px);
+            const double xp = h * quick_div(L[s], yp[s] + ZERO_EPS);
             if (pred) {
                 q0[s] = q[s];
-                p0[s] = p;
+                x0[s] = xp;
+            }
+            const double xm = 0.5 * (x0[s] + xp);  // xp itself on the predictor trip
+            const double x = fmin(xp, 1.0e60);
+            const double N = fma(fma(x + 11.0, x, 60.0), x, 180.0);
+            const double W = fma(x, x, 180.0);  // D - N
+            const double D = N + W;
+            // on the predictor trip q = q0, and N q + W q0 is D q0
+            const double num = fma(-(xm * y0[s]), D, h * fma(N, q[s], W * q0[s]));
+            const double ynew = y0[s] + quick_div(num, fma(N, xm, D));
+            if (pred) {
                 yp0[s] = ynew;
             } else if (ynew >= ZERO_EPS) {
                 if (fabs(ynew - yp0[s]) >= (cd.eps1 * (ynew + cd.delta))) passes = false;
@@ -706,21 +826,22 @@ __device__ __forceinline__ bool alpha_qss_step(const ChemDev& cd, const double* 
 #pragma unroll
         for (int s = 0; s < NSP; ++s) yp[s] = yc[s];
     }
-    double sigma = 0.0;
+    double n = 0.0, d = 1.0;
 #pragma unroll
     for (int s = 0; s < NSP; ++s) {
         if (yc[s] < ZERO_EPS) continue;
-        double test = fabs(yc[s] - yp0[s]) / (cd.eps2 * (yc[s] + cd.delta));
-        if (test > sigma) sigma = test;
+        const double ns = fabs(yc[s] - yp0[s]), ds = cd.eps2 * (yc[s] + cd.delta);
+        if (ns * d > n * ds) {
+            n = ns;
+            d = ds;
+        }
     }
-    if (sigma <= 0.0) {
+    if (n <= 0.0) {
         hSuggest = 10.0 * h;
     } else {
-        double x = sigma;
-        x = x - 0.5 * (x * x - sigma) / x;
-        x = x - 0.5 * (x * x - sigma) / x;
-        x = x - 0.5 * (x * x - sigma) / x;
-        hSuggest = h * ((1.0 / x) + 0.005);
+        const double S = n + d, nd4 = 4.0 * n * d;
+        const double P = fma(S, S, nd4);
+        hSuggest = h * (quick_div(8.0 * d * P * S, fma(P, P, 4.0 * nd4 * S * S)) + 0.005);
     }
     if (converged) {
 #pragma unroll
@@ -730,7 +851,7 @@ __device__ __forceinline__ bool alpha_qss_step(const ChemDev& cd, const double* 
 }
 
 // RKFStep.opCall, chemistry_update.d:385-484 (Cash-Karp tableau); yOut is always written.
-template <int NSP, int NRM, bool DENSE>
+template <int NSP, int NRM, int WALK>
 __device__ __forceinline__ bool rkf_step(const ChemDev& cd, const double* kf, const double* kb, const double* y0, double h,
                          double* yOut, double& hSuggest, double* yLast = nullptr) {
     const double a21 = 1. / 5., a31 = 3. / 40., a32 = 9. / 40., a41 = 3. / 10., a42 = -9. / 10., a43 = 6. / 5.,
@@ -740,7 +861,7 @@ __device__ __forceinline__ bool rkf_step(const ChemDev& cd, const double* kf, co
                  b43 = 18575. / 48384., b44 = 13525. / 55296., b45 = 277. / 14336., b46 = 1.0 / 4.0;
     double k1[NSP], k2[NSP], k3[NSP], k4[NSP], k5[NSP], k6[NSP], yT[NSP], q[NSP], L[NSP];
     auto rates = [&](const double* y, double* k) {
-        eval_split_rates<NSP, NRM, DENSE>(cd, kf, kb, y, q, L);
+        eval_split_rates<NSP, NRM, WALK>(cd, kf, kb, y, q, L);
 #pragma unroll
         for (int s = 0; s < NSP; ++s) k[s] = q[s] - L[s];
     };

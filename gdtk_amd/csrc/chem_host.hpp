@@ -119,11 +119,11 @@ struct Chem {
         if (tu.persistent < 0) tu.persistent = ((long long)n > 2048LL * std::max(num_cu, 1)) ? 1 : 0;
         HIPCHK(hipEventRecord(ev[0], s));
         HIPCHK(launch_chem_clear(w, s));
-        HIPCHK(launch_chem_setup(dev, nsp, nr, host.all_sorted, n, dt, rho, T, massf, dtc, mask,
+        HIPCHK(launch_chem_setup(dev, nsp, nr, host.walk, n, dt, rho, T, massf, dtc, mask,
                                  tu.persistent ? tu.heavy_ratio : 0, w, s));
         HIPCHK(hipEventRecord(ev[1], s));
         int waves = 0;
-        HIPCHK(launch_chem_integrate(dev, nsp, nr, host.all_sorted, host.method, host.tight, n, dt, rho, T, u, dtc,
+        HIPCHK(launch_chem_integrate(dev, nsp, nr, host.walk, host.method, host.tight, n, dt, rho, T, u, dtc,
                                      dtc_out, w, tu, num_cu, &waves, s));
         HIPCHK(hipEventRecord(ev[2], s));
         HIPCHK(launch_chem_finish(dev, nsp, n, rho, T, u, p, massf, dtc, T_out, u_out, p_out, massf_out, dtc_out,

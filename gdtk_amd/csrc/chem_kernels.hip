@@ -34,24 +34,24 @@ static hipError_t run_nsp(int nsp, const ChemCall& c) {
     }
 }
 
-hipError_t launch_chem_setup(const ChemDev* cd, int nsp, int nr, int dense, int n, double dt, const double* rho,
+hipError_t launch_chem_setup(const ChemDev* cd, int nsp, int nr, int walk, int n, double dt, const double* rho,
                              const double* T, const double* massf, const double* dtc, const int* mask,
                              int heavy_ratio, const ChemWork& w, hipStream_t s) {
     ChemCall c{};
     c.phase = CHEM_PHASE_SETUP;
-    c.cd = cd; c.nr = nr; c.dense = dense; c.n = n; c.dt = dt;
+    c.cd = cd; c.nr = nr; c.walk = walk; c.n = n; c.dt = dt;
     c.rho = rho; c.T = T; c.massf = massf; c.dtc_in = dtc; c.mask = mask; c.tu.heavy_ratio = heavy_ratio;
     c.w = w; c.s = s;
     return run_nsp(nsp, c);
 }
 
-hipError_t launch_chem_integrate(const ChemDev* cd, int nsp, int nr, int dense, int method, int tight, int n, double dt,
+hipError_t launch_chem_integrate(const ChemDev* cd, int nsp, int nr, int walk, int method, int tight, int n, double dt,
                                  const double* rho, const double* T, const double* u, const double* dtc_in,
                                  double* dtc_out, const ChemWork& w, const ChemTuning& tu, int num_cu, int* waves,
                                  hipStream_t s) {
     ChemCall c{};
     c.phase = CHEM_PHASE_INTEGRATE;
-    c.cd = cd; c.nr = nr; c.dense = dense; c.method = method; c.tight = tight; c.n = n; c.dt = dt;
+    c.cd = cd; c.nr = nr; c.walk = walk; c.method = method; c.tight = tight; c.n = n; c.dt = dt;
     c.rho = rho; c.T = T; c.u = u; c.dtc_in = dtc_in; c.dtc_out = dtc_out;
     c.w = w; c.tu = tu; c.num_cu = num_cu; c.waves_out = waves; c.s = s;
     return run_nsp(nsp, c);

@@ -24,7 +24,7 @@
 
 namespace gdtk {
 
-template <int NSP, int NRM, bool DENSE>
+template <int NSP, int NRM, int WALK>
 __global__ __launch_bounds__(CHEM_BLOCK) void k_chem_setup(const ChemDev* __restrict__ cdp, int n, double dt,
                                                            const double* __restrict__ rho,
                                                            const double* __restrict__ T,
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(CHEM_BLOCK) void k_chem_setup(const ChemDev* __rest
     // chemistry_update.d:152-158.  The estimate is also the first step of the retry with
     // dt_chem = -1 (fvcell.d:899-905), which starts from the same state.
     const double d = dtc[i];
-    const double est = estimate_step_size<NSP, NRM, DENSE>(cd, kf, kb, conc);
+    const double est = estimate_step_size<NSP, NRM, WALK>(cd, kf, kb, conc);
     double h;
     if (d > dt) h = dt;
     else if (d <= 0.0) h = est;
@@ -138,7 +138,7 @@ __device__ __forceinline__ void load_cell(const ChemDev& cd, int n, int i, const
 // failed T(u) iteration there raises GasModelException in the reference, which the
 // thermochemical_increment of fvcell.d:894-905 does not catch: the cell fails without the
 // retry.
-template <int NSP, int NRM, int METHOD, bool TIGHT, bool DENSE>
+template <int NSP, int NRM, int METHOD, bool TIGHT, int WALK>
 __global__ __launch_bounds__(CHEM_BLOCK) void k_chem_integrate(const ChemDev* __restrict__ cdp, int n, double dt,
                                                                const double* __restrict__ rho,
                                                                const double* __restrict__ T_in,
@@ -253,15 +253,18 @@ __global__ __launch_bounds__(CHEM_BLOCK) void k_chem_integrate(const ChemDev* __
         double y[NSP];
         bool ok;
         if (METHOD == 1) {
-            ok = rkf_step<NSP, NRM, DENSE>(cd, c.kf, c.kb, c.c0, c.h, y, c.dtSug);
+            ok = rkf_step<NSP, NRM, WALK>(cd, c.kf, c.kb, c.c0, c.h, y, c.dtSug);
         } else {
-            ok = alpha_qss_step<NSP, NRM, DENSE>(cd, c.kf, c.kb, c.c0, c.h, y, c.dtSug, c.iters);
+            ok = alpha_qss_step<NSP, NRM, WALK>(cd, c.kf, c.kb, c.c0, c.h, y, c.dtSug, c.iters);
         }
         bool passes = true;
         if (ok) {
-            double mf[NSP];
-            const double massfTotal = conc_to_massf<NSP>(cd, y, c.rho, mf);
-            if (fabs(massfTotal - 1.0) > ALLOWABLE_MASSF_ERROR) passes = false;
+            // chemistry_update.d:180-185: |sum of the mass fractions - 1| > 1e-3, taken on the
+            // sum of the species densities (no division by rho)
+            double rsum = 0.0;
+#pragma unroll
+            for (int s = 0; s < NSP; ++s) rsum = fma(y[s], cd.M[s], rsum);
+            if (fabs(rsum - c.rho) > ALLOWABLE_MASSF_ERROR * c.rho) passes = false;
         }
         int outcome = 0;  // 0 continue, 1 done, -1 this pass failed
         if (ok && passes) {
@@ -468,9 +471,9 @@ static inline unsigned grid_for(int n) { return (unsigned)((n + CHEM_BLOCK - 1) 
 struct SetupL {
     const ChemDev* cd; int n; double dt; const double *rho, *T, *massf, *dtc; const int* mask; int heavy_ratio;
     ChemWork w; hipStream_t s;
-    template <int NSP, int NRM, bool DENSE>
+    template <int NSP, int NRM, int WALK>
     hipError_t run() {
-        hipLaunchKernelGGL((k_chem_setup<NSP, NRM, DENSE>), dim3(grid_for(n)), dim3(CHEM_BLOCK), 0, s, cd, n, dt, rho,
+        hipLaunchKernelGGL((k_chem_setup<NSP, NRM, WALK>), dim3(grid_for(n)), dim3(CHEM_BLOCK), 0, s, cd, n, dt, rho,
                            T, massf, dtc, mask, heavy_ratio, w);
         return hipGetLastError();
     }
@@ -479,14 +482,14 @@ struct SetupL {
 struct IntegrateL {
     const ChemDev* cd; int n; double dt; const double* rho; const double *T, *u; const double* dtc_in;
     double* dtc_out; ChemWork w; ChemTuning tu; int num_cu; int method; int tight; int* waves_out; hipStream_t s;
-    template <int NSP, int NRM, int METHOD, bool TIGHT, bool DENSE>
+    template <int NSP, int NRM, int METHOD, bool TIGHT, int WALK>
     hipError_t launch() {
         unsigned grid = grid_for(n);
         if (tu.persistent) {
             int per_cu = tu.blocks_per_cu;
             if (per_cu <= 0) {
                 hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                    &per_cu, reinterpret_cast<const void*>(&k_chem_integrate<NSP, NRM, METHOD, TIGHT, DENSE>), CHEM_BLOCK,
+                    &per_cu, reinterpret_cast<const void*>(&k_chem_integrate<NSP, NRM, METHOD, TIGHT, WALK>), CHEM_BLOCK,
                     0);
                 if (e != hipSuccess) return e;
                 if (per_cu < 1) per_cu = 1;
@@ -497,14 +500,14 @@ struct IntegrateL {
         }
         if (waves_out) *waves_out = (int)grid * CHEM_WAVES_PER_BLOCK;
         const int chunk = tu.chunk > 0 ? tu.chunk : 64;
-        hipLaunchKernelGGL((k_chem_integrate<NSP, NRM, METHOD, TIGHT, DENSE>), dim3(grid), dim3(CHEM_BLOCK), 0, s, cd,
+        hipLaunchKernelGGL((k_chem_integrate<NSP, NRM, METHOD, TIGHT, WALK>), dim3(grid), dim3(CHEM_BLOCK), 0, s, cd,
                            n, dt, rho, T, u, dtc_in, dtc_out, w, tu.persistent, chunk, tu.refill_period);
         return hipGetLastError();
     }
-    template <int NSP, int NRM, bool DENSE>
+    template <int NSP, int NRM, int WALK>
     hipError_t run() {
-        if (method == 1) return launch<NSP, NRM, 1, false, DENSE>();  // RKF with tight coupling is refused at set-up
-        return tight ? launch<NSP, NRM, 0, true, DENSE>() : launch<NSP, NRM, 0, false, DENSE>();
+        if (method == 1) return launch<NSP, NRM, 1, false, WALK>();  // RKF with tight coupling is refused at set-up
+        return tight ? launch<NSP, NRM, 0, true, WALK>() : launch<NSP, NRM, 0, false, WALK>();
     }
 };
 
@@ -529,26 +532,33 @@ struct TpgL {
     }
 };
 
-// One phase of a chemistry call for NSP species.  Mechanisms in dense form get the
-// branch-free rate walk with the reaction bound 5 for the 5-species, 5-reaction air
-// mechanism, otherwise 8 or 32; the others the list walk with the bound 32.
+// Runs a phase's launcher with the rate code of the mechanism's walk: a structure of its own
+// code, the rows with the reaction bound 8 or 32, or the lists with the bound 32.
+template <int NSP, class L>
+hipError_t chem_walk_run(L& l, const ChemCall& c) {
+    if constexpr (NSP == MechShape<WALK_AIR5_PARK>::nsp) {
+        if (c.walk == WALK_AIR5_PARK) return l.template run<NSP, MechShape<WALK_AIR5_PARK>::nr, WALK_AIR5_PARK>();
+    }
+    if constexpr (NSP == MechShape<WALK_N2_PAIR>::nsp) {
+        if (c.walk == WALK_N2_PAIR) return l.template run<NSP, MechShape<WALK_N2_PAIR>::nr, WALK_N2_PAIR>();
+    }
+    if (c.walk == WALK_LIST) return l.template run<NSP, 32, WALK_LIST>();
+    if (c.nr <= 8) return l.template run<NSP, 8, WALK_ROWS>();
+    return l.template run<NSP, 32, WALK_ROWS>();
+}
+
+// One phase of a chemistry call for NSP species.
 template <int NSP>
 hipError_t chem_run(const ChemCall& c) {
     switch (c.phase) {
     case CHEM_PHASE_SETUP: {
         SetupL l{c.cd, c.n, c.dt, c.rho, c.T, c.massf, c.dtc_in, c.mask, c.tu.heavy_ratio, c.w, c.s};
-        if (!c.dense) return l.template run<NSP, 32, false>();
-        if (NSP == 5 && c.nr == 5) return l.template run<NSP, 5, true>();
-        if (c.nr <= 8) return l.template run<NSP, 8, true>();
-        return l.template run<NSP, 32, true>();
+        return chem_walk_run<NSP>(l, c);
     }
     case CHEM_PHASE_INTEGRATE: {
         IntegrateL l{c.cd,    c.n,  c.dt,     c.rho,  c.T,      c.u,        c.dtc_in, c.dtc_out,
                      c.w,     c.tu, c.num_cu, c.method, c.tight, c.waves_out, c.s};
-        if (!c.dense) return l.template run<NSP, 32, false>();
-        if (NSP == 5 && c.nr == 5) return l.template run<NSP, 5, true>();
-        if (c.nr <= 8) return l.template run<NSP, 8, true>();
-        return l.template run<NSP, 32, true>();
+        return chem_walk_run<NSP>(l, c);
     }
     case CHEM_PHASE_FINISH: {
         FinishL l{c.cd, c.n, c.rho, c.T, c.u, c.p, c.massf, c.dtc_in, c.T_out, c.u_out, c.p_out, c.massf_out,

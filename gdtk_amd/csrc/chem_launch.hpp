@@ -58,7 +58,7 @@ enum ChemPhase : int { CHEM_PHASE_SETUP = 0, CHEM_PHASE_INTEGRATE = 1, CHEM_PHAS
 struct ChemCall {
     int phase;
     const ChemDev* cd;
-    int nr, n, mode, method, tight, dense;
+    int nr, n, mode, method, tight, walk;
     double dt;
     const double *rho, *T, *u, *p, *massf, *dtc_in;
     const int* mask;  // setup: cells with mask[i] != 0 are skipped (may be null)
@@ -87,12 +87,12 @@ extern template hipError_t chem_run<8>(const ChemCall&);
 bool chem_supported(int nsp, int nr);
 // Zero the queue counters (a fill kernel, so the call may be captured).
 hipError_t launch_chem_clear(const ChemWork& w, hipStream_t s);
-// dense: the mechanism's lists are all in ascending species order (ChemDev::all_sorted).
-hipError_t launch_chem_setup(const ChemDev* cd, int nsp, int nr, int dense, int n, double dt, const double* rho,
+// walk: the mechanism's ChemWalk (ChemDev::walk).
+hipError_t launch_chem_setup(const ChemDev* cd, int nsp, int nr, int walk, int n, double dt, const double* rho,
                              const double* T, const double* massf, const double* dtc, const int* mask,
                              int heavy_ratio, const ChemWork& w, hipStream_t s);
 // *waves: the waves launched, each of which writes its statistics entries.
-hipError_t launch_chem_integrate(const ChemDev* cd, int nsp, int nr, int dense, int method, int tight, int n, double dt,
+hipError_t launch_chem_integrate(const ChemDev* cd, int nsp, int nr, int walk, int method, int tight, int n, double dt,
                                  const double* rho, const double* T, const double* u, const double* dtc_in,
                                  double* dtc_out, const ChemWork& w, const ChemTuning& tu, int num_cu, int* waves,
                                  hipStream_t s);

@@ -182,7 +182,7 @@ __device__ __forceinline__ double tt_eval_rate(const ChemDev& cd, const TTDev& t
             if (ir >= cd.nr) break;
             const RateRow& rr = cd.rr[ir];
             if ((rr.code[s] & 15) == 0) continue;  // not a participant
-            const int nu = dense_row_nu(rr, s);
+            const int nu = dense_row_nu<WALK_ROWS>(rr, ir, s);
             const double prod = (nu > 0) ? nu * wf[ir] : (nu < 0) ? -nu * wb[ir] : 0.0;
             const double loss = (nu > 0) ? nu * wb[ir] : (nu < 0) ? -nu * wf[ir] : 0.0;
             chemRate += prod - loss;
@@ -287,7 +287,7 @@ __device__ __forceinline__ int tt_opcall(const ChemDev& cd, const TTDev& td, TTC
     tt_rate_constants<NRM>(cd, Q.T, Q.Tv, kf, kb);
     double t = 0.0, h, dtSave = 0.0;
     if (dtSuggest > tInterval) h = tInterval;
-    else if (dtSuggest <= 0.0) h = estimate_step_size<NSP, NRM, true>(cd, kf, kb, conc0);
+    else if (dtSuggest <= 0.0) h = estimate_step_size<NSP, NRM, WALK_ROWS>(cd, kf, kb, conc0);
     else h = dtSuggest;
     int cycle = 0;
     for (; cycle < cd.maxSubcycles; ++cycle) {
@@ -297,7 +297,7 @@ __device__ __forceinline__ int tt_opcall(const ChemDev& cd, const TTDev& td, TTC
         for (; attempt < cd.maxAttempts; ++attempt) {
             ++cnt.attempts;
             double yLast[NSP];
-            const bool r1 = rkf_step<NSP, NRM, true>(cd, kf, kb, conc0, h, concOut, dtSuggest, yLast);
+            const bool r1 = rkf_step<NSP, NRM, WALK_ROWS>(cd, kf, kb, conc0, h, concOut, dtSuggest, yLast);
             // the reaction rates of the chemistry step's last evaluation
             double wf[NRM], wb[NRM], c2[NSP];
 #pragma unroll
@@ -306,7 +306,7 @@ __device__ __forceinline__ int tt_opcall(const ChemDev& cd, const TTDev& td, TTC
             for (int ir = 0; ir < NRM; ++ir) {
                 wf[ir] = 0.0;
                 wb[ir] = 0.0;
-                if (ir < cd.nr) dense_row_rates<NSP>(cd.rr[ir], kf[ir], kb[ir], yLast, c2, wf[ir], wb[ir]);
+                if (ir < cd.nr) dense_row_rates<NSP, WALK_ROWS>(cd.rr[ir], ir, kf[ir], kb[ir], yLast, c2, wf[ir], wb[ir]);
             }
             const int r2 = tt_energy_step<NSP, NRM>(cd, td, Q, uTotal, h, dtSuggest, wf, wb);
             if (r2 < 0) return -1;
