@@ -10,7 +10,10 @@
 // GPUChem.thermochemical_increment (src/eilmer/cuda_gpu_chem.d:155-191).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
 #include <cstring>
+#include <limits>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -32,6 +35,103 @@ Chem& get_chem(int h) {
     std::lock_guard<std::mutex> lk(g_chem_mu);
     if (h < 0 || h >= (int)g_chems.size() || !g_chems[h]) throw Error(GDTK_ERR_ARG, "bad chemistry handle");
     return *g_chems[h];
+}
+
+// One species' segment expanded about T0 (MixTable): {a0, a1, q0..q4, H0}.
+static void expand_segment(const double* a, long double T0, double* out) {
+    out[0] = a[0];
+    out[1] = a[1];
+    for (int k = 0; k < 5; ++k) {
+        long double q = 0.0L, pw = 1.0L, binom = 1.0L;  // sum over m of a[2 + m] C(m, k) T0^(m - k)
+        for (int m = k; m < 5; ++m) {
+            q += (long double)a[2 + m] * binom * pw;
+            pw *= T0;
+            binom = binom * (m + 1) / (m + 1 - k);
+        }
+        out[2 + k] = (double)q;
+    }
+    long double h = -(long double)a[0] / T0 + (long double)a[1] * std::log(T0) + (long double)a[7], pw = T0;
+    for (int m = 0; m < 5; ++m) {
+        h += (long double)a[2 + m] * pw / (m + 1);
+        pw *= T0;
+    }
+    out[7] = (double)h;
+}
+
+// What a species' curve is at T (cea_thermo_curves.d:56-70, 137-176, tests in its order): the
+// constant-Cp extension (seg = -1 below, -2 above), segment seg alone, or the blend of seg and
+// seg + 1.
+static void curve_at(const CEADev& c, double T, int& seg, bool& blend) {
+    blend = false;
+    const int nb = c.nseg + 1;
+    auto lo = [&](int i) { return c.T_breaks[i] - 0.5 * c.T_blends[i - 1]; };
+    auto hi = [&](int i) { return c.T_breaks[i] + 0.5 * c.T_blends[i - 1]; };
+    if (T < c.T_low) { seg = -1; return; }
+    if (T > c.T_high) { seg = -2; return; }
+    if (T < lo(1)) { seg = 0; return; }
+    if (T > hi(nb - 2)) { seg = c.nseg - 1; return; }
+    for (int i = 1; i < nb - 1; ++i) {
+        seg = i - 1;
+        if (T >= lo(i) && T <= hi(i)) { blend = true; return; }
+        seg = i;
+        if (i < c.nseg - 1 && T > hi(i) && T < lo(i + 1)) return;
+    }
+}
+
+// The regions of the summed curves (MixTable): the line cut at every species' range edges, each
+// piece's coefficients from what the species' curves are at its midpoint.
+static void build_mix_table(ChemDev& cd) {
+    MixTable& t = cd.mix;
+    std::vector<double> cut;
+    for (int i = 0; i < cd.nsp; ++i) {
+        const CEADev& c = cd.cea[i];
+        cut.push_back(c.T_low);
+        cut.push_back(c.T_high);
+        for (int k = 0; k < c.nseg - 1; ++k) {
+            cut.push_back(c.T_breaks[k + 1] - 0.5 * c.T_blends[k]);
+            cut.push_back(c.T_breaks[k + 1] + 0.5 * c.T_blends[k]);
+        }
+    }
+    std::sort(cut.begin(), cut.end());
+    cut.erase(std::unique(cut.begin(), cut.end()), cut.end());
+    const double inf = std::numeric_limits<double>::infinity();
+    t.nreg = (int)cut.size() + 1;
+    for (int r = 0; r < t.nreg; ++r) {
+        t.lo[r] = (r == 0) ? -inf : cut[r - 1];
+        t.hi[r] = (r == t.nreg - 1) ? inf : cut[r];
+        const double mid = (r == 0) ? std::nextafter(t.hi[r], -inf)
+                         : (r == t.nreg - 1) ? std::nextafter(t.lo[r], inf) : 0.5 * (t.lo[r] + t.hi[r]);
+        // the region's lower edge (z >= 0); the forms need T0 > 0
+        const double T0 = std::max((r == 0) ? mid : t.lo[r], 1.0);
+        t.T0[r] = T0;
+        t.iT0[r] = 1.0 / T0;
+        t.flat[r] = 1;
+        for (int i = 0; i < cd.nsp; ++i) {
+            const CEADev& c = cd.cea[i];
+            int seg = 0;
+            bool blend = false;
+            curve_at(c, mid, seg, blend);
+            double* a = t.c[r][0][i];
+            if (seg < 0) {
+                a[2] = ((seg == -1) ? c.Cp_low : c.Cp_high) / c.R;
+                a[7] = (seg == -1) ? (c.h_low - c.Cp_low * (c.T_low - T0)) / c.R
+                                   : (c.h_high + c.Cp_high * (T0 - c.T_high)) / c.R;
+                continue;
+            }
+            expand_segment(c.coeffs[seg], T0, a);
+            if (!blend) continue;
+            // (1 - wB) A + wB B, wB = (T - w0) / width = w + z / width
+            double B[8];
+            expand_segment(c.coeffs[seg + 1], T0, B);
+            const double width = c.T_blends[seg], w = (T0 - (c.T_breaks[seg + 1] - 0.5 * width)) / width;
+            for (int j = 0; j < 8; ++j) {
+                const double A = a[j];
+                a[j] = (1.0 - w) * A + w * B[j];
+                t.c[r][1][i][j] = (B[j] - A) / width;
+            }
+            t.flat[r] = 0;
+        }
+    }
 }
 
 // Gas record -> the gas part of the device table (molecular masses, species gas constants,
@@ -65,6 +165,7 @@ void build_tpg_gas(const gdtk_tpg_gas& g, ChemDev& cd) {
         c.s_low = cea_s(c, c.T_low);
         c.s_high = cea_s(c, c.T_high);
     }
+    build_mix_table(cd);
 }
 
 // Gas and mechanism records -> the device table, with the checks the reference's input

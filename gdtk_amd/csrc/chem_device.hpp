@@ -134,6 +134,25 @@ struct MechShape<WALK_N2_PAIR> {
     static __host__ __device__ constexpr int flags(int) { return 0; }
 };
 
+// The species' curves as the mixture sums them (TpgMix).  The temperature line is cut where any
+// species changes its range (its end points and the edges of its blends, cea_thermo_curves.d:
+// 137-176); region r lies between lo[r] and hi[r] and has an expansion point T0, its lower edge.  There every
+// species' coefficients {a0, a1, q0..q4, H0} are c[0] + z c[1], z = T - T0 (linear in T in a
+// blend of two segments; flat[r] = 1 where no species blends and c[1] is 0), with
+//   h / R  = H0 + a1 log(T / T0) + z (a0 / (T T0) + q0 + z (q1/2 + z (q2/3 + z (q3/4 + z q4/5)))),
+//   Cp / R = (a0 / T + a1) / T + q0 + z (q1 + z (q2 + z (q3 + z q4))):
+// the NASA-9 forms of cea_thermo_curves.d:56-102 expanded about T0 (in extended precision on
+// the host), where every term but H0 vanishes, so that sums do not cancel as the terms of the
+// plain form do (by a factor 60 above 6000 K: u to 8e-16 of Cv T there, rms, against 1e-14 in
+// the plain form).
+constexpr int MIX_REGIONS = 6 * CH_MAX_SP + 1;  // up to 6 cuts a species
+struct MixTable {
+    int nreg;
+    int flat[MIX_REGIONS];
+    double lo[MIX_REGIONS], hi[MIX_REGIONS], T0[MIX_REGIONS], iT0[MIX_REGIONS];
+    double c[MIX_REGIONS][2][CH_MAX_SP][8];
+};
+
 struct ChemDev {
     int nsp, nr;
     double M[CH_MAX_SP], R[CH_MAX_SP];
@@ -141,6 +160,7 @@ struct ChemDev {
     ReacDev r[CH_MAX_R];
     int all_sorted;  // every reaction in dense form: rr[] holds the mechanism
     int walk;        // ChemWalk of the mechanism
+    MixTable mix;
     RateRow rr[CH_MAX_R];
     double T_lower, T_upper;
     int method;  // 0 alpha-QSS, 1 RKF
@@ -306,28 +326,6 @@ __host__ __device__ inline void cea_h_Cp(const CEADev& c, const CeaT& p, double&
                div_by(a[6] * T * T * T * T * T, 5.0, 1.0 / 5.0) + a[7];
     h = c.R * h_on_RT;
 }
-__host__ __device__ inline double cea_h(const CEADev& c, const CeaT& p) {
-    const double T = p.T;
-    if (T < c.T_low) return c.h_low - c.Cp_low * (c.T_low - T);
-    if (T > c.T_high) return c.h_high + c.Cp_high * (T - c.T_high);
-    double a[9];
-    cea_coeffs(c, T, a);
-    double h_on_RT = div_by(-a[0], T, p.rT) + a[1] * p.logT + a[2] * T + a[3] * T * T / 2.0;
-    h_on_RT += div_by(a[4] * T * T * T, 3.0, 1.0 / 3.0) + a[5] * T * T * T * T / 4.0 +
-               div_by(a[6] * T * T * T * T * T, 5.0, 1.0 / 5.0) + a[7];
-    return c.R * h_on_RT;
-}
-__host__ __device__ inline double cea_Cp(const CEADev& c, const CeaT& p) {
-    const double T = p.T;
-    if (T < c.T_low) return c.Cp_low;
-    if (T > c.T_high) return c.Cp_high;
-    double a[9];
-    cea_coeffs(c, T, a);
-    double Cp_on_R = div_by(a[0], p.TT, p.rTT) + div_by(a[1], T, p.rT) + a[2] + a[3] * T;
-    Cp_on_R += a[4] * T * T + a[5] * T * T * T + a[6] * T * T * T * T;
-    return c.R * Cp_on_R;
-}
-
 // cea_h and cea_s (cea_thermo_curves.d:71-130) at one temperature from one coefficient
 // selection, log(T) and the reciprocals of CeaT: the same values bit for bit.  The
 // divisor 2 T T of the entropy is exactly 2 TT, whose reciprocal is exactly rTT / 2.
@@ -366,52 +364,6 @@ __host__ __device__ inline double cea_s(const CEADev& c, double T) {
     return c.R * s_on_R;
 }
 
-// therm_perf_gas_mix_eos.d:61-67 with gas_model.d:410-419 (mass_average)
-// SERIAL: a scheduling barrier after each species, so that the species' evaluations do
-// not interleave (fewer registers live at once, for kernels whose occupancy they limit).
-template <int NSP, bool SERIAL = false>
-__device__ __forceinline__ double tpg_energy(const ChemDev& cd, const double* massf, double T) {
-    const CeaT pw(T, log(T));
-    double u = 0.0;
-#pragma unroll
-    for (int i = 0; i < NSP; ++i) {
-        u += massf[i] * (cea_h(cd.cea[i], pw) - cd.R[i] * T);
-        if (SERIAL) __builtin_amdgcn_sched_barrier(0);
-    }
-    return u;
-}
-// tpg_energy and tpg_Cv at one temperature (the Newton iteration of T(u) evaluates both at
-// each iterate), sharing each species' coefficient selection and log(T).
-template <int NSP, bool SERIAL = false>
-__device__ __forceinline__ void tpg_energy_Cv(const ChemDev& cd, const double* massf, double T, double& u,
-                                              double& Cv) {
-    const CeaT pw(T, log(T));
-    double uu = 0.0, v = 0.0;
-#pragma unroll
-    for (int i = 0; i < NSP; ++i) {
-        double h, Cp;
-        cea_h_Cp(cd.cea[i], pw, h, Cp);
-        uu += massf[i] * (h - cd.R[i] * T);
-        v += massf[i] * (Cp - cd.R[i]);
-        if (SERIAL) __builtin_amdgcn_sched_barrier(0);
-    }
-    u = uu;
-    Cv = v;
-}
-template <int NSP>
-__device__ __forceinline__ double tpg_Cv(const ChemDev& cd, const double* massf, double T) {
-    double v = 0.0;
-#pragma unroll
-    for (int i = 0; i < NSP; ++i) v += massf[i] * (cea_Cp(cd.cea[i], T) - cd.R[i]);
-    return v;
-}
-template <int NSP>
-__device__ __forceinline__ double tpg_Cp(const ChemDev& cd, const double* massf, double T) {
-    double v = 0.0;
-#pragma unroll
-    for (int i = 0; i < NSP; ++i) v += massf[i] * cea_Cp(cd.cea[i], T);
-    return v;
-}
 // perf_gas_mix_eos.d:43-76
 template <int NSP>
 __device__ __forceinline__ double tpg_Rmix(const ChemDev& cd, const double* massf) {
@@ -421,11 +373,137 @@ __device__ __forceinline__ double tpg_Rmix(const ChemDev& cd, const double* mass
     return R;
 }
 
+// a / b for normal operands: the hardware reciprocal refined by one cubic step (residual e:
+// y (1 + e + e^2), relative error e^3), the quotient and one remainder correction, which
+// leaves it within an ulp.  7 instructions, where the compiler's division takes 11 to scale
+// operands that none of the quotients here needs scaled.
+__device__ __forceinline__ double quick_rcp(double b) {
+    const double y = __builtin_amdgcn_rcp(b);
+    const double e = fma(-b, y, 1.0);
+    return fma(y, fma(e, e, e), y);
+}
+__device__ __forceinline__ double quick_div(double a, double b) { return div_by(a, b, quick_rcp(b)); }
+
+// The curves of one composition near one temperature as a single curve: the sums over the
+// species of weight times coefficient (therm_perf_gas_mix_eos.d:61-67 and gas_model.d:410-419
+// take the sum over the species' curves at each temperature; the curves are linear in their
+// coefficients).  An evaluation then costs one logarithm, one reciprocal and 17 fused
+// operations whatever the number of species, where the per-species form takes some 45
+// instructions and a range search for each; a Newton solve evaluates three times on one build.
+// Valid on [lo, hi]; in a blend of two segments the coefficients depend on T and the interval
+// is empty.
+struct TpgMix {
+    double a0, a1, q0, q1, q2, q3, q4, H0, T0, iT0, lo, hi;
+    __device__ __forceinline__ void clear() {  // no curve yet
+        lo = __builtin_huge_val();
+        hi = -__builtin_huge_val();
+    }
+    __device__ __forceinline__ bool covers(double T) const { return T >= lo && T <= hi; }
+};
+
+// The weighted curves at T: sum of y_s (h_s / R_s) - lin T + cst, y_s usually massf_s R_s.  A
+// temperature that is not a number leaves a curve whose value is none either.
+template <int NSP>
+__device__ __forceinline__ void tpg_mix_build(const ChemDev& cd, const double* y, double lin, double cst, double T,
+                                              TpgMix& m) {
+    double c[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) c[j] = 0.0;
+    m.T0 = 0.0;
+    m.iT0 = 1.0;
+    m.clear();
+    bool found = false;
+    const int nreg = cd.mix.nreg;
+#pragma clang loop unroll(disable)
+    for (int r = 0; r < nreg; ++r) {
+        const double lo = cd.mix.lo[r], hi = cd.mix.hi[r];
+        if (!found && T >= lo && T <= hi) {
+            found = true;
+            const bool flat = cd.mix.flat[r] != 0;
+            m.T0 = cd.mix.T0[r];
+            m.iT0 = cd.mix.iT0[r];
+            if (flat) {
+                m.lo = lo;
+                m.hi = hi;
+            }
+            double w = 1.0;
+#pragma clang loop unroll(disable)
+            for (int k = 0; k < (flat ? 1 : 2); ++k) {
+                const double(*t)[8] = cd.mix.c[r][k];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    double acc = y[0] * t[0][j];
+#pragma unroll
+                    for (int s = 1; s < NSP; ++s) acc = fma(y[s], t[s][j], acc);
+                    c[j] = fma(w, acc, c[j]);
+                }
+                w = T - m.T0;
+            }
+        }
+    }
+    m.a0 = c[0];
+    m.a1 = c[1];
+    m.q0 = c[2] - lin;
+    m.q1 = c[3];
+    m.q2 = c[4];
+    m.q3 = c[5];
+    m.q4 = c[6];
+    m.H0 = fma(-lin, m.T0, c[7]) + cst;
+}
+
+__device__ __forceinline__ double tpg_mix_slope(const TpgMix& m, double z, double rT) {
+    const double q = fma(fma(fma(fma(m.q4, z, m.q3), z, m.q2), z, m.q1), z, m.q0);
+    return fma(fma(m.a0, rT, m.a1), rT, q);
+}
+
+// Value and slope of the summed curve at T.  Below 1e-3 K (only a state without physical
+// meaning gets there; the curves' constant-Cp extension has a0 = a1 = 0) the logarithm and the
+// reciprocal are those of 1e-3 K.
+__device__ __forceinline__ void tpg_mix_eval(const TpgMix& m, double T, double& val, double& slope) {
+    const double Tp = fmax(T, 1.0e-3), rT = quick_rcp(Tp), z = T - m.T0;
+    double p = fma(0.2 * m.q4, z, 0.25 * m.q3);
+    p = fma(fma(fma(p, z, (1.0 / 3.0) * m.q2), z, 0.5 * m.q1), z, m.q0);
+    p = fma(m.a0, rT * m.iT0, p);
+    val = fma(p, z, fma(m.a1, log(Tp * m.iT0), m.H0));
+    slope = tpg_mix_slope(m, z, rT);
+}
+
+// The specific energy of a composition at T.
+template <int NSP>
+__device__ __forceinline__ double tpg_energy(const ChemDev& cd, const double* massf, double T) {
+    double y[NSP], Rm = 0.0, u, Cv;
+#pragma unroll
+    for (int i = 0; i < NSP; ++i) {
+        y[i] = massf[i] * cd.R[i];
+        Rm += y[i];
+    }
+    TpgMix m;
+    tpg_mix_build<NSP>(cd, y, Rm, 0.0, T, m);
+    tpg_mix_eval(m, T, u, Cv);
+    return u;
+}
+
+// Cv at T from the curve of a temperature solve (rebuilt if T lies outside its range).
+template <int NSP>
+__device__ __forceinline__ double tpg_Cv(const ChemDev& cd, const double* massf, double T, TpgMix& m) {
+    if (!m.covers(T)) {
+        double y[NSP], Rm = 0.0;
+#pragma unroll
+        for (int i = 0; i < NSP; ++i) {
+            y[i] = massf[i] * cd.R[i];
+            Rm += y[i];
+        }
+        tpg_mix_build<NSP>(cd, y, Rm, 0.0, T, m);
+    }
+    return tpg_mix_slope(m, T - m.T0, quick_rcp(fmax(T, 1.0e-3)));
+}
+
 // therm_perf_gas_mix_eos.d:68-151 with the safeguarded Newton of nm/newton.d:71-140.
 // T and u are in/out as in the reference: every evaluation of the zero function writes T
 // and u, and a converged root then overwrites T, so u ends as the energy of the last
 // evaluated temperature.  Returns false where the reference throws; T is then restored
-// and u = energy(T), which is the state the reference leaves behind.
+// and u = energy(T), which is the state the reference leaves behind.  m: the summed curve of
+// the last evaluation, for the callers that go on to Cv.
 //
 // The reference evaluates u at both ends of the bracket [T1, T2] = [T - 500, T + 500] only
 // for the signs of f = e_tgt - u there (and exact zeros), then starts the Newton iteration
@@ -437,111 +515,116 @@ __device__ __forceinline__ double tpg_Rmix(const ChemDev& cd, const double* mass
 // When the first bound is above and the second below a rounding margin (1e-6 of the
 // energies + 1 J/kg, against ~1e5 J/kg of slope over 500 K), f(T1) > 0 > f(T2) as the
 // reference would compute them: its pass 0 takes the bracket (xH, xL) = (T1, T2) and the
-// same iteration from T, so T and u come out bit for bit the same.  Otherwise (a root far
-// from T, a temperature near the 10 K floor, a negative mass fraction) the ends are
-// evaluated and the reference's passes run as written.  SERIAL as for tpg_energy.
-template <int NSP, bool SERIAL = false>
-__device__ __forceinline__ bool tpg_update_temperature(const ChemDev& cd, const double* massf, double& T, double& u) {
+// same iteration from T.  Otherwise (a root far from T, a temperature near the 10 K floor, a
+// negative mass fraction) the ends are evaluated and the reference's passes run as written.
+// One loop serves every evaluation (at T, at the ends, at the iterates), so the curve's code
+// stands once: a kernel that calls this is 6 to 10 times smaller than with an inlined
+// evaluation at each place, which lone waves of small grids feel as instruction fetches.
+template <int NSP>
+__device__ __forceinline__ bool tpg_update_temperature(const ChemDev& cd, const double* massf, double& T, double& u,
+                                                       TpgMix& m) {
+    enum { AT_T, AT_MIN, AT_MAX, ITERATE };
     const double Tsave = T;
     const double TOL = 1.0e-6;
     const double e_tgt = u;
     const double delT = 1000.0;
     const double T1 = fmax(T - 0.5 * delT, CH_T_MIN);
     const double T2 = T1 + delT;
-    double u0, Cv0;
-    tpg_energy_Cv<NSP, SERIAL>(cd, massf, Tsave, u0, Cv0);
-    bool signs_known;
-    {
-        double Rm = 0.0;
-        bool nonneg = true;
+    double y[NSP], Rm = 0.0;
+    bool nonneg = true;
 #pragma unroll
-        for (int i = 0; i < NSP; ++i) {
-            Rm += massf[i] * cd.R[i];
-            nonneg = nonneg && (massf[i] >= 0.0);
-        }
-        const double g = e_tgt - u0;
-        const double slope = 1.4 * Rm;
-        const double margin = 1.0e-6 * (fabs(e_tgt) + fabs(u0)) + 1.0;
-        signs_known = nonneg && (Tsave - T1 >= 1.0) && (T2 - Tsave >= 1.0) &&
-                      (g + slope * (Tsave - T1) > margin) && (g - slope * (T2 - Tsave) < -margin);
+    for (int i = 0; i < NSP; ++i) {
+        y[i] = massf[i] * cd.R[i];
+        Rm += y[i];
+        nonneg = nonneg && (massf[i] >= 0.0);
     }
-    for (int pass = 0; pass < 2; ++pass) {
-        const double xMin = (pass == 0) ? T1 : CH_T_MIN;
-        const double xMax = (pass == 0) ? T2 : CH_T_MAX;
-        double xL, xH;
-        if (pass == 0 && signs_known) {
-            xH = xMin;
-            xL = xMax;
-        } else {
-            xL = xMin;
-            xH = xMax;
-            T = xL;
-            u = tpg_energy<NSP, SERIAL>(cd, massf, T);
-            const double fL = e_tgt - u;
-            T = xH;
-            u = tpg_energy<NSP, SERIAL>(cd, massf, T);
-            const double fH = e_tgt - u;
-            if ((fL > 0.0 && fH > 0.0) || (fL < 0.0 && fH < 0.0)) continue;
-            if (fL == 0.0) { T = xMin; return true; }
-            if (fH == 0.0) { T = xMax; return true; }
-            if (fL < 0.0) { xL = xMin; xH = xMax; }
-            else { xH = xMin; xL = xMax; }
-        }
-        double rts = Tsave;
-        double dxold = (xMax - xMin);
-        double dx = dxold;
-        T = rts;
+    m.clear();
+    int at = AT_T, pass = 0, j = 0;
+    double u0 = 0.0, Cv0 = 0.0, fL = 0.0, xL = 0.0, xH = 0.0, rts = Tsave, dx = 0.0, dxold = 0.0;
+    while (true) {
         double Cv;
-        if (pass == 0 && signs_known) {
-            Cv = Cv0;
-            u = u0;
-        } else {
-            // the same evaluation again (fewer registers live across the end evaluations)
-            tpg_energy_Cv<NSP, SERIAL>(cd, massf, T, u, Cv);
-        }
+        if (!m.covers(T)) tpg_mix_build<NSP>(cd, y, Rm, 0.0, T, m);
+        tpg_mix_eval(m, T, u, Cv);
         double f0 = e_tgt - u;
-        double df0 = -1.0 * Cv;
-        for (int j = 0; j < 30; ++j) {
-            if ((((rts - xH) * df0 - f0) * ((rts - xL) * df0 - f0) > 0.0) || (fabs(2.0 * f0) > fabs(dxold * df0))) {
-                dxold = dx;
-                dx = 0.5 * (xH - xL);
-                rts = xL + dx;
-                if (xL == rts) { T = rts; return true; }
-            } else {
-                dxold = dx;
-                dx = f0 / df0;
-                double tmp = rts;
-                rts -= dx;
-                if (tmp == rts) { T = rts; return true; }
-            }
-            if (fabs(dx) < TOL) { T = rts; return true; }
-            T = rts;
-            tpg_energy_Cv<NSP, SERIAL>(cd, massf, T, u, Cv);
-            f0 = e_tgt - u;
-            df0 = -1.0 * Cv;
+        bool next_pass = false;
+        if (at == ITERATE) {
             if (f0 < 0.0) xL = rts;
             else xH = rts;
+            next_pass = (++j == 30);
+        } else if (at == AT_T) {
+            u0 = u;
+            Cv0 = Cv;
+            const double slope = 1.4 * Rm;
+            const double margin = 1.0e-6 * (fabs(e_tgt) + fabs(u0)) + 1.0;
+            const bool signs_known = nonneg && (Tsave - T1 >= 1.0) && (T2 - Tsave >= 1.0) &&
+                                     (f0 + slope * (Tsave - T1) > margin) && (f0 - slope * (T2 - Tsave) < -margin);
+            if (!signs_known) {
+                T = T1;
+                at = AT_MIN;
+                continue;
+            }
+            xH = T1;
+            xL = T2;
+            dx = dxold = T2 - T1;
+            at = ITERATE;
+        } else if (at == AT_MIN) {
+            fL = f0;
+            T = (pass == 0) ? T2 : CH_T_MAX;
+            at = AT_MAX;
+            continue;
+        } else {
+            const double xMin = (pass == 0) ? T1 : CH_T_MIN, xMax = (pass == 0) ? T2 : CH_T_MAX, fH = f0;
+            if ((fL > 0.0 && fH > 0.0) || (fL < 0.0 && fH < 0.0)) {
+                next_pass = true;
+            } else {
+                if (fL == 0.0) { T = xMin; return true; }
+                if (fH == 0.0) { T = xMax; return true; }
+                if (fL < 0.0) { xL = xMin; xH = xMax; }
+                else { xH = xMin; xL = xMax; }
+                rts = Tsave;
+                dx = dxold = xMax - xMin;
+                u = u0;
+                Cv = Cv0;
+                f0 = e_tgt - u0;
+                j = 0;
+                at = ITERATE;
+            }
         }
+        if (next_pass) {
+            if (++pass == 2) break;
+            T = CH_T_MIN;
+            at = AT_MIN;
+            continue;
+        }
+        const double df0 = -1.0 * Cv;
+        if ((((rts - xH) * df0 - f0) * ((rts - xL) * df0 - f0) > 0.0) || (fabs(2.0 * f0) > fabs(dxold * df0))) {
+            dxold = dx;
+            dx = 0.5 * (xH - xL);
+            rts = xL + dx;
+            T = rts;
+            if (xL == rts) return true;
+        } else {
+            dxold = dx;
+            dx = quick_div(f0, df0);
+            const double tmp = rts;
+            rts -= dx;
+            T = rts;
+            if (tmp == rts) return true;
+        }
+        if (fabs(dx) < TOL) return true;
     }
     T = Tsave;
-    u = tpg_energy<NSP, SERIAL>(cd, massf, T);
+    u = u0;
     return false;
 }
 
-// therm_perf_gas.d:394-404: frozen sound speed sqrt(gamma * (R T)), gamma = Cp/Cv, with
-// tpg_Cp and tpg_Cv summed from one curve evaluation per species (the same sums).
+// therm_perf_gas.d:394-404: frozen sound speed sqrt(gamma * (R T)), gamma = Cp/Cv, from the
+// curve of a temperature solve.
 template <int NSP>
-__device__ __forceinline__ double tpg_sound_speed(const ChemDev& cd, const double* massf, double T) {
-    const CeaT pw(T, 0.0);
-    double Cp = 0.0, Cv = 0.0;
-#pragma unroll
-    for (int i = 0; i < NSP; ++i) {
-        const double c = cea_Cp(cd.cea[i], pw);
-        Cp += massf[i] * c;
-        Cv += massf[i] * (c - cd.R[i]);
-    }
-    double gamma = Cp / Cv;
-    double R = tpg_Rmix<NSP>(cd, massf);
+__device__ __forceinline__ double tpg_sound_speed(const ChemDev& cd, const double* massf, double T, TpgMix& m) {
+    const double R = tpg_Rmix<NSP>(cd, massf);
+    const double Cv = tpg_Cv<NSP>(cd, massf, T, m);
+    const double gamma = quick_div(Cv + R, Cv);
     return sqrt(gamma * (R * T));
 }
 
@@ -746,17 +829,6 @@ __device__ __forceinline__ double estimate_step_size(const ChemDev& cd, const do
     dt_chem = (dt_chem < 1.0e-15) ? 1.0e-15 : dt_chem;
     return dt_chem;
 }
-
-// a / b for normal operands: the hardware reciprocal refined by one cubic step (residual e:
-// y (1 + e + e^2), relative error e^3), the quotient and one remainder correction, which
-// leaves it within an ulp.  7 instructions, where the compiler's division takes 11 to scale
-// operands that none of the quotients here needs scaled.
-__device__ __forceinline__ double quick_rcp(double b) {
-    const double y = __builtin_amdgcn_rcp(b);
-    const double e = fma(-b, y, 1.0);
-    return fma(y, fma(e, e, e), y);
-}
-__device__ __forceinline__ double quick_div(double a, double b) { return div_by(a, b, quick_rcp(b)); }
 
 // AlphaQssStep.opCall, chemistry_update.d:533-655: predictor, up to maxIters correctors
 // with alpha-bar from p_p, convergence against the first predictor, and the step

@@ -278,7 +278,8 @@ __global__ __launch_bounds__(CHEM_BLOCK) void k_chem_integrate(const ChemDev* __
             if (TIGHT) {
                 double mf[NSP];
                 (void)conc_to_massf<NSP>(cd, c.c0, c.rho, mf);
-                if (tpg_update_temperature<NSP>(cd, mf, c.T, c.u)) eval_rate_constants<NSP, NRM>(cd, c.T, c.kf, c.kb);
+                TpgMix mix;
+                if (tpg_update_temperature<NSP>(cd, mf, c.T, c.u, mix)) eval_rate_constants<NSP, NRM>(cd, c.T, c.kf, c.kb);
                 else fatal = true;
             }
             if (fatal) {
@@ -409,7 +410,8 @@ __global__ __launch_bounds__(CHEM_BLOCK, 3) void k_chem_finish(const ChemDev* __
             Tn = w.Tend[i];
             un = w.uend[i];
         }
-        if (tpg_update_temperature<NSP>(cd, mfn, Tn, un)) {
+        TpgMix mix;
+        if (tpg_update_temperature<NSP>(cd, mfn, Tn, un, mix)) {
             const double Rm = tpg_Rmix<NSP>(cd, mfn);
             pi = r * Rm * Tn;
             Ti = Tn;
@@ -441,6 +443,8 @@ __global__ __launch_bounds__(CHEM_BLOCK) void k_tpg_update(const ChemDev* __rest
 #pragma unroll
     for (int s = 0; s < NSP; ++s) mf[s] = massf[(size_t)s * n + i];
     int stat = 0;
+    TpgMix mix;
+    mix.clear();
     if (mode == 0) {
         const double Rm = tpg_Rmix<NSP>(cd, mf);
         const double denom = Rm * T[i];
@@ -448,7 +452,7 @@ __global__ __launch_bounds__(CHEM_BLOCK) void k_tpg_update(const ChemDev* __rest
         u[i] = tpg_energy<NSP>(cd, mf, T[i]);
     } else if (mode == 1) {
         double Tn = T[i], un = u[i];
-        const bool ok = tpg_update_temperature<NSP>(cd, mf, Tn, un);
+        const bool ok = tpg_update_temperature<NSP>(cd, mf, Tn, un, mix);
         T[i] = Tn;
         u[i] = un;
         if (ok) {
@@ -462,7 +466,7 @@ __global__ __launch_bounds__(CHEM_BLOCK) void k_tpg_update(const ChemDev* __rest
         const double Rm = tpg_Rmix<NSP>(cd, mf);
         p[i] = rho[i] * Rm * T[i];
     }
-    if (stat == 0) a[i] = tpg_sound_speed<NSP>(cd, mf, T[i]);
+    if (stat == 0) a[i] = tpg_sound_speed<NSP>(cd, mf, T[i], mix);
     status[i] = stat;
 }
 

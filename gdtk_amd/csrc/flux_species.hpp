@@ -72,14 +72,11 @@ __device__ __forceinline__ bool scale_mass_fractions(double* massf) {
 
 // update_thermo_from_rhou of the thermally perfect mixture (therm_perf_gas.d:235-239):
 // Newton T(u) from the state's T, then p = rho R_mix T (perf_gas_mix_eos.d:43-49).  The
-// sound speed is not updated, as in the reference's face reconstruction.  The species
-// evaluations run one after another (SERIAL): 162 instead of 202 VGPRs, 3 waves per SIMD
-// instead of 2, and face launches 26 % shorter on the Mach-10 cylinder.  (Holding the face
-// frame and velocity outside registers during the iteration reaches 4 waves per SIMD with
-// a small spill, 1 % faster: not kept.)
+// sound speed is not updated, as in the reference's face reconstruction.  m: the curve of the
+// solve.
 template <int NSP>
-__device__ __forceinline__ bool tpg_update_rhou(const ChemDev& cd, FaceStateT<NSP>& s) {
-    if (!tpg_update_temperature<NSP, true>(cd, s.massf, s.T, s.u)) return false;
+__device__ __forceinline__ bool tpg_update_rhou(const ChemDev& cd, FaceStateT<NSP>& s, TpgMix& m) {
+    if (!tpg_update_temperature<NSP>(cd, s.massf, s.T, s.u, m)) return false;
     s.p = s.rho * tpg_Rmix<NSP>(cd, s.massf) * s.T;
     return true;
 }
@@ -189,12 +186,16 @@ __device__ __forceinline__ bool face_flux_species_pair(const BlockDev& b, const 
         c.prepare(l0, l1, l2, 0.0);
         build(c);
     }
-    if (!tpg_update_rhou<NSP>(cd, st)) copy_cell_state<NSP>(fs, np, c1, v1, st);
+    TpgMix mix;
+    if (!tpg_update_rhou<NSP>(cd, st, mix)) {
+        copy_cell_state<NSP>(fs, np, c1, v1, st);
+        mix.clear();  // another composition
+    }
     st.vel = to_local(to_global(st.vel, g), g);
     // EFM's specific heats, each at its own side.
     const bool shocked = flux_is_adaptive(FC) && ((b.shock[cL0] | b.shock[cR0]) != 0);
     const bool efm = FC == 1 || (FC == 2 && shocked);
-    const double Cv = efm ? tpg_Cv<NSP>(cd, st.massf, st.T) : 0.0;
+    const double Cv = efm ? tpg_Cv<NSP>(cd, st.massf, st.T, mix) : 0.0;
     // swap the two sides' states
     FaceStateT<NSP> o;
     o.rho = pair_swap(st.rho);
@@ -268,7 +269,8 @@ __device__ __forceinline__ int decode_species(const ChemDev& cd, double* U, doub
         massf[i] = U[C::species + i] * dinv;
         rho_s[i] = U[C::species + i];
     }
-    if (tpg_update_temperature<NSP, true>(cd, massf, T, u)) {
+    TpgMix mix;
+    if (tpg_update_temperature<NSP>(cd, massf, T, u, mix)) {
         p = rho * tpg_Rmix<NSP>(cd, massf) * T;
     } else {
         // update_thermo_from_rhoT at the suggested low temperature, then encode_conserved
@@ -286,7 +288,7 @@ __device__ __forceinline__ int decode_species(const ChemDev& cd, double* U, doub
         reencoded = true;
     }
     if (T <= 0.0) return 1;
-    a = tpg_sound_speed<NSP>(cd, massf, T);
+    a = tpg_sound_speed<NSP>(cd, massf, T, mix);
     return 0;
 }
 

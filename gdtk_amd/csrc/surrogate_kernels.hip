@@ -223,7 +223,8 @@ __global__ __launch_bounds__(256) void k_surr_finish(int n, const int* __restric
     const double dc = dtc_in[i];
 #pragma unroll
     for (int s = 0; s < NSP; ++s) mf[s] = massf_new[(size_t)s * n + j];
-    if (!tpg_update_temperature<NSP>(*cd, mf, Tn, un)) {
+    TpgMix mix;
+    if (!tpg_update_temperature<NSP>(*cd, mf, Tn, un, mix)) {
         path[i] = 3;
         const double pv = p_in[i];
         T_out[i] = T[i];
