@@ -249,39 +249,15 @@ __host__ __device__ inline double cea_Cp(const CEADev& c, double T) {
     return c.R * Cp_on_R;
 }
 
-// cea_thermo_curves.d:71-102, with log(T) given (it is the same for every species)
-__host__ __device__ inline double cea_h(const CEADev& c, double T, double logT) {
+// cea_thermo_curves.d:71-102
+__host__ __device__ inline double cea_h(const CEADev& c, double T) {
     if (T < c.T_low) return c.h_low - c.Cp_low * (c.T_low - T);
     if (T > c.T_high) return c.h_high + c.Cp_high * (T - c.T_high);
     double a[9];
     cea_coeffs(c, T, a);
-    double h_on_RT = -a[0] / T + a[1] * logT + a[2] * T + a[3] * T * T / 2.0;
+    double h_on_RT = -a[0] / T + a[1] * log(T) + a[2] * T + a[3] * T * T / 2.0;
     h_on_RT += a[4] * T * T * T / 3.0 + a[5] * T * T * T * T / 4.0 + a[6] * T * T * T * T * T / 5.0 + a[7];
     return c.R * h_on_RT;
-}
-__host__ __device__ inline double cea_h(const CEADev& c, double T) { return cea_h(c, T, log(T)); }
-
-// cea_h and cea_Cp at one temperature from one coefficient selection (the same values as
-// the two separate calls).
-__host__ __device__ inline void cea_h_Cp(const CEADev& c, double T, double logT, double& h, double& Cp) {
-    if (T < c.T_low) {
-        h = c.h_low - c.Cp_low * (c.T_low - T);
-        Cp = c.Cp_low;
-        return;
-    }
-    if (T > c.T_high) {
-        h = c.h_high + c.Cp_high * (T - c.T_high);
-        Cp = c.Cp_high;
-        return;
-    }
-    double a[9];
-    cea_coeffs(c, T, a);
-    double Cp_on_R = a[0] / (T * T) + a[1] / T + a[2] + a[3] * T;
-    Cp_on_R += a[4] * T * T + a[5] * T * T * T + a[6] * T * T * T * T;
-    Cp = c.R * Cp_on_R;
-    double h_on_RT = -a[0] / T + a[1] * logT + a[2] * T + a[3] * T * T / 2.0;
-    h_on_RT += a[4] * T * T * T / 3.0 + a[5] * T * T * T * T / 4.0 + a[6] * T * T * T * T * T / 5.0 + a[7];
-    h = c.R * h_on_RT;
 }
 
 // a / b correctly rounded from y = RN(1 / b): q = RN(a y) lies within an ulp of a / b, the
@@ -302,30 +278,6 @@ struct CeaT {
     __host__ __device__ explicit CeaT(double t, double lg) : T(t), TT(t * t), rT(1.0 / t), rTT(1.0 / (t * t)), logT(lg) {}
 };
 
-// cea_h_Cp with the divisions of cea_thermo_curves.d:56-102 taken through div_by: the same
-// values bit for bit.
-__host__ __device__ inline void cea_h_Cp(const CEADev& c, const CeaT& p, double& h, double& Cp) {
-    const double T = p.T;
-    if (T < c.T_low) {
-        h = c.h_low - c.Cp_low * (c.T_low - T);
-        Cp = c.Cp_low;
-        return;
-    }
-    if (T > c.T_high) {
-        h = c.h_high + c.Cp_high * (T - c.T_high);
-        Cp = c.Cp_high;
-        return;
-    }
-    double a[9];
-    cea_coeffs(c, T, a);
-    double Cp_on_R = div_by(a[0], p.TT, p.rTT) + div_by(a[1], T, p.rT) + a[2] + a[3] * T;
-    Cp_on_R += a[4] * T * T + a[5] * T * T * T + a[6] * T * T * T * T;
-    Cp = c.R * Cp_on_R;
-    double h_on_RT = div_by(-a[0], T, p.rT) + a[1] * p.logT + a[2] * T + a[3] * T * T / 2.0;
-    h_on_RT += div_by(a[4] * T * T * T, 3.0, 1.0 / 3.0) + a[5] * T * T * T * T / 4.0 +
-               div_by(a[6] * T * T * T * T * T, 5.0, 1.0 / 5.0) + a[7];
-    h = c.R * h_on_RT;
-}
 // cea_h and cea_s (cea_thermo_curves.d:71-130) at one temperature from one coefficient
 // selection, log(T) and the reciprocals of CeaT: the same values bit for bit.  The
 // divisor 2 T T of the entropy is exactly 2 TT, whose reciprocal is exactly rTT / 2.
@@ -638,53 +590,88 @@ __device__ __forceinline__ double ch_pow_nusum(double x, double nuSum) {
     return (nuSum == 0.0) ? 1.0 : (nuSum == 1.0) ? x : (nuSum == -1.0) ? 1.0 / x : (nuSum == 2.0) ? x * x : pow(x, nuSum);
 }
 
+// ln t to about twice the working precision's last bit: the rounding of log (up to 9e-16 for a
+// temperature) is what t exp(-log t) differs from 1 by.
+struct LnPair {
+    double hi, lo;
+};
+__device__ __forceinline__ LnPair ln_pair(double t) {
+    LnPair l;
+    l.hi = log(t);
+    l.lo = fma(t, exp(-l.hi), -1.0);
+    return l;
+}
+
+// A T^n exp(-C / T) of rate_constant.d as A exp(n ln T - C / T), rT = 1 / T: one exponential
+// instead of a power and an exponential (a power is four times the exponential's code and
+// time).  The rounding errors of the exponent, some 1e-15 and so of the rate constant where they
+// stay, are summed apart and applied to first order.
+__device__ __forceinline__ double arrhenius(double A, double n, double C, double T, double rT, const LnPair& l) {
+    const double a = n * l.hi, b = C * rT;
+    const double x = a - b, bb = x - a;
+    double e = (a - (x - bb)) - (b + bb);                           // x + e = a - b
+    e += fma(n, l.hi, -a) - fma(C, rT, -b);                         // the products' errors
+    e += fma(n, l.lo, -(b * fma(-T, rT, 1.0)));                     // those of ln T and of 1 / T
+    const double v = A * exp(x);
+    return fma(v, e, v);
+}
+
 // reaction_mechanism.d:50-63 with reaction.d:27-52 (equilibrium constant), 94-143 and
 // rate_constant.d (Arrhenius A T^n exp(-C/T)); T clamped to the mechanism's tempLimits.
 // Participants are summed in ascending species order, the order of the reference's
-// sorted participant list.
+// sorted participant list.  The reactions pass through one copy of the code: unrolled, with
+// its powers, the setup kernel of 5 reactions was 64 KB of code, and the 12 workgroups of a
+// small grid spent 30 us on fetching it.
 template <int NSP, int NRM>
 __device__ __forceinline__ void eval_rate_constants(const ChemDev& cd, double Tin, double* kf, double* kb) {
     double T = Tin;
     if (T < cd.T_lower) T = cd.T_lower;
     if (T > cd.T_upper) T = cd.T_upper;
+    const LnPair lnT = ln_pair(T);
+    const CeaT pw(T, lnT.hi);
     double g[NSP];
-    const CeaT pw(T, log(T));
 #pragma unroll
     for (int s = 0; s < NSP; ++s) {
         double h, sv;
         cea_h_s(cd.cea[s], pw, h, sv);
-        g[s] = h - T * sv;
+        g[s] = (h - T * sv) * cd.M[s];
     }
 #pragma unroll
     for (int ir = 0; ir < NRM; ++ir) {
-        if (ir >= cd.nr) {
-            kf[ir] = 0.0;
-            kb[ir] = 0.0;
-            continue;
-        }
+        kf[ir] = 0.0;
+        kb[ir] = 0.0;
+    }
+    const double RT = CH_R_UNIVERSAL * T, c_atm = CH_P_ATM / RT;
+    const int nr = cd.nr;
+#pragma clang loop unroll(disable)
+    for (int ir = 0; ir < nr; ++ir) {
         const ReacDev& r = cd.r[ir];
-        double Keq = 0.0;
+        double Keq = 1.0;
         if (r.f_from_eq || r.b_from_eq) {
             double dG = 0.0, nuSum = 0.0;
 #pragma unroll
             for (int s = 0; s < NSP; ++s) {
                 if (!r.part[s]) continue;
-                dG += r.nu[s] * g[s] * cd.M[s];
+                dG += r.nu[s] * g[s];
                 nuSum += r.nu[s];
             }
-            double K_p = exp(-dG / (CH_R_UNIVERSAL * T));
-            Keq = K_p * ch_pow_nusum(CH_P_ATM / (CH_R_UNIVERSAL * T), nuSum);
+            Keq = exp(-dG / RT) * ch_pow_nusum(c_atm, nuSum);
         }
-        double kfv, kbv;
-        if (!r.f_from_eq) {
-            kfv = r.fA * pow(T, r.fn) * exp(div_by(-r.fC, T, pw.rT));
-            kbv = r.b_from_eq ? kfv / Keq : r.bA * pow(T, r.bn) * exp(div_by(-r.bC, T, pw.rT));
+        double kfv = 0.0, kbv = 0.0;
+        if (!r.f_from_eq) kfv = arrhenius(r.fA, r.fn, r.fC, T, pw.rT, lnT);
+        if (!r.b_from_eq) kbv = arrhenius(r.bA, r.bn, r.bC, T, pw.rT, lnT);
+        if (r.f_from_eq) kfv = kbv * Keq;
+        if (r.b_from_eq) kbv = kfv / Keq;
+        if constexpr (NRM > 8) {  // arrays of this size live in memory
+            kf[ir] = kfv;
+            kb[ir] = kbv;
         } else {
-            kbv = r.bA * pow(T, r.bn) * exp(div_by(-r.bC, T, pw.rT));
-            kfv = kbv * Keq;
+#pragma unroll
+            for (int j = 0; j < NRM; ++j) {
+                kf[j] = (j == ir) ? kfv : kf[j];
+                kb[j] = (j == ir) ? kbv : kb[j];
+            }
         }
-        kf[ir] = kfv;
-        kb[ir] = kbv;
     }
 }
 

@@ -22,7 +22,7 @@ constexpr int TT_BLOCK = 64;
 // Cells with T <= T_frozen are left as they are.  A reactor failure restores the input state
 // and retries with dt_chem = -1; a second failure, or a Tv iteration that does not converge,
 // fails the cell (status -1, the input state written back).  Outputs may alias inputs.
-template <int NSP, int NRM>
+template <int NSP, int NRM, int WALK>
 __global__ __launch_bounds__(TT_BLOCK) void k_tt_step(const ChemDev* __restrict__ cdp, const TTDev* __restrict__ tdp,
                                                      int n, double dt, const double* rho, const double* T,
                                                      const double* Tv, const double* u, const double* uv,
@@ -48,13 +48,16 @@ __global__ __launch_bounds__(TT_BLOCK) void k_tt_step(const ChemDev* __restrict_
     TTCounts cnt{0, 0};
     int st = 0;
     if (Q0.T > cd.T_frozen) {
-        int r = tt_opcall<NSP, NRM>(cd, td, Q, dt, dc, cnt);
-        if (r == 0) {
+        int r = 0;
+#pragma clang loop unroll(disable)
+        for (int pass = 0; pass < 2 && r == 0; ++pass) {  // the second from the input state, dt_chem = -1
             Q = Q0;
-            dc = -1.0;
-            r = tt_opcall<NSP, NRM>(cd, td, Q, dt, dc, cnt);
+            if (pass == 1) dc = -1.0;
+            r = tt_opcall<NSP, NRM, WALK>(cd, td, Q, dt, dc, cnt);
         }
-        if (r != 1 || !tt_update_from_rhou<NSP>(cd, td, Q)) {
+        TpgMix m;
+        m.clear();
+        if (r != 1 || !tt_update_from_rhou<NSP>(cd, td, Q, m)) {
             st = -1;
             Q = Q0;
         }
@@ -136,11 +139,11 @@ int gdtk_hip_tt_create(const gdtk_tpg_gas* gas, const gdtk_mechanism* mech, cons
             td.sB[s] = td.Cp_tr_rot[s] - R;
             td.A_MW[s] = td.molecular[s] ? prm->A_MW[s] : 0.0;
             if (td.molecular[s] && !(td.A_MW[s] > 0.0)) throw Error(GDTK_ERR_ARG, "A_MW must be positive for molecules");
-            td.mpart[s] = cd.M[s] / TT_AVOGADRO;
+            td.cbar[s] = std::sqrt(8 * TT_BOLTZMANN / (TT_PI * (cd.M[s] / TT_AVOGADRO)));
             for (int c = 0; c < cd.nsp; ++c) {
                 double mu = (cd.M[s] * cd.M[c]) / (cd.M[s] + cd.M[c]);
                 mu *= 1000.0;
-                td.mu_q[s][c] = std::pow(mu, 0.25);
+                td.K_MW[s][c] = std::exp(-0.015 * td.A_MW[s] * std::pow(mu, 0.25) - 18.42);
             }
         }
         td.abs_tol = prm->abs_tol;
@@ -184,14 +187,14 @@ int gdtk_hip_tt_step_device(int tt, int n, const double* rho, const double* T, c
         HIPCHK(hipEventRecord(t.ev[0], s));
         if (n > 0) {
             const dim3 grid((unsigned)((n + TT_BLOCK - 1) / TT_BLOCK));
-            if (t.host.nr <= 6)
-                hipLaunchKernelGGL((k_tt_step<5, 6>), grid, dim3(TT_BLOCK), 0, s, t.dev, t.tdev, n, dt, rho, T, Tv, u,
-                                   uv, p, massf, dt_chem, T_out, Tv_out, u_out, uv_out, p_out, massf_out, dt_chem_out,
-                                   status, t.nsub.p, t.natt.p);
-            else
-                hipLaunchKernelGGL((k_tt_step<5, 8>), grid, dim3(TT_BLOCK), 0, s, t.dev, t.tdev, n, dt, rho, T, Tv, u,
-                                   uv, p, massf, dt_chem, T_out, Tv_out, u_out, uv_out, p_out, massf_out, dt_chem_out,
-                                   status, t.nsub.p, t.natt.p);
+#define GDTK_TT(NR, WK)                                                                                              \
+    hipLaunchKernelGGL((k_tt_step<5, NR, WK>), grid, dim3(TT_BLOCK), 0, s, t.dev, t.tdev, n, dt, rho, T, Tv, u, uv, p, \
+                       massf, dt_chem, T_out, Tv_out, u_out, uv_out, p_out, massf_out, dt_chem_out, status, t.nsub.p, \
+                       t.natt.p)
+            // the structure of the shipped mechanism, or the row walk (at most 8 reactions)
+            if (t.host.walk == WALK_AIR5_GUPTA) GDTK_TT(MechShape<WALK_AIR5_GUPTA>::nr, WALK_AIR5_GUPTA);
+            else GDTK_TT(8, WALK_ROWS);
+#undef GDTK_TT
             HIPCHK(hipGetLastError());
         }
         HIPCHK(hipEventRecord(t.ev[1], s));

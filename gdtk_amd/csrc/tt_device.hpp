@@ -23,8 +23,10 @@ struct TTDev {
     double Cp_tr_rot[CH_MAX_SP], del_hf[CH_MAX_SP];
     double sA[CH_MAX_SP], sB[CH_MAX_SP];      // Cp_tr_rot T_REF - del_hf, Cp_tr_rot - R
     double A_MW[CH_MAX_SP];                   // Millikan-White A (0 for atoms)
-    double mu_q[CH_MAX_SP][CH_MAX_SP];        // pow(mu_ij in g/mol, 0.25)
-    double mpart[CH_MAX_SP];                  // M / N_A (kg)
+    // exp(-0.015 A_s mu_sc^(1/4) - 18.42), mu_sc the reduced mass in g/mol: the part of the
+    // correlation that does not depend on T
+    double K_MW[CH_MAX_SP][CH_MAX_SP];
+    double cbar[CH_MAX_SP];                   // sqrt(8 k / (pi m)), m = M / N_A
     double abs_tol, rel_tol;                  // energy step
 };
 
@@ -35,67 +37,63 @@ struct TTCell {
     double massf[NSP];
 };
 
-// two_temperature_air.d:573-583, one species at Tve with log(Tve) given
-__device__ __forceinline__ double tt_ev(const ChemDev& cd, const TTDev& td, int s, double Tve, double logTve) {
-    const double h_at_Tve = cea_h(cd.cea[s], Tve, logTve);
-    return h_at_Tve - td.Cp_tr_rot[s] * (Tve - TT_T_REF) - td.del_hf[s];
-}
-
-// :584-591 and :673-680 at one temperature (one coefficient selection per species)
+// The vibro-electronic energy of a weighted mixture, sum of y_s / R_s e_ve,s(T) with
+// e_ve = h - Cp_tr,rot (T - T_REF) - del_hf (two_temperature_air.d:573-591, its slope
+// :673-680), as one curve (TpgMix); w: weights per unit mass.
 template <int NSP>
-__device__ __forceinline__ void tt_ev_cv_mix(const ChemDev& cd, const TTDev& td, const double* massf, double Tve,
-                                             double& e, double& cv) {
-    const CeaT pw(Tve, log(Tve));
-    e = 0.0;
-    cv = 0.0;
+__device__ __forceinline__ void tt_ev_build(const ChemDev& cd, const TTDev& td, const double* w, double T, TpgMix& m) {
+    double y[NSP], lin = 0.0, cst = 0.0;
 #pragma unroll
     for (int s = 0; s < NSP; ++s) {
-        double h, Cp;
-        cea_h_Cp(cd.cea[s], pw, h, Cp);
-        e += massf[s] * (h - td.Cp_tr_rot[s] * (Tve - TT_T_REF) - td.del_hf[s]);
-        cv += massf[s] * (Cp - td.Cp_tr_rot[s]);
+        y[s] = w[s] * cd.R[s];
+        lin += w[s] * td.Cp_tr_rot[s];
+        cst += w[s] * td.sA[s];
     }
+    tpg_mix_build<NSP>(cd, y, lin, cst, T, m);
 }
 
 // :698-740 vibElecTemperature: Newton from the state's Tv; false where the reference throws.
+// m: the mixture's curve, kept from one call to the next while the mass fractions stay (the six
+// stages of an energy step share one build).
 template <int NSP>
 __device__ __forceinline__ bool tt_vib_temperature(const ChemDev& cd, const TTDev& td, const TTCell<NSP>& Q,
-                                                   double& Tv_out) {
+                                                   TpgMix& m, double& Tv_out) {
     const int MAX_ITERATIONS = 20;
     const double TOL = 1.0e-6, E_TOL = 0.01;
     double T_guess = Q.Tv;
-    double e, Cv;
-    tt_ev_cv_mix<NSP>(cd, td, Q.massf, T_guess, e, Cv);
-    double f_guess = e - Q.uv;
-    if (fabs(f_guess) < E_TOL) {
-        Tv_out = Q.Tv;
-        return true;
-    }
-    int count = 0;
-    for (int iter = 0; iter < MAX_ITERATIONS; ++iter) {
-        const double dT = -f_guess / Cv;
+    for (int count = 0;; ++count) {
+        double e, Cv;
+        if (!m.covers(T_guess)) tt_ev_build<NSP>(cd, td, Q.massf, T_guess, m);
+        tpg_mix_eval(m, T_guess, e, Cv);
+        const double f_guess = e - Q.uv;
+        if (count == 0 && fabs(f_guess) < E_TOL) {
+            Tv_out = Q.Tv;
+            return true;
+        }
+        if (count == MAX_ITERATIONS) break;
+        const double dT = quick_div(-f_guess, Cv);
         T_guess += dT;
-        if (fabs(dT) < TOL) break;
-        tt_ev_cv_mix<NSP>(cd, td, Q.massf, T_guess, e, Cv);
-        f_guess = e - Q.uv;
-        ++count;
+        if (fabs(dT) < TOL) {
+            Tv_out = T_guess;
+            return true;
+        }
     }
-    Tv_out = T_guess;
-    return count != MAX_ITERATIONS;
+    return false;
 }
 
 // :275-291 update_thermo_from_rhou: T by direct inversion, Tv by Newton, p (perf_gas_mix_eos.d:43-49)
 template <int NSP>
-__device__ __forceinline__ bool tt_update_from_rhou(const ChemDev& cd, const TTDev& td, TTCell<NSP>& Q) {
+__device__ __forceinline__ bool tt_update_from_rhou(const ChemDev& cd, const TTDev& td, TTCell<NSP>& Q,
+                                                    TpgMix& m) {
     double sumA = 0.0, sumB = 0.0;
 #pragma unroll
     for (int s = 0; s < NSP; ++s) {
         sumA += Q.massf[s] * td.sA[s];
         sumB += Q.massf[s] * td.sB[s];
     }
-    Q.T = (Q.u + sumA) / sumB;
+    Q.T = quick_div(Q.u + sumA, sumB);
     double Tv;
-    if (!tt_vib_temperature<NSP>(cd, td, Q, Tv)) return false;
+    if (!tt_vib_temperature<NSP>(cd, td, Q, m, Tv)) return false;
     Q.Tv = Tv;
     double Rmix = 0.0;
 #pragma unroll
@@ -105,133 +103,147 @@ __device__ __forceinline__ bool tt_update_from_rhou(const ChemDev& cd, const TTD
 }
 
 // reaction_mechanism.d:50-63 with rate_constant.d:72-75 (Arrhenius at T) and :391-394
-// (Park at T^s Tv^(1-s)); T clamped to the temperature limits, Tv not.
+// (Park at T^s Tv^(1-s)); T clamped to the temperature limits, Tv not.  The logarithm of
+// Park's temperature is the weighted sum of the two, kept as a pair like theirs.  The reactions
+// pass through one copy of the code.
 template <int NRM>
 __device__ __forceinline__ void tt_rate_constants(const ChemDev& cd, double Tin, double Tv, double* kf, double* kb) {
     double T = Tin;
     if (T < cd.T_lower) T = cd.T_lower;
     if (T > cd.T_upper) T = cd.T_upper;
+    const LnPair lnT = ln_pair(T), lnTv = ln_pair(Tv);
+    const double rT = quick_rcp(T);
 #pragma unroll
     for (int ir = 0; ir < NRM; ++ir) {
-        if (ir >= cd.nr) {
-            kf[ir] = 0.0;
-            kb[ir] = 0.0;
-            continue;
-        }
+        kf[ir] = 0.0;
+        kb[ir] = 0.0;
+    }
+    const int nr = cd.nr;
+#pragma clang loop unroll(disable)
+    for (int ir = 0; ir < nr; ++ir) {
         const ReacDev& r = cd.r[ir];
-        double Tf = T, Tb = T;
-        if (r.f_park) Tf = pow(T, r.f_s) * pow(Tv, 1.0 - r.f_s);
-        if (r.b_park) Tb = pow(T, r.b_s) * pow(Tv, 1.0 - r.b_s);
-        kf[ir] = r.fA * pow(Tf, r.fn) * exp(-r.fC / Tf);
-        kb[ir] = r.bA * pow(Tb, r.bn) * exp(-r.bC / Tb);
+        double k[2];
+#pragma clang loop unroll(disable)
+        for (int way = 0; way < 2; ++way) {
+            const double A = way ? r.bA : r.fA, n = way ? r.bn : r.fn, C = way ? r.bC : r.fC;
+            double Tk = T, rTk = rT;
+            LnPair l = lnT;
+            if (way ? r.b_park : r.f_park) {
+                const double p = way ? r.b_s : r.f_s, q = 1.0 - p;
+                const double a = p * lnT.hi, b = q * lnTv.hi;
+                l.hi = a + b;
+                const double bb = l.hi - a;
+                l.lo = (a - (l.hi - bb)) + (b - bb) + fma(p, lnT.hi, -a) + fma(q, lnTv.hi, -b);
+                l.lo = fma(p, lnT.lo, fma(q, lnTv.lo, l.lo));
+                const double ex = exp(l.hi);
+                Tk = fma(ex, l.lo, ex);
+                rTk = quick_rcp(Tk);
+            }
+            const double v = arrhenius(A, n, C, Tk, rTk, l);
+            if (way == 0) k[0] = v;
+            else k[1] = v;
+        }
+#pragma unroll
+        for (int j = 0; j < NRM; ++j) {
+            kf[j] = (j == ir) ? k[0] : kf[j];
+            kb[j] = (j == ir) ? k[1] : kb[j];
+        }
     }
 }
 
 // two_temperature_air_kinetics.d:398-441 (relaxation time of molecular species isp, from the
 // mole fractions and number densities of evalRate) and :444-460 + :521-543 (the exchange
-// rate of u_v: Landau-Teller per molecular species plus the chemical source, whose reaction
-// rates wf, wb are those of the chemistry step's last evaluation).
-template <int NSP, int NRM>
+// rate of u_v: Landau-Teller per molecular species plus the chemical source).  g: per species
+// the net mass rate per unit mass of mixture of the chemistry step's last evaluation, which
+// the source multiplies with e_ve,s(Tv).
+//
+// What the reference evaluates per species is summed first, since e_ve enters linearly:
+//   sum over molecules of w_s (e_ve,s(T) - e_ve,s(Tv)) + sum of g_s e_ve,s(Tv),
+//   w_s = massf_s / tau_s,
+// are two curves, one at T with weights w and one at Tv with weights g - w (a pass of one loop
+// each).  1 / tau_s with tau_s = tauMW + tauP is c_s / (tauMW c_s + 1), c_s = 1 / tauP; the
+// Millikan-White exponential is exp(A_s T^(-1/3)) times a constant per pair (3 exponentials a
+// rate, not 15).
+template <int NSP>
 __device__ __forceinline__ double tt_eval_rate(const ChemDev& cd, const TTDev& td, const TTCell<NSP>& Q,
-                                               const double* wf, const double* wb) {
-    double M_inv = 0.0;
-#pragma unroll
-    for (int s = 0; s < NSP; ++s) M_inv += Q.massf[s] / cd.M[s];
-    const double mixMolMass = 1.0 / M_inv;
-    double molef[NSP], numden[NSP];
+                                               const double* g) {
+    double moles[NSP], nsum = 0.0;  // mol per kg
 #pragma unroll
     for (int s = 0; s < NSP; ++s) {
-        molef[s] = Q.massf[s] * mixMolMass / cd.M[s];
-        numden[s] = TT_AVOGADRO * Q.massf[s] * Q.rho / cd.M[s];
+        moles[s] = quick_div(Q.massf[s], cd.M[s]);
+        nsum += moles[s];
     }
-    const double lgT = log(Q.T), lgTv = log(Q.Tv);
-    const double Tm13 = pow(Q.T, -1. / 3);
-    double evTv[NSP];
-#pragma unroll
-    for (int s = 0; s < NSP; ++s) evTv[s] = tt_ev(cd, td, s, Q.Tv, lgTv);
-    double rate = 0.0;
+    const double Tm13 = rcbrt(Q.T), sqrtT = sqrt(Q.T);
+    const double sigma_s = 1e-20, navo = TT_AVOGADRO * Q.rho;
+    double w[NSP];
 #pragma unroll
     for (int s = 0; s < NSP; ++s) {
+        w[s] = 0.0;
         if (!td.molecular[s]) continue;
-        double totalND = 0.0, sum = 0.0;
+        double total = 0.0, sum = 0.0;
 #pragma unroll
         for (int c = 0; c < NSP; ++c) {
-            if (molef[c] >= TT_SMALL_MOLE_FRACTION) {
-                const double nd = numden[c];
-                sum += nd * exp(td.A_MW[s] * (Tm13 - 0.015 * td.mu_q[s][c]) - 18.42);
-                totalND += nd;
+            if (moles[c] >= TT_SMALL_MOLE_FRACTION * nsum) {
+                sum = fma(moles[c], td.K_MW[s][c], sum);
+                total += moles[c];
             }
         }
-        double tauMW = sum / totalND;
-        tauMW *= CH_P_ATM / Q.p;
-        const double cBar_s = sqrt(8 * TT_BOLTZMANN * Q.T / (TT_PI * td.mpart[s]));
-        const double sigma_s = 1e-20;
-        const double tauP = 1.0 / (sigma_s * cBar_s * numden[s]);
-        const double tau = tauMW + tauP;
-        const double evStar = tt_ev(cd, td, s, Q.T, lgT);
-        rate += Q.massf[s] * (evStar - evTv[s]) / tau;
+        const double tauMW = quick_div(sum * exp(td.A_MW[s] * Tm13) * CH_P_ATM, total * Q.p);
+        const double coll = sigma_s * (td.cbar[s] * sqrtT) * (navo * moles[s]);  // 1 / tauP
+        w[s] = Q.massf[s] * quick_div(coll, fma(tauMW, coll, 1.0));
     }
-    // EnergyReactiveSourceTerm: per species, the net molar rate over the reactions it takes
-    // part in (reaction order), times M and e_ve(Tv); then per unit mass of mixture.
-    double src = 0.0;
+    double rate = 0.0;
+#pragma clang loop unroll(disable)
+    for (int k = 0; k < 2; ++k) {
+        const double Tk = (k == 0) ? Q.T : Q.Tv;
+        TpgMix m;
+        double e, slope;
+        tt_ev_build<NSP>(cd, td, w, Tk, m);
+        tpg_mix_eval(m, Tk, e, slope);
+        rate += e;
 #pragma unroll
-    for (int s = 0; s < NSP; ++s) {
-        double chemRate = 0.0;
-#pragma unroll
-        for (int ir = 0; ir < NRM; ++ir) {
-            if (ir >= cd.nr) break;
-            const RateRow& rr = cd.rr[ir];
-            if ((rr.code[s] & 15) == 0) continue;  // not a participant
-            const int nu = dense_row_nu<WALK_ROWS>(rr, ir, s);
-            const double prod = (nu > 0) ? nu * wf[ir] : (nu < 0) ? -nu * wb[ir] : 0.0;
-            const double loss = (nu > 0) ? nu * wb[ir] : (nu < 0) ? -nu * wf[ir] : 0.0;
-            chemRate += prod - loss;
-        }
-        chemRate *= cd.M[s];
-        src += chemRate * evTv[s];
+        for (int s = 0; s < NSP; ++s) w[s] = g[s] - w[s];
     }
-    src /= Q.rho;
-    rate += src;
     return rate;
 }
 
+// Cash-Karp: row st of the tableau's stage weights (the last row is the fifth-order result) and
+// the fourth-order weights.
+__device__ constexpr double TT_CK[6][6] = {{1. / 5., 0, 0, 0, 0, 0},
+                                           {3. / 40., 9. / 40., 0, 0, 0, 0},
+                                           {3. / 10., -9. / 10., 6. / 5., 0, 0, 0},
+                                           {-11. / 54., 5. / 2., -70. / 27., 35. / 27., 0, 0},
+                                           {1631. / 55296., 175. / 512., 575. / 13824., 44275. / 110592., 253. / 4096., 0},
+                                           {37. / 378., 0, 250. / 621., 125. / 594., 0, 512. / 1771.}};
+
 // :546-706 EnergyStep: Cash-Karp on u_v at fixed total energy uTotal; every stage ends in
 // update_thermo_from_rhou.  Returns 1 success, 0 failure (the state keeps the last stage,
-// as in the reference), -1 where the Tv iteration fails.
-template <int NSP, int NRM>
+// as in the reference), -1 where the Tv iteration fails.  The six stages are passes of one
+// loop: unrolled, with the relaxation rate and the Newton iteration inlined six times, the
+// kernel was 1.4 MB of code, and its waves waited for instructions.
+template <int NSP>
 __device__ __forceinline__ int tt_energy_step(const ChemDev& cd, const TTDev& td, TTCell<NSP>& Q, double uTotal,
-                                              double h, double& hSuggest, const double* wf, const double* wb) {
-    const double a21 = 1. / 5., a31 = 3. / 40., a32 = 9. / 40., a41 = 3. / 10., a42 = -9. / 10., a43 = 6. / 5.,
-                 a51 = -11. / 54., a52 = 5. / 2., a53 = -70. / 27., a54 = 35. / 27., a61 = 1631. / 55296.,
-                 a62 = 175. / 512., a63 = 575. / 13824., a64 = 44275. / 110592., a65 = 253. / 4096.;
-    const double b51 = 37. / 378., b53 = 250. / 621., b54 = 125. / 594., b56 = 512. / 1771., b41 = 2825. / 27648.,
-                 b43 = 18575. / 48384., b44 = 13525. / 55296., b45 = 277. / 14336., b46 = 1.0 / 4.0;
+                                              double h, double& hSuggest, const double* g, TpgMix& m) {
+    const double b41 = 2825. / 27648., b43 = 18575. / 48384., b44 = 13525. / 55296., b45 = 277. / 14336.,
+                 b46 = 1.0 / 4.0;
     const double uv0 = Q.uv;
-    const double k1 = tt_eval_rate<NSP, NRM>(cd, td, Q, wf, wb);
-    Q.uv = uv0 + h * (a21 * k1);
-    Q.u = uTotal - Q.uv;
-    if (!tt_update_from_rhou<NSP>(cd, td, Q)) return -1;
-    const double k2 = tt_eval_rate<NSP, NRM>(cd, td, Q, wf, wb);
-    Q.uv = uv0 + h * (a31 * k1 + a32 * k2);
-    Q.u = uTotal - Q.uv;
-    if (!tt_update_from_rhou<NSP>(cd, td, Q)) return -1;
-    const double k3 = tt_eval_rate<NSP, NRM>(cd, td, Q, wf, wb);
-    Q.uv = uv0 + h * (a41 * k1 + a42 * k2 + a43 * k3);
-    Q.u = uTotal - Q.uv;
-    if (!tt_update_from_rhou<NSP>(cd, td, Q)) return -1;
-    const double k4 = tt_eval_rate<NSP, NRM>(cd, td, Q, wf, wb);
-    Q.uv = uv0 + h * (a51 * k1 + a52 * k2 + a53 * k3 + a54 * k4);
-    Q.u = uTotal - Q.uv;
-    if (!tt_update_from_rhou<NSP>(cd, td, Q)) return -1;
-    const double k5 = tt_eval_rate<NSP, NRM>(cd, td, Q, wf, wb);
-    Q.uv = uv0 + h * (a61 * k1 + a62 * k2 + a63 * k3 + a64 * k4 + a65 * k5);
-    Q.u = uTotal - Q.uv;
-    if (!tt_update_from_rhou<NSP>(cd, td, Q)) return -1;
-    const double k6 = tt_eval_rate<NSP, NRM>(cd, td, Q, wf, wb);
-    Q.uv = uv0 + h * (b51 * k1 + b53 * k3 + b54 * k4 + b56 * k6);
-    Q.u = uTotal - Q.uv;
-    if (!tt_update_from_rhou<NSP>(cd, td, Q)) return -1;
-    const double errEst = Q.uv - (uv0 + h * (b41 * k1 + b43 * k3 + b44 * k4 + b45 * k5 + b46 * k6));
+    double k[6];
+#pragma unroll
+    for (int j = 0; j < 6; ++j) k[j] = 0.0;
+#pragma clang loop unroll(disable)
+    for (int st = 0; st < 6; ++st) {
+        const double ks = tt_eval_rate<NSP>(cd, td, Q, g);
+        double sum = 0.0;
+#pragma unroll
+        for (int j = 0; j < 6; ++j) {
+            k[j] = (j == st) ? ks : k[j];
+            sum += TT_CK[st][j] * k[j];
+        }
+        Q.uv = uv0 + h * sum;
+        Q.u = uTotal - Q.uv;
+        if (!tt_update_from_rhou<NSP>(cd, td, Q, m)) return -1;
+    }
+    const double errEst = Q.uv - (uv0 + h * (b41 * k[0] + b43 * k[2] + b44 * k[3] + b45 * k[4] + b46 * k[5]));
     const double sk = td.abs_tol + td.rel_tol * fmax(fabs(uv0), fabs(Q.uv));
     const double err = fabs(errEst / sk);
     const double maxscale = 10.0, minscale = 0.2, safe = 0.9, alpha = 0.2;
@@ -269,7 +281,7 @@ struct TTCounts {
 // two_temperature_air_kinetics.d:162-358 opCall: 1 success, 0 where the reference throws
 // ThermochemicalReactorUpdateException (the caller restores the input state), -1 where a
 // GasModelException escapes (a failed Tv iteration, a bad density).
-template <int NSP, int NRM>
+template <int NSP, int NRM, int WALK>
 __device__ __forceinline__ int tt_opcall(const ChemDev& cd, const TTDev& td, TTCell<NSP>& Q, double tInterval,
                                          double& dtSuggest, TTCounts& cnt) {
     const double DT_INCREASE_PERCENT = 10.0, DT_REDUCTION_FACTOR = 10.0, H_MIN = 1.0e-15,
@@ -283,11 +295,13 @@ __device__ __forceinline__ int tt_opcall(const ChemDev& cd, const TTDev& td, TTC
         concOut[s] = 0.0;
     }
     const double uTotal = Q.u + Q.uv;
+    TpgMix m;  // the mixture's e_ve curve of the current mass fractions
+    m.clear();
     double kf[NRM], kb[NRM];
     tt_rate_constants<NRM>(cd, Q.T, Q.Tv, kf, kb);
     double t = 0.0, h, dtSave = 0.0;
     if (dtSuggest > tInterval) h = tInterval;
-    else if (dtSuggest <= 0.0) h = estimate_step_size<NSP, NRM, WALK_ROWS>(cd, kf, kb, conc0);
+    else if (dtSuggest <= 0.0) h = estimate_step_size<NSP, NRM, WALK>(cd, kf, kb, conc0);
     else h = dtSuggest;
     int cycle = 0;
     for (; cycle < cd.maxSubcycles; ++cycle) {
@@ -297,23 +311,21 @@ __device__ __forceinline__ int tt_opcall(const ChemDev& cd, const TTDev& td, TTC
         for (; attempt < cd.maxAttempts; ++attempt) {
             ++cnt.attempts;
             double yLast[NSP];
-            const bool r1 = rkf_step<NSP, NRM, WALK_ROWS>(cd, kf, kb, conc0, h, concOut, dtSuggest, yLast);
+            const bool r1 = rkf_step<NSP, NRM, WALK>(cd, kf, kb, conc0, h, concOut, dtSuggest, yLast);
             // the reaction rates of the chemistry step's last evaluation
-            double wf[NRM], wb[NRM], c2[NSP];
+            // (EnergyReactiveSourceTerm: production less loss in reaction order, times M, per
+            // unit mass of mixture)
+            double q[NSP], L[NSP], g[NSP];
+            eval_split_rates<NSP, NRM, WALK>(cd, kf, kb, yLast, q, L);
 #pragma unroll
-            for (int s = 0; s < NSP; ++s) c2[s] = yLast[s] * yLast[s];
-#pragma unroll
-            for (int ir = 0; ir < NRM; ++ir) {
-                wf[ir] = 0.0;
-                wb[ir] = 0.0;
-                if (ir < cd.nr) dense_row_rates<NSP, WALK_ROWS>(cd.rr[ir], ir, kf[ir], kb[ir], yLast, c2, wf[ir], wb[ir]);
-            }
-            const int r2 = tt_energy_step<NSP, NRM>(cd, td, Q, uTotal, h, dtSuggest, wf, wb);
+            for (int s = 0; s < NSP; ++s) g[s] = quick_div((q[s] - L[s]) * cd.M[s], Q.rho);
+            const int r2 = tt_energy_step<NSP>(cd, td, Q, uTotal, h, dtSuggest, g, m);
             if (r2 < 0) return -1;
             const bool ok = r1 && (r2 == 1);
             bool passes = true;
             if (ok) {
                 tt_conc_to_massf<NSP>(cd, concOut, Q);
+                m.clear();
                 const double massfTotal = phobos_sum<NSP>(Q.massf);
                 if (fabs(massfTotal - 1.0) > ALLOWABLE_MASSF_ERROR) passes = false;
             }
@@ -332,8 +344,9 @@ __device__ __forceinline__ int tt_opcall(const ChemDev& cd, const TTDev& td, TTC
         ++cnt.substeps;
         if (cd.tight) {
             tt_conc_to_massf<NSP>(cd, conc0, Q);
+            m.clear();
             Q.u = uTotal - Q.uv;
-            if (!tt_update_from_rhou<NSP>(cd, td, Q)) return -1;
+            if (!tt_update_from_rhou<NSP>(cd, td, Q, m)) return -1;
             tt_rate_constants<NRM>(cd, Q.T, Q.Tv, kf, kb);
         }
         if (t >= tInterval) {
