@@ -117,6 +117,19 @@ struct SideDev {
     int64_t start;
 };
 
+// One ghost cell of the fill, resolved once: where it is, where its state comes from (another
+// block's cell, the block's own, or a row of constants with plane stride 1), the frame of the
+// wall that mirrors its velocity, and the shock indicators' places (adaptive calculators).
+struct alignas(64) GhostRec {
+    double* dst;
+    const double* src;
+    const double* wall;  // frame of the slip wall's face, null otherwise
+    unsigned char* sdst;
+    const unsigned char* ssrc;  // null: indicator 0 (inflow)
+    int npd, nps, nface;  // plane strides of the destination, the source and the frame
+    int pad_;
+};
+
 // The faces of every direction of every block in one launch: per direction d, the first
 // launch index of each block's faces (multiples of the 256-thread workgroup) and the
 // direction's launch size; the directions follow each other in the launch.

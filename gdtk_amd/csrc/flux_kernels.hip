@@ -25,73 +25,44 @@ __device__ __forceinline__ int64_t ghost_pidx(const BlockDev& b, int side, int a
     return pidx(b, a, bb, b.nkc + layer);
 }
 
-// Ghost-cell effect of one ghost cell (layer `layer` at in-face position (a, bb) of side
-// `side`) for the boundary kinds that read the block's own cells:
-// internal_copy_then_reflect.d:111-134, flow_state_copy.d:92-107,
-// extrapolate_copy.d:124-140 (xOrder 0).
-// With `shock`, the ghost cell also takes its source's shock indicator (0 for an inflow), as
-// the reference's ghost cells copy the whole flow state, fs.S included.
-__device__ __forceinline__ void ghost_one(const BlockDev& b, double* fs, int side, int a, int bb, int layer,
-                                          bool shock) {
-    int i0, j0, k0;  // face location in the side
-    int d;           // index direction normal to the side
-    int fi, fj, fk;  // face index
-    if (side <= 1) {
-        d = 0; j0 = a; k0 = bb; i0 = 0;
-        fi = (side == 0) ? 0 : b.nic; fj = j0; fk = k0;
-    } else if (side <= 3) {
-        d = 1; i0 = a; k0 = bb; j0 = 0;
-        fi = i0; fj = (side == 2) ? 0 : b.njc; fk = k0;
-    } else {
-        d = 2; i0 = a; j0 = bb; k0 = 0;
-        fi = i0; fj = j0; fk = (side == 4) ? 0 : b.nkc;
-    }
+// The record of one ghost cell (layer `layer` at in-face position (a, bb) of side `side`) for the
+// boundary kinds that read the block's own cells: internal_copy_then_reflect.d:111-134,
+// flow_state_copy.d:92-107, extrapolate_copy.d:124-140 (xOrder 0).
+__device__ __forceinline__ GhostRec ghost_own(const BlockDev& b, int side, int a, int bb, int layer) {
+    const int d = side / 2;
     const bool lo = (side % 2) == 0;
     const int nd = (d == 0) ? b.nic : (d == 1) ? b.njc : b.nkc;
-    // Ghost position and interior source position along d.
-    int g_at = lo ? (-1 - layer) : (nd + layer);
-    int kind = b.bc_kind[side];
-    int src_at;
-    if (kind == BC_SLIP_WALL) src_at = lo ? layer : (nd - 1 - layer);
-    else src_at = lo ? 0 : (nd - 1);
-    auto at = [&](int s) -> int64_t {
-        if (d == 0) return pidx(b, s, j0, k0);
-        if (d == 1) return pidx(b, i0, s, k0);
-        return pidx(b, i0, j0, s);
-    };
-    int64_t g = at(g_at);
-    const int64_t np = b.npad;
+    const int kind = b.bc_kind[side];
+    double* fs = const_cast<double*>(b.fs_in);
+    const int64_t g = ghost_pidx(b, side, a, bb, layer);
+    GhostRec r{};
+    r.dst = fs + g;
+    r.npd = r.nps = (int)b.npad;
+    r.sdst = b.shock ? b.shock + g : nullptr;
     if (kind == BC_INFLOW_SUPERSONIC) {
-        for (int f = 0; f < b.nfs; ++f) fs[g + f * np] = b.inflow[side][f];
-        if (shock) b.shock[g] = 0;
-        return;
+        r.src = b.inflow[side];
+        r.nps = 1;
+        return r;
     }
-    if (kind == BC_EXCHANGE) return;
-    int64_t s = at(src_at);
-    for (int f = 0; f < b.nfs; ++f) fs[g + f * np] = fs[s + f * np];
-    if (shock) b.shock[g] = b.shock[s];
+    const int from = (kind == BC_SLIP_WALL) ? layer : 0;  // cells inside the side
+    const int64_t s = ghost_pidx(b, side, a, bb, -1 - from);
+    r.src = fs + s;
+    r.ssrc = b.shock ? b.shock + s : nullptr;
     if (kind == BC_SLIP_WALL) {
-        // ghost_cell.d:33-43
-        FaceGeom fg = load_face(b.fgeom[d], b.nface[d], face_index(b, d, fi, fj, fk));
-        Vec3d v{fs[s + FS_VX * np], fs[s + FS_VY * np], fs[s + FS_VZ * np]};
-        Vec3d l = to_local(v, fg);
-        l.x = -(l.x);
-        Vec3d w = to_global(l, fg);
-        fs[g + FS_VX * np] = w.x;
-        fs[g + FS_VY * np] = w.y;
-        fs[g + FS_VZ * np] = w.z;
+        const int pos = lo ? 0 : nd;
+        const int64_t f = (d == 0) ? face_index(b, 0, pos, a, bb) : (d == 1) ? face_index(b, 1, a, pos, bb)
+                                                                             : face_index(b, 2, a, bb, pos);
+        r.wall = b.fgeom[d] + f;
+        r.nface = (int)b.nface[d];
     }
+    return r;
 }
 
-// Ghost cells of every side of every block in one launch: full-face-copy exchange from the
-// source block's cells (simcore_exchange.d:96-135 -> full_face_copy.d:1888-1900, the
-// same-process copy of the whole flow state) and the other ghost-cell effects.  Each block
-// record's fs_in is the flow-state copy this stage reads, so the ghost cells are written
-// there.  mode 1 copies the exchange sides' cell lengths instead (the geometry exchange
-// of full_face_copy.d:1576-1625, done once); mode 2 is mode 0 with the shock indicators
-// (the fill that precedes shock detection).
-__global__ void k_ghost_batch(const BlockDev* __restrict__ tab, const SideDev* __restrict__ sides, int nsides,
-                              int64_t total, int mode) {
+// Ghost cells of every side of every block: the records of the fill for one flow-state copy
+// (the blocks' fs_in), made once, or (lengths) the geometry exchange of
+// full_face_copy.d:1576-1625, the cell lengths of exchange sides, done once too.
+__global__ void k_ghost_setup(const BlockDev* __restrict__ tab, const SideDev* __restrict__ sides, int nsides,
+                              int64_t total, GhostRec* __restrict__ rec, int lengths) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= total) return;
     int lo = 0, hi = nsides - 1;
@@ -106,23 +77,63 @@ __global__ void k_ghost_batch(const BlockDev* __restrict__ tab, const SideDev* _
     const int64_t face = r / NGHOST;
     const int a = (int)(face % sd.na), bb = (int)(face / sd.na);
     const BlockDev& b = tab[sd.blk];
-    if (sd.kind == BC_EXCHANGE) {
-        const BlockDev& o = tab[sd.oblk];
-        int i, j, k;
-        ffc_source(b.dims, sd.side, sd.oside, sd.orient, a, bb, layer, o.nic, o.njc, o.nkc, i, j, k);
-        const int64_t src = pidx(o, i, j, k);
-        const int64_t dst = ghost_pidx(b, sd.side, a, bb, layer);
-        if (mode != 1) {
-            double* fs = const_cast<double*>(b.fs_in);
-            for (int f = 0; f < b.nfs; ++f) fs[dst + f * b.npad] = o.fs_in[src + f * o.npad];
-            if (mode == 2) b.shock[dst] = o.shock[src];
-        } else {
-            double* len = const_cast<double*>(b.len);
-            for (int f = 0; f < 3; ++f) len[dst + f * b.npad] = o.len[src + f * o.npad];
-        }
-    } else if (mode != 1) {
-        ghost_one(b, const_cast<double*>(b.fs_in), sd.side, a, bb, layer, mode == 2);
+    if (sd.kind != BC_EXCHANGE) {
+        if (!lengths) rec[t] = ghost_own(b, sd.side, a, bb, layer);
+        return;
     }
+    const BlockDev& o = tab[sd.oblk];
+    int i, j, k;
+    ffc_source(b.dims, sd.side, sd.oside, sd.orient, a, bb, layer, o.nic, o.njc, o.nkc, i, j, k);
+    const int64_t src = pidx(o, i, j, k);
+    const int64_t dst = ghost_pidx(b, sd.side, a, bb, layer);
+    if (lengths) {
+        double* len = const_cast<double*>(b.len);
+        for (int f = 0; f < 3; ++f) len[dst + f * b.npad] = o.len[src + f * o.npad];
+        return;
+    }
+    GhostRec g{};
+    g.dst = const_cast<double*>(b.fs_in) + dst;
+    g.src = o.fs_in + src;
+    g.npd = (int)b.npad;
+    g.nps = (int)o.npad;
+    g.sdst = b.shock ? b.shock + dst : nullptr;
+    g.ssrc = o.shock ? o.shock + src : nullptr;
+    rec[t] = g;
+}
+
+// Ghost cells of every side of every block in one launch: full-face-copy exchange from the
+// source block's cells (simcore_exchange.d:96-135 -> full_face_copy.d:1888-1900, the
+// same-process copy of the whole flow state) and the other ghost-cell effects.  With `shock`
+// (the fill that precedes shock detection) the indicators too, as the reference's ghost cells
+// copy the whole flow state, fs.S included.
+//
+// The launch is bound by the chain of dependent memory accesses of one lane: resolved on the
+// fly (a search in the side table, the side, the blocks' records, the mapping, then a plane
+// at a time) it was some ten of them behind each other, each to memory that the other
+// kernels have pushed out of the caches.  With a record per cell it is two, the record and
+// the state, all planes at once: 13.3 -> 3.5 us a launch over the 960 ghost cells of the nitrogen
+// cylinder (its step 211 -> 188 us), a 2-D tube of 200 x 100 cells 70 -> 66 us a step.
+template <int NFS>
+__global__ __launch_bounds__(64) void k_ghost_fill(const GhostRec* __restrict__ rec, int64_t total, int shock) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= total) return;
+    const GhostRec r = rec[t];
+    double v[NFS];
+#pragma unroll
+    for (int f = 0; f < NFS; ++f) v[f] = r.src[(int64_t)f * r.nps];
+    if (r.wall) {
+        // ghost_cell.d:33-43
+        const FaceGeom fg = load_face(r.wall, r.nface, 0);
+        Vec3d l = to_local(Vec3d{v[FS_VX], v[FS_VY], v[FS_VZ]}, fg);
+        l.x = -(l.x);
+        const Vec3d w = to_global(l, fg);
+        v[FS_VX] = w.x;
+        v[FS_VY] = w.y;
+        v[FS_VZ] = w.z;
+    }
+#pragma unroll
+    for (int f = 0; f < NFS; ++f) r.dst[(int64_t)f * r.npd] = v[f];
+    if (shock) *r.sdst = r.ssrc ? *r.ssrc : 0;
 }
 
 // PJ shock detector (shockdetectors.d:21-113) for the face between cells cl and cr with
@@ -493,10 +504,21 @@ hipError_t launch_cell_update_batch(const BlockDev* tab, const int64_t* start, i
     return hipGetLastError();
 }
 
-hipError_t launch_ghost_batch(const BlockDev* tab, const SideDev* sides, int nsides, int64_t total, int mode,
+hipError_t launch_ghost_setup(const BlockDev* tab, const SideDev* sides, int nsides, int64_t total, GhostRec* rec,
                               hipStream_t s) {
     if (total <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_ghost_batch, dim3(nblk(total, 256)), dim3(256), 0, s, tab, sides, nsides, total, mode);
+    hipLaunchKernelGGL(k_ghost_setup, dim3(nblk(total, 256)), dim3(256), 0, s, tab, sides, nsides, total, rec,
+                       rec ? 0 : 1);
+    return hipGetLastError();
+}
+
+hipError_t launch_ghost_fill(const GhostRec* rec, int64_t total, int nfs, int shock, hipStream_t s) {
+    if (total <= 0) return hipSuccess;
+    const dim3 g(nblk(total, 64)), blk(64);
+    if (nfs == FS_BASE_PLANES) hipLaunchKernelGGL(k_ghost_fill<FS_BASE_PLANES>, g, blk, 0, s, rec, total, shock);
+    else if (nfs == FS_BASE_PLANES + 4) hipLaunchKernelGGL(k_ghost_fill<FS_BASE_PLANES + 4>, g, blk, 0, s, rec, total, shock);
+    else if (nfs == FS_BASE_PLANES + 10) hipLaunchKernelGGL(k_ghost_fill<FS_BASE_PLANES + 10>, g, blk, 0, s, rec, total, shock);
+    else return hipErrorInvalidValue;  // 1, 2 or 5 species
     return hipGetLastError();
 }
 

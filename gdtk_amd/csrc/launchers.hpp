@@ -61,13 +61,14 @@ hipError_t launch_cells_scatter(const BlockDev* tab, const int64_t* start, const
                                 const double* p_o, const double* massf_o, const double* dtc_o, double* dtc,
                                 const int* status, unsigned* nfail, hipStream_t s);
 hipError_t launch_fill_f64(double* p, int64_t n, double v, hipStream_t s);
-// Ghost cells of all blocks in one launch (exchange and the other ghost-cell effects);
-// mode 1 exchanges the cell lengths of the exchange sides instead; mode 2 also copies the
-// shock indicators.
+// Ghost cells of all blocks: the records of the fill for one flow-state copy (tab's fs_in), or
+// with rec null the exchange of the cell lengths; and the fill itself (exchange and the other
+// ghost-cell effects), with the shock indicators where shock is set.
+hipError_t launch_ghost_setup(const BlockDev* tab, const SideDev* sides, int nsides, int64_t total, GhostRec* rec,
+                              hipStream_t s);
+hipError_t launch_ghost_fill(const GhostRec* rec, int64_t total, int nfs, int shock, hipStream_t s);
 // Shock detection over all blocks' interior cells (PJ detector, strict rule applied by
 // the adaptive flux kernels), launched like the cell update.
-hipError_t launch_ghost_batch(const BlockDev* tab, const SideDev* sides, int nsides, int64_t total, int mode,
-                              hipStream_t s);
 hipError_t launch_shock_detect(const BlockDev* tab, const FaceBatch& fb, const int64_t* cstart, int nblocks,
                                int64_t ctotal, int dims, double comp_tol, double shear_tol, int damped_outflow,
                                hipStream_t s);

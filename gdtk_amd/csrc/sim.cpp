@@ -112,6 +112,7 @@ struct Sim {
     DevArr<SideDev> sides;
     int nsides = 0;
     int64_t nghost = 0;
+    DevArr<GhostRec> ghosts[2];  // per flow-state copy
     DevArr<int> tile_start;
     int total_tiles = 0, kchunk = 16, tile_x = 64, tiles_kc = -1, tiles_tx = -1;
     DevArr<unsigned> ctr;
@@ -364,6 +365,11 @@ struct Sim {
                     }
         tabs.alloc(h.size());
         HIPCHK(hipMemcpy(tabs.p, h.data(), h.size() * sizeof(BlockDev), hipMemcpyHostToDevice));
+        // The ghost records of each copy (inflow rows are read from the block records).
+        for (int c = 0; c < 2; ++c) {
+            ghosts[c].reserve((size_t)nghost);
+            HIPCHK(launch_ghost_setup(tab(1, c, 0), sides.p, nsides, nghost, ghosts[c].p, stream));
+        }
     }
 
     // Sets up the batched launches once every block exists (the reference does the same
@@ -410,7 +416,7 @@ struct Sim {
         build_tiles(kchunk, tile_x);
         // Geometry exchange: ghost cells of exchange sides take their source cells' lengths.
         if (any_exchange) {
-            HIPCHK(launch_ghost_batch(tab(1, 0, 0), sides.p, nsides, nghost, 1, stream));
+            HIPCHK(launch_ghost_setup(tab(1, 0, 0), sides.p, nsides, nghost, nullptr, stream));
             HIPCHK(hipStreamSynchronize(stream));
         }
         finalized = true;
@@ -444,7 +450,7 @@ struct Sim {
             if (d < nd) nfaces += nfaces_total(d);
         }
         timed(3, (double)nghost,
-              [&] { return launch_ghost_batch(t, sides.p, nsides, nghost, detect ? 2 : 0, stream); });
+              [&] { return launch_ghost_fill(ghosts[c].p, nghost, nfs(), detect ? 1 : 0, stream); });
         if (detect)
             timed(4, nc, [&] {
                 return launch_shock_detect(t, fb, cstart.p, nb, ctotal, cfg.dimensions, sdet.compression_tolerance,
