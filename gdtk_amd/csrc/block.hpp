@@ -153,6 +153,27 @@ __host__ __device__ inline int face_batch_dir(const FaceBatch& fb, int64_t& w0) 
     return d;
 }
 
+// Steps queued one behind the other without the host between them.  Three control words on the
+// device: [0] stop, [1] steps finished, [2] a step is running.  The control kernel at the start
+// of each step and behind the last one judges the step before it by its counters (the
+// reference's stage-by-stage checks, simcore_gasdynamic_step.d:946-1000, and the failed cells
+// of its chemistry; a flux update also before its chemistry) and counts it as finished or sets
+// stop; from then on the kernels that
+// write what a repeated step starts from (U, the saved flow state, the shock indicators,
+// dt_chem) return at once, so the host finds the failed step's counters and starting state
+// as if it had waited for that step.
+enum StepPoint : int {
+    STEP_BEGIN,      // judge and count the step before, clear the counters
+    STEP_FLUX_DONE,  // before the chemistry: judge the flux update
+    STEP_END,        // behind the last step: judge and count it
+};
+struct StepControl {
+    unsigned* ctl;
+    unsigned* chem_fail;  // failed cells of the step's chemistry (null without chemistry)
+    int nblocks, region, cells;  // counters: two regions of `region` words, 4 per block from `cells`
+    unsigned max_invalid;
+};
+
 // Batched stage launch over every block: per-block device records for this stage (their
 // buffers already point at this stage's input and output copies), the prefix sums of the
 // blocks' tile counts, and the per-XCD tile queues (8 counters, TILE_QSTRIDE apart).
@@ -161,6 +182,7 @@ struct StageBatch {
     const BlockDev* tab;
     const int* tile_start;
     unsigned* queue;
+    const unsigned* stop;  // StepControl
     int nblocks, total_tiles, per_xcd, KC;
 };
 

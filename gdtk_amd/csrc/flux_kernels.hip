@@ -205,7 +205,9 @@ __global__ __launch_bounds__(256) void k_shock_faces_batch(const BlockDev* __res
 // cells marked too).
 template <int DIM>
 __global__ __launch_bounds__(256) void k_shock_cells_batch(const BlockDev* __restrict__ tab,
-                                                           const int64_t* __restrict__ start, int nblocks) {
+                                                           const int64_t* __restrict__ start, int nblocks,
+                                                           const unsigned* __restrict__ stop) {
+    if (*stop) return;  // StepControl: the run waits for the host
     const int64_t w0 = (int64_t)blockIdx.x * blockDim.x;
     int lo = 0, hi = nblocks - 1;
     while (lo < hi) {
@@ -271,7 +273,8 @@ template <int DIM, int STAGE>
 __global__ __launch_bounds__(256) void k_cell_update_batch(const BlockDev* __restrict__ tab,
                                                            const int64_t* __restrict__ start, int nblocks,
                                                            const double* __restrict__ dtp, CellLimits lim,
-                                                           IdealGasDev gas) {
+                                                           IdealGasDev gas, const unsigned* __restrict__ stop) {
+    if (*stop) return;  // StepControl: the run waits for the host
     const int64_t w0 = (int64_t)blockIdx.x * blockDim.x;
     int lo = 0, hi = nblocks - 1;
     while (lo < hi) {
@@ -473,33 +476,33 @@ hipError_t launch_face_flux_batch(const BlockDev* tab, const FaceBatch& fb, int 
 
 hipError_t launch_shock_detect(const BlockDev* tab, const FaceBatch& fb, const int64_t* cstart, int nblocks,
                                int64_t ctotal, int dims, double comp_tol, double shear_tol, int damped_outflow,
-                               hipStream_t s) {
+                               const unsigned* stop, hipStream_t s) {
     const int64_t ftotal = fb.total[0] + fb.total[1] + fb.total[2];
     if (ctotal <= 0 || ftotal <= 0) return hipSuccess;
     dim3 fgrid(nblk(ftotal, 256)), cgrid(nblk(ctotal, 256)), blk(256);
     if (dims == 3) {
         hipLaunchKernelGGL((k_shock_faces_batch<3>), fgrid, blk, 0, s, tab, fb, nblocks, comp_tol, shear_tol,
                            damped_outflow);
-        hipLaunchKernelGGL((k_shock_cells_batch<3>), cgrid, blk, 0, s, tab, cstart, nblocks);
+        hipLaunchKernelGGL((k_shock_cells_batch<3>), cgrid, blk, 0, s, tab, cstart, nblocks, stop);
     } else {
         hipLaunchKernelGGL((k_shock_faces_batch<2>), fgrid, blk, 0, s, tab, fb, nblocks, comp_tol, shear_tol,
                            damped_outflow);
-        hipLaunchKernelGGL((k_shock_cells_batch<2>), cgrid, blk, 0, s, tab, cstart, nblocks);
+        hipLaunchKernelGGL((k_shock_cells_batch<2>), cgrid, blk, 0, s, tab, cstart, nblocks, stop);
     }
     return hipGetLastError();
 }
 
 hipError_t launch_cell_update_batch(const BlockDev* tab, const int64_t* start, int nblocks, int64_t total, int dims,
                                    int stage, const double* dtp, const CellLimits& lim, const IdealGasDev& gas,
-                                   hipStream_t s) {
+                                   const unsigned* stop, hipStream_t s) {
     if (total <= 0) return hipSuccess;
     dim3 grid(nblk(total, 256)), blk(256);
     if (dims == 3) {
-        if (stage == 1) hipLaunchKernelGGL((k_cell_update_batch<3, 1>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas);
-        else hipLaunchKernelGGL((k_cell_update_batch<3, 2>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas);
+        if (stage == 1) hipLaunchKernelGGL((k_cell_update_batch<3, 1>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas, stop);
+        else hipLaunchKernelGGL((k_cell_update_batch<3, 2>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas, stop);
     } else {
-        if (stage == 1) hipLaunchKernelGGL((k_cell_update_batch<2, 1>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas);
-        else hipLaunchKernelGGL((k_cell_update_batch<2, 2>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas);
+        if (stage == 1) hipLaunchKernelGGL((k_cell_update_batch<2, 1>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas, stop);
+        else hipLaunchKernelGGL((k_cell_update_batch<2, 2>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas, stop);
     }
     return hipGetLastError();
 }

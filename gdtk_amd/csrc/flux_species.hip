@@ -13,7 +13,9 @@ template <int DIM, int STAGE, int NSP>
 __global__ __launch_bounds__(256) void k_cell_update_species(const BlockDev* __restrict__ tab,
                                                              const int64_t* __restrict__ start, int nblocks,
                                                              const double* __restrict__ dtp, CellLimits lim,
-                                                             const ChemDev* __restrict__ cdp) {
+                                                             const ChemDev* __restrict__ cdp,
+                                                             const unsigned* __restrict__ stop) {
+    if (*stop) return;  // StepControl: the run waits for the host
     const int64_t w0 = (int64_t)blockIdx.x * blockDim.x;
     int lo = 0, hi = nblocks - 1;
     while (lo < hi) {
@@ -85,14 +87,15 @@ bool species_supported(int nsp) { return nsp == 2 || nsp == 5; }
 
 template <int NSP>
 static void cell_species(const BlockDev* tab, const int64_t* start, int nb, int64_t total, int dims, int stage,
-                         const double* dtp, const CellLimits& lim, const ChemDev* cd, hipStream_t s) {
+                         const double* dtp, const CellLimits& lim, const ChemDev* cd, const unsigned* stop,
+                         hipStream_t s) {
     dim3 g(nblk256(total)), blk(256);
     if (dims == 3) {
-        if (stage == 1) hipLaunchKernelGGL((k_cell_update_species<3, 1, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd);
-        else hipLaunchKernelGGL((k_cell_update_species<3, 2, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd);
+        if (stage == 1) hipLaunchKernelGGL((k_cell_update_species<3, 1, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd, stop);
+        else hipLaunchKernelGGL((k_cell_update_species<3, 2, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd, stop);
     } else {
-        if (stage == 1) hipLaunchKernelGGL((k_cell_update_species<2, 1, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd);
-        else hipLaunchKernelGGL((k_cell_update_species<2, 2, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd);
+        if (stage == 1) hipLaunchKernelGGL((k_cell_update_species<2, 1, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd, stop);
+        else hipLaunchKernelGGL((k_cell_update_species<2, 2, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd, stop);
     }
 }
 
@@ -109,10 +112,10 @@ hipError_t launch_face_flux_species(const BlockDev* tab, const FaceBatch& fb, in
 
 hipError_t launch_cell_update_species(const BlockDev* tab, const int64_t* start, int nblocks, int64_t total, int dims,
                                      int stage, const double* dtp, const CellLimits& lim, int nsp, const ChemDev* cd,
-                                     hipStream_t s) {
+                                     const unsigned* stop, hipStream_t s) {
     if (total <= 0) return hipSuccess;
-    if (nsp == 2) cell_species<2>(tab, start, nblocks, total, dims, stage, dtp, lim, cd, s);
-    else if (nsp == 5) cell_species<5>(tab, start, nblocks, total, dims, stage, dtp, lim, cd, s);
+    if (nsp == 2) cell_species<2>(tab, start, nblocks, total, dims, stage, dtp, lim, cd, stop, s);
+    else if (nsp == 5) cell_species<5>(tab, start, nblocks, total, dims, stage, dtp, lim, cd, stop, s);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }
@@ -148,14 +151,18 @@ namespace gdtk {
 // gathered into dense arrays for the batched reactor, and the results written back as
 // thermochemical_increment leaves them (fvcell.d:858-972): T, u, p and the mass fractions
 // of the flow state, and U[0]'s species densities rho * massf.  The sound speed and the
-// cell's species densities are left as they are, as in the reference.
+// cell's species densities are left as they are, as in the reference.  Once a run waits for the
+// host (*stop), the gather hands over frozen cells (T = 0) and the scatter writes nothing.
 template <bool SCATTER>
 __global__ __launch_bounds__(256) void k_cells_chem(const BlockDev* __restrict__ tab, const int64_t* __restrict__ start,
                                                     const int64_t* __restrict__ coff, int nblocks, int nsp, int64_t n,
                                                     double* rho, double* T, double* u, double* p, double* massf,
                                                     const double* T_o, const double* u_o, const double* p_o,
                                                     const double* massf_o, const double* dtc_o, double* dtc,
-                                                    const int* status, unsigned* nfail) {
+                                                    const int* status, unsigned* nfail,
+                                                    const unsigned* __restrict__ stop) {
+    const bool stopped = *stop != 0;
+    if (SCATTER && stopped) return;
     const int64_t w0 = (int64_t)blockIdx.x * blockDim.x;
     int lo = 0, hi = nblocks - 1;
     while (lo < hi) {
@@ -175,7 +182,7 @@ __global__ __launch_bounds__(256) void k_cells_chem(const BlockDev* __restrict__
     double* fs = const_cast<double*>(b.fs_in);
     if (!SCATTER) {
         rho[x] = fs[c + FS_RHO * np];
-        T[x] = fs[c + FS_T * np];
+        T[x] = stopped ? 0.0 : fs[c + FS_T * np];
         u[x] = fs[c + FS_U * np];
         p[x] = fs[c + FS_P * np];
         for (int s = 0; s < nsp; ++s) massf[(int64_t)s * n + x] = fs[c + (FS_BASE_PLANES + s) * np];
@@ -198,20 +205,21 @@ __global__ __launch_bounds__(256) void k_cells_chem(const BlockDev* __restrict__
 
 hipError_t launch_cells_gather(const BlockDev* tab, const int64_t* start, const int64_t* coff, int nblocks,
                                int64_t total, int nsp, int64_t n, double* rho, double* T, double* u, double* p,
-                               double* massf, hipStream_t s) {
+                               double* massf, const unsigned* stop, hipStream_t s) {
     if (total <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_cells_chem<false>, dim3(nblk256(total)), dim3(256), 0, s, tab, start, coff, nblocks, nsp, n,
-                       rho, T, u, p, massf, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+                       rho, T, u, p, massf, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, stop);
     return hipGetLastError();
 }
 
 hipError_t launch_cells_scatter(const BlockDev* tab, const int64_t* start, const int64_t* coff, int nblocks,
                                 int64_t total, int nsp, int64_t n, const double* T_o, const double* u_o,
                                 const double* p_o, const double* massf_o, const double* dtc_o, double* dtc,
-                                const int* status, unsigned* nfail, hipStream_t s) {
+                                const int* status, unsigned* nfail, const unsigned* stop, hipStream_t s) {
     if (total <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_cells_chem<true>, dim3(nblk256(total)), dim3(256), 0, s, tab, start, coff, nblocks, nsp, n,
-                       nullptr, nullptr, nullptr, nullptr, nullptr, T_o, u_o, p_o, massf_o, dtc_o, dtc, status, nfail);
+                       nullptr, nullptr, nullptr, nullptr, nullptr, T_o, u_o, p_o, massf_o, dtc_o, dtc, status, nfail,
+                       stop);
     return hipGetLastError();
 }
 

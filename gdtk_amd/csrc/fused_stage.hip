@@ -230,6 +230,7 @@ __device__ __forceinline__ void fused_tile(const BlockDev& b, const IdealGasDev&
 template <int DIM, int FC, int STAGE, int TX>
 __global__ __launch_bounds__(FT_THREADS, GDTK_FUSED_WAVES_PER_EU) void k_fused_batch(
     StageBatch sb, IdealGasDev gas, const double* __restrict__ dtp, double eps, CellLimits lim) {
+    if (*sb.stop) return;  // StepControl: the run waits for the host
     constexpr int TY = FT_THREADS / TX;
     __shared__ TileLds<CQ<DIM>::n, TX> L;
     __shared__ int s_tile;
@@ -353,7 +354,9 @@ hipError_t launch_clear_u32(unsigned* p, int n, hipStream_t s) {
 // block), so that the copies are one node of a captured step.  Segment q covers chunks
 // [segs[q].start, segs[q + 1].start) of 1024 doubles; each lane moves 4 doubles of one
 // chunk (two 16-byte loads and stores where the chunk is whole).
-__global__ __launch_bounds__(256) void k_copy_segments(const CopySeg* __restrict__ segs, int nseg) {
+__global__ __launch_bounds__(256) void k_copy_segments(const CopySeg* __restrict__ segs, int nseg,
+                                                       const unsigned* __restrict__ stop) {
+    if (*stop) return;  // StepControl: the run waits for the host
     const int64_t chunk = blockIdx.x;
     int lo = 0, hi = nseg - 1;
     while (lo < hi) {
@@ -374,9 +377,59 @@ __global__ __launch_bounds__(256) void k_copy_segments(const CopySeg* __restrict
     }
 }
 
-hipError_t launch_copy_segments(const CopySeg* segs, int nseg, int64_t nchunks, hipStream_t s) {
+hipError_t launch_copy_segments(const CopySeg* segs, int nseg, int64_t nchunks, const unsigned* stop, hipStream_t s) {
     if (nchunks <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_copy_segments, dim3((unsigned)nchunks), dim3(256), 0, s, segs, nseg);
+    hipLaunchKernelGGL(k_copy_segments, dim3((unsigned)nchunks), dim3(256), 0, s, segs, nseg, stop);
+    return hipGetLastError();
+}
+
+// The control block of steps that are queued without the host between them (StepControl).
+__device__ __forceinline__ unsigned step_outcome(const unsigned* ctr, const StepControl& c, bool chem) {
+    unsigned fail = 0;
+    for (int q = threadIdx.x; q < c.nblocks; q += blockDim.x)
+        for (int st = 0; st < 2; ++st) {
+            const unsigned* k = ctr + st * c.region + c.cells + 4 * q;
+            if (k[0] > 0u || k[1] > c.max_invalid) fail = 1;
+        }
+    if (chem && threadIdx.x == 0 && c.chem_fail && *c.chem_fail > 0u) fail = 1;
+    return __syncthreads_or(fail) ? 1u : 0u;
+}
+
+__global__ __launch_bounds__(256) void k_step_control(unsigned* ctr, StepControl c, int at) {
+    const bool begin = at == STEP_BEGIN;
+    unsigned* ctl = c.ctl;
+    const unsigned stopped = ctl[0], pending = ctl[2];
+    __syncthreads();  // every thread has read the control words before thread 0 writes them
+    if (stopped) return;
+    if (pending) {
+        const unsigned fail = step_outcome(ctr, c, at != STEP_FLUX_DONE);
+        if (threadIdx.x == 0) {
+            if (fail) ctl[0] = 1;
+            else if (at != STEP_FLUX_DONE) ctl[1] += 1;
+        }
+        if (fail) return;
+    }
+    if (at == STEP_FLUX_DONE) return;
+    if (threadIdx.x == 0) {
+        ctl[2] = begin ? 1u : 0u;
+        if (begin && c.chem_fail) *c.chem_fail = 0u;
+    }
+    if (begin)
+        for (int k = threadIdx.x; k < 2 * c.region; k += blockDim.x) ctr[k] = 0u;
+}
+
+hipError_t launch_step_control(unsigned* ctr, const StepControl& c, StepPoint at, hipStream_t s) {
+    hipLaunchKernelGGL(k_step_control, dim3(1), dim3(256), 0, s, ctr, c, (int)at);
+    return hipGetLastError();
+}
+
+__global__ void k_window_begin(unsigned* ctl, double* dtp, double dt) {
+    if (threadIdx.x < 3) ctl[threadIdx.x] = 0u;
+    if (threadIdx.x == 0) *dtp = dt;
+}
+
+hipError_t launch_window_begin(unsigned* ctl, double* dtp, double dt, hipStream_t s) {
+    hipLaunchKernelGGL(k_window_begin, dim3(1), dim3(64), 0, s, ctl, dtp, dt);
     return hipGetLastError();
 }
 

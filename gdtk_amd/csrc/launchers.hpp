@@ -35,7 +35,7 @@ hipError_t launch_face_flux_batch(const BlockDev* tab, const FaceBatch& fb, int 
                                  int numerics, double eps, const IdealGasDev& gas, hipStream_t s);
 hipError_t launch_cell_update_batch(const BlockDev* tab, const int64_t* start, int nblocks, int64_t total, int dims,
                                    int stage, const double* dtp, const CellLimits& lim, const IdealGasDev& gas,
-                                   hipStream_t s);
+                                   const unsigned* stop, hipStream_t s);
 // Multi-species thermally perfect gas (flux_species.hip), nsp = 2 or 5: the same batched
 // face and cell-update launches, and one block's encode/decode at start-up.
 struct ChemDev;
@@ -46,7 +46,7 @@ hipError_t launch_face_flux_species_lmr(const BlockDev* tab, const FaceBatch& fb
                                        double eps, int nsp, const ChemDev* cd, int64_t total, hipStream_t s);
 hipError_t launch_cell_update_species(const BlockDev* tab, const int64_t* start, int nblocks, int64_t total, int dims,
                                      int stage, const double* dtp, const CellLimits& lim, int nsp, const ChemDev* cd,
-                                     hipStream_t s);
+                                     const unsigned* stop, hipStream_t s);
 hipError_t launch_encode_species(const BlockDev& b, double* U, hipStream_t s);
 hipError_t launch_decode_species(const BlockDev& b, const ChemDev* cd, double* U, double* fs, double low_T,
                                  hipStream_t s);
@@ -55,11 +55,11 @@ hipError_t launch_decode_species(const BlockDev& b, const ChemDev* cd, double* U
 // scatter counts failed cells into nfail.  coff[q] = first dense index of block q.
 hipError_t launch_cells_gather(const BlockDev* tab, const int64_t* start, const int64_t* coff, int nblocks,
                                int64_t total, int nsp, int64_t n, double* rho, double* T, double* u, double* p,
-                               double* massf, hipStream_t s);
+                               double* massf, const unsigned* stop, hipStream_t s);
 hipError_t launch_cells_scatter(const BlockDev* tab, const int64_t* start, const int64_t* coff, int nblocks,
                                 int64_t total, int nsp, int64_t n, const double* T_o, const double* u_o,
                                 const double* p_o, const double* massf_o, const double* dtc_o, double* dtc,
-                                const int* status, unsigned* nfail, hipStream_t s);
+                                const int* status, unsigned* nfail, const unsigned* stop, hipStream_t s);
 hipError_t launch_fill_f64(double* p, int64_t n, double v, hipStream_t s);
 // Ghost cells of all blocks: the records of the fill for one flow-state copy (tab's fs_in), or
 // with rec null the exchange of the cell lengths; and the fill itself (exchange and the other
@@ -71,7 +71,7 @@ hipError_t launch_ghost_fill(const GhostRec* rec, int64_t total, int nfs, int sh
 // the adaptive flux kernels), launched like the cell update.
 hipError_t launch_shock_detect(const BlockDev* tab, const FaceBatch& fb, const int64_t* cstart, int nblocks,
                                int64_t ctotal, int dims, double comp_tol, double shear_tol, int damped_outflow,
-                               hipStream_t s);
+                               const unsigned* stop, hipStream_t s);
 // Fused LDS-tiled stage kernel over all blocks (fused_stage.hip): tiles of one block for
 // k chunks of kc planes, the persistent grid size for the device, and the launch (dt is
 // read from device memory).
@@ -90,7 +90,11 @@ struct CopySeg {
     double* dst;
     int64_t n, start;
 };
-hipError_t launch_copy_segments(const CopySeg* segs, int nseg, int64_t nchunks, hipStream_t s);
+hipError_t launch_copy_segments(const CopySeg* segs, int nseg, int64_t nchunks, const unsigned* stop, hipStream_t s);
+// The control kernel of queued steps (StepControl) at a point of a step, and the start of a queue
+// of steps of size dt.
+hipError_t launch_step_control(unsigned* ctr, const StepControl& c, StepPoint at, hipStream_t s);
+hipError_t launch_window_begin(unsigned* ctl, double* dtp, double dt, hipStream_t s);
 // Flow-solution records of one block (flow_io.hip): pack the flow state (fs_in) into nv
 // doubles per active cell, and unpack records into the flow-state planes fs.
 hipError_t launch_pack_flow(const BlockDev& b, const double* pos, const double* mu, const double* kc, const double* dtc,

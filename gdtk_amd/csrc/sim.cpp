@@ -115,8 +115,12 @@ struct Sim {
     DevArr<GhostRec> ghosts[2];  // per flow-state copy
     DevArr<int> tile_start;
     int total_tiles = 0, kchunk = 16, tile_x = 64, tiles_kc = -1, tiles_tx = -1;
-    DevArr<unsigned> ctr;
+    DevArr<unsigned> ctr;  // the stages' counters, then the control words of queued steps
     StageCounters sc;
+    unsigned* ctr_host = nullptr;  // pinned copy of ctr
+    // Events around the chemistry of each queued step.
+    static constexpr int MAX_QUEUED = 16;
+    std::vector<hipEvent_t> qev;
     DevArr<double> dt_dev;
     int grid = 0, wg_per_cu = 0;
     bool use_graph = true;
@@ -130,6 +134,7 @@ struct Sim {
     // Block time-step estimates: one partial per workgroup of the cell launch, each block's
     // last signal, and the per-block results {dt, cfl, last signal}.
     DevArr<double> dt_part, dt_last, dt_out;
+    double* dt_host = nullptr;  // pinned copy of dt_out
     // Step-start copy of every block's flow state (multi-species gas): segments per
     // flow-state copy (cur = 0, 1), one launch, part of the captured step.
     DevArr<CopySeg> save_segs[2];
@@ -175,6 +180,10 @@ struct Sim {
         if (cev0) (void)hipEventDestroy(cev0);
         if (cev1) (void)hipEventDestroy(cev1);
         if (cfail_host) (void)hipHostFree(cfail_host);
+        if (ctr_host) (void)hipHostFree(ctr_host);
+        if (dt_host) (void)hipHostFree(dt_host);
+        for (auto& e : qev)
+            if (e) (void)hipEventDestroy(e);
         blocks.clear();
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
@@ -244,7 +253,7 @@ struct Sim {
     // kernel's launch shape, whether stage 1 detects shocks and the numerics.
     long long launch_signature() const {
         return (use_fused() ? 1000000LL + 1000LL * kchunk + tile_x + 100000000LL * wg_per_cu : 0LL) +
-               (detect_now() ? 10000000000LL : 0LL) + 100000000000LL * numerics;
+               (chem_h >= 0 ? 1000000000000LL : 0LL) + (detect_now() ? 10000000000LL : 0LL) + 100000000000LL * numerics;
     }
 
     void build_starts() {
@@ -268,6 +277,7 @@ struct Sim {
         dt_part.alloc(2 * (size_t)(ctotal / 256));
         dt_last.alloc(nb);
         dt_out.alloc(3 * nb);
+        HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&dt_host), 3 * nb * sizeof(double)));
     }
 
     // Face-flux arrays of the face-per-thread kernels, allocated the first time they run.
@@ -408,7 +418,8 @@ struct Sim {
         sides.alloc(hs.size());
         HIPCHK(hipMemcpy(sides.p, hs.data(), hs.size() * sizeof(SideDev), hipMemcpyHostToDevice));
         sc.nblocks = (int)blocks.size();
-        ctr.alloc((size_t)2 * sc.region());
+        ctr.alloc(ctr_words());
+        HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&ctr_host), ctr_words() * sizeof(unsigned)));
         dt_dev.alloc(1);
         for (auto& bp : blocks) refresh_dev(*bp);
         build_tabs();
@@ -420,6 +431,13 @@ struct Sim {
             HIPCHK(hipStreamSynchronize(stream));
         }
         finalized = true;
+    }
+
+    size_t ctr_words() const { return (size_t)2 * sc.region() + 4; }
+    unsigned* ctl() const { return ctr.p + 2 * sc.region(); }
+    StepControl step_control() const {
+        return StepControl{ctl(), chem_h >= 0 ? cfail.p : nullptr, sc.nblocks, sc.region(), sc.cells(1, 0),
+                           (unsigned)cfg.max_invalid_cells};
     }
 
     int launch_grid() const {
@@ -454,7 +472,7 @@ struct Sim {
         if (detect)
             timed(4, nc, [&] {
                 return launch_shock_detect(t, fb, cstart.p, nb, ctotal, cfg.dimensions, sdet.compression_tolerance,
-                                           sdet.shear_tolerance, sdet.damped_outflow, stream);
+                                           sdet.shear_tolerance, sdet.damped_outflow, ctl(), stream);
             });
         if (!use_fused()) {
             timed(0, (double)nfaces, [&] {
@@ -467,9 +485,9 @@ struct Sim {
             timed(1, nc, [&] {
                 if (nsp > 1)
                     return launch_cell_update_species(t, cstart.p, nb, ctotal, cfg.dimensions, stage, dt_dev.p, lim,
-                                                      nsp, tpg_dev.p, stream);
+                                                      nsp, tpg_dev.p, ctl(), stream);
                 return launch_cell_update_batch(t, cstart.p, nb, ctotal, cfg.dimensions, stage, dt_dev.p, lim, gas,
-                                                stream);
+                                                ctl(), stream);
             });
             return;
         }
@@ -477,6 +495,7 @@ struct Sim {
         sb.tab = t;
         sb.tile_start = tile_start.p;
         sb.queue = ctr.p + sc.queue(stage);
+        sb.stop = ctl();
         sb.nblocks = nb;
         sb.total_tiles = total_tiles;
         sb.per_xcd = (total_tiles + 7) / 8;
@@ -500,10 +519,10 @@ struct Sim {
     }
 
     // Reads the cell counters of the given stages: (decode failures summed over blocks,
-    // invalid cells of the worst block) per stage.
+    // invalid cells of the worst block) per stage; the control words come with them.
     void read_counters(int s_lo, int s_hi, int nf[3], int ni[3]) {
-        std::vector<unsigned> h((size_t)2 * sc.region());
-        HIPCHK(hipMemcpyAsync(h.data(), ctr.p, h.size() * sizeof(unsigned), hipMemcpyDeviceToHost, stream));
+        const unsigned* h = ctr_host;
+        HIPCHK(hipMemcpyAsync(ctr_host, ctr.p, ctr_words() * sizeof(unsigned), hipMemcpyDeviceToHost, stream));
         HIPCHK(hipStreamSynchronize(stream));
         for (int st = s_lo; st <= s_hi; ++st) {
             nf[st] = 0;
@@ -515,8 +534,9 @@ struct Sim {
         }
     }
 
-    // The whole pc step of all blocks as one captured graph (per U parity): clear the
-    // counters, then ghost cells + stage kernels for stage 1 and stage 2.
+    // The whole pc step of all blocks as one captured graph (per U parity): the control kernel
+    // (which judges the step before it and clears the counters), then ghost cells + stage kernels
+    // for stage 1 and stage 2.
     hipGraphExec_t step_graph(int u) {
         const long long sig = launch_signature();
         if (graph[u] && graph_sig[u] == sig) return graph[u];
@@ -529,10 +549,11 @@ struct Sim {
         bool saved = profile;
         profile = false;
         try {
-            HIPCHK(launch_clear_u32(ctr.p, 2 * sc.region(), stream));
+            HIPCHK(launch_step_control(ctr.p, step_control(), STEP_BEGIN, stream));
             launch_save(0);
             launch_batched_stage(1, 0, u);
             launch_batched_stage(2, 1, u);
+            if (chem_h >= 0) HIPCHK(launch_step_control(ctr.p, step_control(), STEP_FLUX_DONE, stream));
         } catch (...) {
             profile = saved;
             hipGraph_t dummy = nullptr;
@@ -1030,9 +1051,9 @@ struct Sim {
     void determine_time_step_size() {
         if ((step % cfg.cfl_count) != 0) return;
         const size_t nb = blocks.size();
-        std::vector<double> h(3 * nb);
         launch_dt(0, (int)nb, dt_global, cfg.cfl_value);
-        HIPCHK(hipMemcpyAsync(h.data(), dt_out.p, 3 * nb * sizeof(double), hipMemcpyDeviceToHost, stream));
+        const double* h = dt_host;
+        HIPCHK(hipMemcpyAsync(dt_host, dt_out.p, 3 * nb * sizeof(double), hipMemcpyDeviceToHost, stream));
         HIPCHK(hipStreamSynchronize(stream));
         double da = std::numeric_limits<double>::max(), cm = 0.0;
         for (size_t q = 0; q < nb; ++q) {
@@ -1066,47 +1087,58 @@ struct Sim {
         }
     }
 
-    // chemistry_step (simcore.d:1619-1638) for the full_T_full_R splitting: every cell's
-    // thermochemical_increment over dt on the device (the batched reactor, or the surrogate
-    // that serves it), dt_chem kept per cell (initially -1, simcore.d:335).  A failed cell
-    // ends the run, as the reference's FlowSolverException does.
-    void chemistry_step(double dt) {
-        if (chem_h < 0) return;
+    void ensure_chemistry() {
+        if (chem_h < 0 || ncell_all) return;
         finalize();
         const int nb = (int)blocks.size();
-        if (!ncell_all) {
-            std::vector<int64_t> off(nb + 1, 0);
-            for (int q = 0; q < nb; ++q) off[q + 1] = off[q] + blocks[q]->ncell();
-            ncell_all = off[nb];
-            coff.alloc(off.size());
-            HIPCHK(hipMemcpy(coff.p, off.data(), off.size() * sizeof(int64_t), hipMemcpyHostToDevice));
-            const size_t n = (size_t)ncell_all;
-            cin.alloc((4 + (size_t)nsp) * n);
-            cout_.alloc((4 + (size_t)nsp) * n);
-            dtc.alloc(n);
-            cstatus.alloc(n);
-            cfail.alloc(1);
-            HIPCHK(launch_fill_f64(dtc.p, ncell_all, -1.0, stream));
-        }
+        std::vector<int64_t> off(nb + 1, 0);
+        for (int q = 0; q < nb; ++q) off[q + 1] = off[q] + blocks[q]->ncell();
+        coff.alloc(off.size());
+        HIPCHK(hipMemcpy(coff.p, off.data(), off.size() * sizeof(int64_t), hipMemcpyHostToDevice));
+        const size_t n = (size_t)off[nb];
+        cin.alloc((4 + (size_t)nsp) * n);
+        cout_.alloc((4 + (size_t)nsp) * n);
+        dtc.alloc(n);
+        cstatus.alloc(n);
+        cfail.alloc(1);
+        HIPCHK(launch_fill_f64(dtc.p, off[nb], -1.0, stream));
+        ncell_all = off[nb];
+        drop_graphs();  // the control kernel reads the failure count from now on
+    }
+
+    // chemistry_step (simcore.d:1619-1638) for the full_T_full_R splitting: every cell's
+    // thermochemical_increment over dt on the device (the batched reactor, or the surrogate
+    // that serves it) on the flow state of copy 0 or 1 (c) and U parity u, dt_chem kept per
+    // cell (initially -1, simcore.d:335); failed cells are added to cfail.
+    void launch_chemistry(int c, int u, double dt) {
+        const int nb = (int)blocks.size();
         const int64_t n = ncell_all;
-        double *rho = cin.p, *T = cin.p + n, *u = cin.p + 2 * n, *p = cin.p + 3 * n, *mf = cin.p + 4 * n;
+        double *rho = cin.p, *T = cin.p + n, *ue = cin.p + 2 * n, *p = cin.p + 3 * n, *mf = cin.p + 4 * n;
         double *To = cout_.p, *uo = cout_.p + n, *po = cout_.p + 2 * n, *mfo = cout_.p + 3 * n,
                *dto = cout_.p + (3 + nsp) * n;
-        const BlockDev* t = tab(1, cur, u0);
-        HIPCHK(hipEventRecord(cev0, stream));
-        HIPCHK(launch_cells_gather(t, cstart.p, coff.p, nb, ctotal, nsp, n, rho, T, u, p, mf, stream));
+        const BlockDev* t = tab(1, c, u);
+        HIPCHK(launch_cells_gather(t, cstart.p, coff.p, nb, ctotal, nsp, n, rho, T, ue, p, mf, ctl(), stream));
         int rc;
         if (surr_h >= 0) {
-            rc = gdtk_hip_surrogate_step_device(surr_h, (int)n, rho, T, u, p, mf, dtc.p, dt, To, uo, po, mfo, dto,
+            rc = gdtk_hip_surrogate_step_device(surr_h, (int)n, rho, T, ue, p, mf, dtc.p, dt, To, uo, po, mfo, dto,
                                                 cstatus.p, nullptr, stream);
         } else {
-            rc = gdtk_hip_chem_step_device(chem_h, (int)n, rho, T, u, p, mf, dtc.p, dt, To, uo, po, mfo, dto,
+            rc = gdtk_hip_chem_step_device(chem_h, (int)n, rho, T, ue, p, mf, dtc.p, dt, To, uo, po, mfo, dto,
                                            cstatus.p, stream);
         }
         if (rc < 0) throw Error(rc, g_last_error);
-        HIPCHK(launch_clear_u32(cfail.p, 1, stream));
         HIPCHK(launch_cells_scatter(t, cstart.p, coff.p, nb, ctotal, nsp, n, To, uo, po, mfo, dto, dtc.p, cstatus.p,
-                                    cfail.p, stream));
+                                    cfail.p, ctl(), stream));
+    }
+
+    // The chemistry of a step run by itself.  A failed cell ends the run, as the reference's
+    // FlowSolverException does.
+    void chemistry_step(double dt) {
+        if (chem_h < 0) return;
+        ensure_chemistry();
+        HIPCHK(hipEventRecord(cev0, stream));
+        HIPCHK(launch_clear_u32(cfail.p, 1, stream));
+        launch_chemistry(cur, u0, dt);
         HIPCHK(hipMemcpyAsync(cfail_host, cfail.p, sizeof(unsigned), hipMemcpyDeviceToHost, stream));
         HIPCHK(hipEventRecord(cev1, stream));
         chem_pending = true;
@@ -1172,47 +1204,96 @@ struct Sim {
     // Keeps the flow state the step starts from (fs[cur]) for a retry (restore_from_U0).
     void launch_save(int c) {
         if (nsp <= 1) return;
-        HIPCHK(launch_copy_segments(save_segs[c].p, (int)blocks.size(), save_chunks, stream));
+        HIPCHK(launch_copy_segments(save_segs[c].p, (int)blocks.size(), save_chunks, ctl(), stream));
     }
 
-    // One attempt of the pc step as the captured graph: both stages run, then the counters
-    // decide as the reference's stage-by-stage checks would (a failed stage 1 makes stage
-    // 2's results irrelevant; the retry restarts from U[0], which the attempt leaves
-    // untouched).  Returns true when the attempt failed.
-    bool graph_attempt() {
+    bool can_queue() const { return use_graph && !profile && cur == 0 && cfg.max_invalid_cells >= 0; }
+
+    // Queues up to `want` whole steps (captured graph and chemistry) of size dt_global one
+    // behind the other and waits once, behind the last: nothing between two time-step estimates
+    // needs the host, which otherwise waits for every step's counters.  The control kernel
+    // (StepControl) keeps the checks: the steps behind a failed one leave everything as the
+    // failed one found it, and it is repeated here at dt * 0.2 as the reference does, from
+    // U[0].  A failed stage 1 makes stage 2's results irrelevant, so one look at both stages'
+    // counters decides as the stage-by-stage checks would.  Returns the steps taken; time,
+    // step and the U parity follow them.
+    // With one wait per 10 steps a step of the 2-D tube of 200 x 100 cells takes 43 us instead of
+    // 66, one of the nitrogen cylinder 161 us instead of 188.
+    int queued_steps(int want) {
+        ensure_chemistry();
         prepare_launches();
-        hipGraphExec_t ex = step_graph(u0);
-        HIPCHK(launch_set_f64(dt_dev.p, dt_global, stream));
-        HIPCHK(hipGraphLaunch(ex, stream));
-        int nf[3], ni[3];
-        read_counters(1, 2, nf, ni);
-        for (int st = 1; st <= 2; ++st) {
-            if (nf[st] > 0) return true;
-            if (ni[st] > cfg.max_invalid_cells)
-                throw Error(GDTK_ERR_TOO_MANY_BAD_CELLS, "Too many bad cells during explicit gasdynamic update.");
+        ensure_save();
+        const bool chem = chem_h >= 0;
+        if (chem && qev.empty()) {
+            qev.assign(2 * MAX_QUEUED, nullptr);
+            for (auto& e : qev) HIPCHK(hipEventCreate(&e));
         }
-        return false;
+        int n = std::min(want, MAX_QUEUED), taken = 0;
+        int attempt = 1;  // of the step at the head of the queue
+        while (true) {
+            HIPCHK(launch_window_begin(ctl(), dt_dev.p, dt_global, stream));
+            int u = u0;
+            for (int w = 0; w < n; ++w) {
+                HIPCHK(hipGraphLaunch(step_graph(u), stream));
+                u = 1 - u;  // swap(U[0], U[end]) (simcore_gasdynamic_step.d:1557-1562)
+                if (!chem) continue;
+                HIPCHK(hipEventRecord(qev[2 * w], stream));
+                launch_chemistry(0, u, dt_global);
+                HIPCHK(hipEventRecord(qev[2 * w + 1], stream));
+            }
+            HIPCHK(launch_step_control(ctr.p, step_control(), STEP_END, stream));
+            int nf[3], ni[3];
+            read_counters(1, 2, nf, ni);
+            const unsigned* c = ctr_host + 2 * sc.region();
+            const bool stopped = c[0] != 0;
+            const int done = (int)c[1];
+            if (stopped) HIPCHK(launch_clear_u32(ctl(), 3, stream));
+            const bool flux_ok = stopped && nf[1] == 0 && nf[2] == 0 && ni[1] <= cfg.max_invalid_cells &&
+                                 ni[2] <= cfg.max_invalid_cells;  // then its chemistry failed
+            for (int w = 0; w < done + (flux_ok ? 1 : 0); ++w) {
+                u0 = 1 - u0;
+                time += dt_global;
+                step += 1;
+                ++taken;
+                attempts_last = (w == 0) ? attempt : 1;
+                if (!chem) continue;
+                float ms = 0.0f;
+                HIPCHK(hipEventElapsedTime(&ms, qev[2 * w], qev[2 * w + 1]));
+                chem_ms += ms;
+                ++chem_calls;
+            }
+            for (auto& bp : blocks) refresh_dev(*bp);
+            if (!stopped) return taken;
+            if (flux_ok) throw Error(GDTK_ERR_STEP_FAILED, "The thermochemical_increment() failed.");
+            if (done > 0) attempt = 1;
+            for (int st = 1; st <= 2; ++st) {
+                if (nf[st] > 0) break;
+                if (ni[st] > cfg.max_invalid_cells)
+                    throw Error(GDTK_ERR_TOO_MANY_BAD_CELLS, "Too many bad cells during explicit gasdynamic update.");
+            }
+            dt_global = dt_global * 0.2;
+            restore_from_U0();
+            if (attempt >= cfg.max_attempts_for_step) {
+                attempts_last = attempt;
+                throw Error(GDTK_ERR_STEP_FAILED, "Explicit update failed after max attempts; giving up.");
+            }
+            ++attempt;
+            n = 1;  // the failed step alone, at its new size
+        }
     }
 
-    // simcore_gasdynamic_step.d:906-1575 for the pc scheme.
+    // simcore_gasdynamic_step.d:906-1575 for the pc scheme, stage by stage with the host's checks
+    // between them (profiling, captured steps switched off, or single stages run before).
     void gasdynamic_step() {
         double t0 = time;
-        const bool graphed = use_graph && !profile && cur == 0;
+        finalize();
         ensure_save();
-        if (!graphed) launch_save(cur);  // the captured step saves as its first node
+        launch_save(cur);
         int attempt = 0;
         bool failed = false;
         do {
             ++attempt;
             failed = false;
-            if (graphed) {
-                failed = graph_attempt();
-                if (failed) {
-                    dt_global = dt_global * 0.2;
-                    restore_from_U0();
-                }
-                continue;
-            }
             for (int s = 1; s <= 2; ++s) {
                 int nf, ni;
                 stage_checked(s, dt_global, nf, ni);
@@ -1236,14 +1317,41 @@ struct Sim {
         time = t0 + dt_global;
     }
 
+    // One step of size dt_global and its chemistry.
+    void one_step() {
+        if (can_queue()) {
+            queued_steps(1);
+            return;
+        }
+        gasdynamic_step();
+        chemistry_step(dt_global);
+        step += 1;
+    }
+
+    // The steps that need nothing from the host: up to the next time-step estimate, the last
+    // one wanted, the one that reaches max_time, or the step at which detection freezes.
+    int steps_to_queue(int wanted, double max_time) const {
+        int n = std::min(wanted, cfg.cfl_count - step % cfg.cfl_count);
+        if (adaptive() && sdet.frozen_shock_detector && sdet.shock_detector_freeze_step > step)
+            n = std::min(n, sdet.shock_detector_freeze_step - step);
+        double t = time;
+        for (int w = 1; w <= n && w <= MAX_QUEUED; ++w) {
+            t += dt_global;
+            if (t >= max_time) return w;
+        }
+        return std::max(n, 1);
+    }
+
     int run(int max_steps, double max_time) {
         int taken = 0;
         while (true) {
             determine_time_step_size();
-            gasdynamic_step();
-            chemistry_step(dt_global);
-            step += 1;
-            ++taken;
+            if (can_queue()) {
+                taken += queued_steps(steps_to_queue(max_steps - taken, max_time));
+            } else {
+                one_step();
+                ++taken;
+            }
             if (time >= max_time) break;
             if (taken >= max_steps) break;
         }
@@ -1409,9 +1517,7 @@ int gdtk_hip_sim_step_fixed_dt(int sim, double dt, double* state) {
     int rc = guarded([&] {
         sp = &get_sim(sim);
         sp->dt_global = dt;
-        sp->gasdynamic_step();
-        sp->chemistry_step(sp->dt_global);
-        sp->step += 1;
+        sp->one_step();
         sp->check_chem();
         return GDTK_OK;
     });
