@@ -19,6 +19,8 @@
 #pragma once
 #include <cstdint>
 
+#include "quick_math.hpp"
+
 namespace gdtk {
 
 enum BCKind : int {
@@ -51,6 +53,13 @@ struct BlockDev {
     const double* fgeom[3];       // 10 planes each
     double* flux[3];              // ncq planes each (face-flux kernels)
     int nf[3][3];                 // face-array extents per direction
+    // Divisors of the face and cell indices: extents of i and of j per direction's face array,
+    // and of the cells.
+    FastDiv fdiv[3][2], cdiv[2];
+    // Frames of direction d that are one signed permutation of the axes on every face (grid
+    // lines along the axes): local component q is axis[d][q] & 3 of the global ones, negative
+    // where bit 2 is set; axis[d][0] = -1 where the faces have frames of their own.
+    int axis[3][3];
     int64_t nface[3];
     int bc_kind[6];
     double inflow[6][FS_MAX_PLANES];  // an inflow face's flow state, plane order

@@ -11,6 +11,8 @@
 
 #include <cmath>
 
+#include "quick_math.hpp"
+
 namespace gdtk {
 
 constexpr int CH_MAX_SP = 8;
@@ -260,17 +262,6 @@ __host__ __device__ inline double cea_h(const CEADev& c, double T) {
     return c.R * h_on_RT;
 }
 
-// a / b correctly rounded from y = RN(1 / b): q = RN(a y) lies within an ulp of a / b, the
-// remainder a - b q is exact in one fma, and RN(q + r y) is the correctly rounded quotient
-// (Markstein's theorem; P. Markstein, IA-64 and Elementary Functions, 2000).  Bit for bit
-// a / b for the normal operands met here; a true division costs ~10 instructions, this 3,
-// and a divisor shared by several quotients needs its reciprocal once.
-__host__ __device__ inline double div_by(double a, double b, double y) {
-    const double q = a * y;
-    const double r = fma(-b, q, a);
-    return fma(r, y, q);
-}
-
 // The powers of T that every species' curve divides by, with their reciprocals, once per
 // temperature.
 struct CeaT {
@@ -324,17 +315,6 @@ __device__ __forceinline__ double tpg_Rmix(const ChemDev& cd, const double* mass
     for (int i = 0; i < NSP; ++i) R += massf[i] * cd.R[i];
     return R;
 }
-
-// a / b for normal operands: the hardware reciprocal refined by one cubic step (residual e:
-// y (1 + e + e^2), relative error e^3), the quotient and one remainder correction, which
-// leaves it within an ulp.  7 instructions, where the compiler's division takes 11 to scale
-// operands that none of the quotients here needs scaled.
-__device__ __forceinline__ double quick_rcp(double b) {
-    const double y = __builtin_amdgcn_rcp(b);
-    const double e = fma(-b, y, 1.0);
-    return fma(y, fma(e, e, e), y);
-}
-__device__ __forceinline__ double quick_div(double a, double b) { return div_by(a, b, quick_rcp(b)); }
 
 // The curves of one composition near one temperature as a single curve: the sums over the
 // species of weight times coefficient (therm_perf_gas_mix_eos.d:61-67 and gas_model.d:410-419

@@ -111,7 +111,7 @@ __global__ void k_ghost_setup(const BlockDev* __restrict__ tab, const SideDev* _
 // fly (a search in the side table, the side, the blocks' records, the mapping, then a plane
 // at a time) it was some ten of them behind each other, each to memory that the other
 // kernels have pushed out of the caches.  With a record per cell it is two, the record and
-// the state, all planes at once: 13.3 -> 3.5 us a launch over the 960 ghost cells of the nitrogen
+// the state, all planes at once: 13.3 -> 4.5 us a launch over the 960 ghost cells of the nitrogen
 // cylinder (its step 211 -> 188 us), a 2-D tube of 200 x 100 cells 70 -> 66 us a step.
 template <int NFS>
 __global__ __launch_bounds__(64) void k_ghost_fill(const GhostRec* __restrict__ rec, int64_t total, int shock) {
@@ -229,39 +229,80 @@ __global__ __launch_bounds__(256) void k_shock_cells_batch(const BlockDev* __res
     b.shock[pidx(b, i, j, k)] = s ? 1 : 0;
 }
 
+// Compares every face's frame with its direction's first (FaceBatch order; lengths and areas may
+// differ).  Each thread writes a plain store of the same value, so no atomics.
+__global__ __launch_bounds__(256) void k_frame_check(const BlockDev* __restrict__ tab, FaceBatch fb, int nblocks,
+                                                     double* frames) {
+    int64_t w0 = (int64_t)blockIdx.x * blockDim.x;
+    const int d = __builtin_amdgcn_readfirstlane(face_batch_dir(fb, w0));
+    const int64_t* __restrict__ start = fb.start[d];
+    int lo = 0, hi = nblocks - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (start[mid] <= w0) lo = mid;
+        else hi = mid - 1;
+    }
+    const int q = __builtin_amdgcn_readfirstlane(lo);
+    const BlockDev& b = tab[q];
+    const int64_t f = w0 - start[q] + threadIdx.x;
+    if (f >= b.nface[d]) return;
+    double* r = frames + (3 * q + d) * 10;
+    bool same = true;
+    for (int e = 0; e < 9; ++e) {
+        const double* pl = b.fgeom[d] + e * b.nface[d];
+        const double first = pl[0];
+        same = same && pl[f] == first;
+        if (f == 0) r[e] = first;
+    }
+    if (!same) r[9] = 1.0;
+}
+
+hipError_t launch_frame_check(const BlockDev* tab, const FaceBatch& fb, int nblocks, double* frames, hipStream_t s) {
+    const int64_t total = fb.total[0] + fb.total[1] + fb.total[2];
+    if (total <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_frame_check, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, tab, fb, nblocks, frames);
+    return hipGetLastError();
+}
+
 // Per interior cell: time derivatives (fvcell.d:824-854), the pc stage update
 // (simcore_gasdynamic_step.d:1225-1321), decode (fvcell.d:586-821) and the
 // invalid-cell check (fluidblock.d:607-676).
 template <int DIM, int STAGE>
 __device__ __forceinline__ void cell_update_one(const BlockDev& b, const IdealGasDev& gas, double dt, double low_T,
-                                                double max_vel, double min_T, double max_T, int64_t t) {
+                                                double max_vel, double min_T, double max_T, unsigned t) {
     using C = CQ<DIM>;
-    int i = (int)(t % b.nic);
-    int64_t rest = t / b.nic;
-    int j = (int)(rest % b.njc);
-    int k = (int)(rest / b.njc);
-    int64_t c = pidx(b, i, j, k);
-    // Faces in the order W, E, S, N, B, T with outsigns -1, +1.
-    const int nfaces = (DIM == 3) ? 6 : 4;
-    int64_t fidx[6];
-    int fdir[6];
-    fidx[0] = face_index(b, 0, i, j, k); fdir[0] = 0;
-    fidx[1] = face_index(b, 0, i + 1, j, k); fdir[1] = 0;
-    fidx[2] = face_index(b, 1, i, j, k); fdir[2] = 1;
-    fidx[3] = face_index(b, 1, i, j + 1, k); fdir[3] = 1;
-    if (DIM == 3) {
-        fidx[4] = face_index(b, 2, i, j, k); fdir[4] = 2;
-        fidx[5] = face_index(b, 2, i, j, k + 1); fdir[5] = 2;
+    unsigned i, j;
+    const unsigned rest = b.cdiv[0].divmod(t, i);
+    const unsigned k = b.cdiv[1].divmod(rest, j);
+    const unsigned c = (i + NGHOST) + (unsigned)b.NI * ((j + NGHOST) + (unsigned)b.NJ * (k + (DIM == 3 ? NGHOST : 0)));
+    // Faces in the order W, E, S, N, B, T with outsigns -1, +1: per direction the low face and
+    // the one `step` behind it.
+    unsigned lo[3], step[3], org[3];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) {
+        lo[d] = i + (unsigned)b.nf[d][0] * (j + (unsigned)b.nf[d][1] * k);
+        step[d] = (d == 0) ? 1u : (d == 1) ? (unsigned)b.nf[1][0] : (unsigned)(b.nf[2][0] * b.nf[2][1]);
     }
-    double area[6];
-    for (int q = 0; q < nfaces; ++q) {
-        double A = b.fgeom[fdir[q]][fidx[q] + 9 * b.nface[fdir[q]]];
-        area[q] = ((q % 2 == 0) ? -1 : 1) * A;
+    double A[DIM][2];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) {
+        const double* area = b.fgeom[d] + 9 * b.nface[d];
+        org[d] = wave_origin(lo[d]);
+        lo[d] -= org[d];
+        area += org[d];
+        A[d][0] = ld_plane(area, lo[d]);
+        A[d][1] = ld_plane(area, lo[d] + step[d]);
     }
     double si[C::n];
+#pragma unroll
     for (int jq = 0; jq < C::n; ++jq) {
         double s = 0.0;
-        for (int q = 0; q < nfaces; ++q) s -= b.flux[fdir[q]][fidx[q] + jq * b.nface[fdir[q]]] * area[q];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            const double* fl = b.flux[d] + jq * b.nface[d] + org[d];
+            s -= ld_plane(fl, lo[d]) * -A[d][0];
+            s -= ld_plane(fl, lo[d] + step[d]) * A[d][1];
+        }
         si[jq] = s;
     }
     update_decode_store<DIM, STAGE>(b, gas, c, si, dt, low_T, max_vel, min_T, max_T);
@@ -286,7 +327,7 @@ __global__ __launch_bounds__(256) void k_cell_update_batch(const BlockDev* __res
     const BlockDev& b = tab[q];
     const int64_t t = w0 - start[q] + threadIdx.x;
     if (t >= (int64_t)b.nic * b.njc * b.nkc) return;
-    cell_update_one<DIM, STAGE>(b, gas, *dtp, lim.low_T, lim.max_vel, lim.min_T, lim.max_T, t);
+    cell_update_one<DIM, STAGE>(b, gas, *dtp, lim.low_T, lim.max_vel, lim.min_T, lim.max_T, (unsigned)t);
 }
 
 // The block time-step estimates of many blocks in two launches (fluidblock.d:987-1084 per

@@ -218,7 +218,7 @@ __device__ __forceinline__ void fused_tile(const BlockDev& b, const IdealGasDev&
                 }
                 si[q] = s;
             }
-            update_decode_store<DIM, STAGE>(b, gas, pidx(b, i, j, k), si, dt, lim.low_T, lim.max_vel, lim.min_T,
+            update_decode_store<DIM, STAGE>(b, gas, (unsigned)pidx(b, i, j, k), si, dt, lim.low_T, lim.max_vel, lim.min_T,
                                             lim.max_T);
             if (DIM == 3)
                 for (int q = 0; q < NQ; ++q) FAb[q] = FAt[q];

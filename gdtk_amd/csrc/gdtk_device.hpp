@@ -9,6 +9,8 @@
 
 #include <cmath>
 
+#include "quick_math.hpp"
+
 namespace gdtk {
 
 // Flow-state field slots in the structure-of-arrays cell storage.
@@ -74,11 +76,11 @@ struct L2R2 {
     __device__ __forceinline__ void prepare(double lenL1, double lL0, double lR0, double lenR1) {
         lenL0 = lL0;
         lenR0 = lR0;
-        aL0 = 0.5 * lL0 / (lenL1 + 2.0 * lL0 + lR0);
-        aR0 = 0.5 * lR0 / (lL0 + 2.0 * lR0 + lenR1);
-        tL01 = 2.0 / (lL0 + lenL1);
-        tR0L0 = 2.0 / (lR0 + lL0);
-        tR1R0 = 2.0 / (lenR1 + lR0);
+        aL0 = quick_div(0.5 * lL0, lenL1 + 2.0 * lL0 + lR0);
+        aR0 = quick_div(0.5 * lR0, lL0 + 2.0 * lR0 + lenR1);
+        tL01 = quick_div(2.0, lL0 + lenL1);
+        tR0L0 = quick_div(2.0, lR0 + lL0);
+        tR1R0 = quick_div(2.0, lenR1 + lR0);
         twoL0L1 = (2.0 * lL0 + lenL1);
         twoR0R1 = (2.0 * lR0 + lenR1);
     }
@@ -97,8 +99,8 @@ struct L2R2 {
             const double qq = fmax(fmax(1e-12, fabs(qL0)), fmax(1e-12, fabs(qR0)));
             eps = qq * eps_va * tR0L0;
         }
-        double sL = (delLminus * del + fabs(delLminus * del) + eps) / (delLminus * delLminus + del * del + eps);
-        double sR = (del * delRplus + fabs(del * delRplus) + eps) / (del * del + delRplus * delRplus + eps);
+        double sL = quick_div(delLminus * del + fabs(delLminus * del) + eps, delLminus * delLminus + del * del + eps);
+        double sR = quick_div(del * delRplus + fabs(del * delRplus) + eps, del * del + delRplus * delRplus + eps);
         qL = qL0 + beta * sL * aL0 * (del * twoL0L1 + delLminus * lenR0);
         qR = qR0 - beta * sR * aR0 * (delRplus * lenL0 + del * twoR0R1);
         qL = clip_to_limits(qL, qL0, qR0);
@@ -115,15 +117,15 @@ struct L2R2Side {
     __device__ __forceinline__ void prepare(double lenL1, double lL0, double lR0, double lenR1) {
         if (!RIGHT) {
             len_other = lR0;
-            a = 0.5 * lL0 / (lenL1 + 2.0 * lL0 + lR0);
-            tO = 2.0 / (lL0 + lenL1);
-            tD = 2.0 / (lR0 + lL0);
+            a = quick_div(0.5 * lL0, lenL1 + 2.0 * lL0 + lR0);
+            tO = quick_div(2.0, lL0 + lenL1);
+            tD = quick_div(2.0, lR0 + lL0);
             two = (2.0 * lL0 + lenL1);
         } else {
             len_other = lL0;
-            a = 0.5 * lR0 / (lL0 + 2.0 * lR0 + lenR1);
-            tD = 2.0 / (lR0 + lL0);
-            tO = 2.0 / (lenR1 + lR0);
+            a = quick_div(0.5 * lR0, lL0 + 2.0 * lR0 + lenR1);
+            tD = quick_div(2.0, lR0 + lL0);
+            tO = quick_div(2.0, lenR1 + lR0);
             two = (2.0 * lR0 + lenR1);
         }
     }
@@ -141,13 +143,14 @@ struct L2R2Side {
         if (!RIGHT) {
             const double delLminus = (q1 - q0) * tO;
             const double del = (q2 - q1) * tD;
-            const double sL = (delLminus * del + fabs(delLminus * del) + eps) / (delLminus * delLminus + del * del + eps);
+            const double sL =
+                quick_div(delLminus * del + fabs(delLminus * del) + eps, delLminus * delLminus + del * del + eps);
             const double qL = q1 + beta * sL * a * (del * two + delLminus * len_other);
             return clip_to_limits(qL, q1, q2);
         } else {
             const double del = (q1 - q0) * tD;
             const double delRplus = (q2 - q1) * tO;
-            const double sR = (del * delRplus + fabs(del * delRplus) + eps) / (del * del + delRplus * delRplus + eps);
+            const double sR = quick_div(del * delRplus + fabs(del * delRplus) + eps, del * del + delRplus * delRplus + eps);
             const double qR = q1 - beta * sR * a * (delRplus * len_other + del * two);
             return clip_to_limits(qR, q0, q1);
         }
@@ -181,21 +184,22 @@ __device__ __forceinline__ void ausmdv(const FaceStateT<NSP>& L, const FaceState
     using C = CQ<DIM, NSP>;
     const double factor = 1.0;
     double rL = L.rho, pL = L.p;
-    double pLrL = pL / rL;
+    double pLrL = quick_div(pL, rL);
     double uL = L.vel.x, vL = L.vel.y, wL = L.vel.z;
     double eL = L.u;
     double aL = L.a;
     double keL = 0.5 * (uL * uL + vL * vL + wL * wL);
     double HL = eL + pLrL + keL;
     double rR = R.rho, pR = R.p;
-    double pRrR = pR / rR;
+    double pRrR = quick_div(pR, rR);
     double uR = R.vel.x, vR = R.vel.y, wR = R.vel.z;
     double eR = R.u;
     double aR = R.a;
     double keR = 0.5 * (uR * uR + vR * vR + wR * wR);
     double HR = eR + pRrR + keR;
-    double alphaL = 2.0 * pLrL / (pLrL + pRrR);
-    double alphaR = 2.0 * pRrR / (pLrL + pRrR);
+    const double sum_pr = pLrL + pRrR, r_pr = quick_rcp(sum_pr);
+    double alphaL = div_by(2.0 * pLrL, sum_pr, r_pr);
+    double alphaR = div_by(2.0 * pRrR, sum_pr, r_pr);
     double am;
     if (LMR) {
         const double da = aL - aR;
@@ -205,31 +209,32 @@ __device__ __forceinline__ void ausmdv(const FaceStateT<NSP>& L, const FaceState
     } else {
         am = fmax(aL, aR);
     }
-    double ML = uL / am;
-    double MR = uR / am;
+    const double r_am = quick_rcp(am);  // and 1 / (4 am) exactly 0.25 of it
+    double ML = div_by(uL, am, r_am);
+    double MR = div_by(uR, am, r_am);
     double pLplus, uLplus;
     double duL = 0.5 * (uL + fabs(uL));
     if (fabs(ML) <= 1.0) {
         pLplus = pL * (ML + 1.0) * (ML + 1.0) * (2.0 - ML) * 0.25;
-        uLplus = alphaL * ((uL + am) * (uL + am) / (4.0 * am) - duL) + duL;
+        uLplus = alphaL * (div_by((uL + am) * (uL + am), 4.0 * am, 0.25 * r_am) - duL) + duL;
     } else {
-        pLplus = pL * duL / uL;
+        pLplus = quick_div(pL * duL, uL);
         uLplus = duL;
     }
     double pRminus, uRminus;
     double duR = 0.5 * (uR - fabs(uR));
     if (fabs(MR) <= 1.0) {
         pRminus = pR * (MR - 1.0) * (MR - 1.0) * (2.0 + MR) * 0.25;
-        uRminus = alphaR * (-(uR - am) * (uR - am) / (4.0 * am) - duR) + duR;
+        uRminus = alphaR * (div_by(-(uR - am) * (uR - am), 4.0 * am, 0.25 * r_am) - duR) + duR;
     } else {
-        pRminus = pR * duR / uR;
+        pRminus = quick_div(pR * duR, uR);
         uRminus = duR;
     }
     double ru_half = uLplus * rL + uRminus * rR;
     double p_half = pLplus + pRminus;
     double dp = pL - pR;
     const double K_SWITCH = 10.0;
-    dp = K_SWITCH * fabs(dp) / fmin(pL, pR);
+    dp = quick_div(K_SWITCH * fabs(dp), fmin(pL, pR));
     double s = 0.5 * fmin(1.0, dp);
     double ru2_AUSMV = uLplus * rL * uL + uRminus * rR * uR;
     double ru2_AUSMD = 0.5 * (ru_half * (uL + uR) - fabs(ru_half) * (uR - uL));
@@ -283,7 +288,7 @@ __device__ __forceinline__ void exxef(double sn, double& exx, double& ef) {
     } else {
         double snsq = sn * sn;
         exx = exp(-snsq);
-        double y = 1.0 / (1.0 + P * fabs(sn));
+        double y = quick_rcp(1.0 + P * fabs(sn));
         ef1 = 1.0 - y * (A1 + y * (A2 + y * (A3 + y * (A4 + A5 * y)))) * exx;
     }
     ef = copysign(ef1, sn);
@@ -299,36 +304,37 @@ __device__ __forceinline__ void efmflx(const FaceStateT<NSP>& L, const FaceState
     const double dtwspi = 0.282094792;
     double rhoL = L.rho, presL = L.p;
     double eL = L.u;
-    double hL = eL + presL / rhoL;
+    double hL = eL + quick_div(presL, rhoL);
     double tL = L.T;
     double vnL = L.vel.x, vpL = L.vel.y, vqL = L.vel.z;
     double rhoR = R.rho, presR = R.p;
     double eR = R.u;
-    double hR = eR + presR / rhoR;
+    const double presR_rhoR = quick_div(presR, rhoR);
+    double hR = eR + presR_rhoR;
     double tR = R.T;
     double vnR = R.vel.x, vpR = R.vel.y, vqR = R.vel.z;
-    double RgasL = presL / (rhoL * tL);
-    double RgasR = presR / (rhoR * tR);
+    double RgasL = quick_div(presL, rhoL * tL);
+    double RgasR = quick_div(presR, rhoR * tR);
     double rLsqrt = sqrt(rhoL);
     double rRsqrt = sqrt(rhoR);
-    double alpha = rLsqrt / (rLsqrt + rRsqrt);
+    double alpha = quick_div(rLsqrt, rLsqrt + rRsqrt);
     double cv = alpha * cvL + (1.0 - alpha) * cvR;
     double Rgas = alpha * RgasL + (1.0 - alpha) * RgasR;
     double cp = cv + Rgas;
-    double gam = cp / cv;
-    double con = 0.5 * (gam + 1.0) / (gam - 1.0);
+    double gam = quick_div(cp, cv);
+    double con = quick_div(0.5 * (gam + 1.0), gam - 1.0);
     double rtL = Rgas * tL;
     double cmpL = sqrt(2.0 * rtL);
     double hvsqL = 0.5 * (vnL * vnL + vpL * vpL + vqL * vqL);
-    double snL = vnL / (PHI * cmpL);
+    double snL = quick_div(vnL, PHI * cmpL);
     double exL, efL;
     exxef(snL, exL, efL);
     double wL = 0.5 * (1.0 + efL);
     double dL = exL * dtwspi;
-    double rtR = presR / rhoR;  // as coded in the reference
+    double rtR = presR_rhoR;  // as coded in the reference
     double cmpR = sqrt(2.0 * rtR);
     double hvsqR = 0.5 * (vnR * vnR + vpR * vpR + vqR * vqR);
-    double snR = vnR / (PHI * cmpR);
+    double snR = quick_div(vnR, PHI * cmpR);
     double exR, efR;
     exxef(snR, exR, efR);
     double wR = 0.5 * (1.0 - efR);
@@ -372,14 +378,23 @@ struct FallbackFS {
     int64_t np, cL0, cR0;
 };
 
-template <int DIM, int FC, bool LMR = false>
+// AXIS: the stencil's velocities are already in the face frame and the flux stays there, for
+// frames that are a signed permutation of the axes (the caller permutes; what the rotations
+// would multiply and add are zeros and ones).
+template <int DIM, int FC, bool LMR = false, bool AXIS = false>
 __device__ __forceinline__ void face_flux_l2r2(const IdealGasDev& gas, const FaceGeom& g, const StencilCell& L1,
                                                const StencilCell& L0, const StencilCell& R0, const StencilCell& R1,
                                                double aL0, double aR0, const FallbackFS& fb, double lenL1,
                                                double lenL0, double lenR0, double lenR1, double eps, double* F,
                                                bool shocked = false) {
     using C = CQ<DIM>;
-    Vec3d vL1 = to_local(L1.vel, g), vL0 = to_local(L0.vel, g), vR0 = to_local(R0.vel, g), vR1 = to_local(R1.vel, g);
+    Vec3d vL1 = L1.vel, vL0 = L0.vel, vR0 = R0.vel, vR1 = R1.vel;
+    if (!AXIS) {
+        vL1 = to_local(vL1, g);
+        vL0 = to_local(vL0, g);
+        vR0 = to_local(vR0, g);
+        vR1 = to_local(vR1, g);
+    }
     L2R2 c;
     c.prepare(lenL1, lenL0, lenR0, lenR1);
     FaceState Ls, Rs;
@@ -403,8 +418,10 @@ __device__ __forceinline__ void face_flux_l2r2(const IdealGasDev& gas, const Fac
     }
     // Back to the global frame (onedinterp.d:979-987), then into the face frame
     // again for the flux calculator (fluxcalc.d:65-67).
-    Ls.vel = to_local(to_global(Ls.vel, g), g);
-    Rs.vel = to_local(to_global(Rs.vel, g), g);
+    if (!AXIS) {
+        Ls.vel = to_local(to_global(Ls.vel, g), g);
+        Rs.vel = to_local(to_global(Rs.vel, g), g);
+    }
     for (int j = 0; j < C::n; ++j) F[j] = 0.0;
     // FC 2, 4: adaptive_efm_ausmdv, adaptive_hanel_ausmdv (fluxcalc.d:1315-1348) with the
     // face's indicator 0 or 1, so one calculator runs with factor 1.
@@ -416,6 +433,7 @@ __device__ __forceinline__ void face_flux_l2r2(const IdealGasDev& gas, const Fac
     // x + y or x - y, so it is never -0 (a sum is -0 only if both terms are -0), and
     // adding a signed zero to a value that is not -0 returns that value bit for bit.  The
     // terms are therefore omitted without changing any result.
+    if (AXIS) return;
     double fz = (DIM == 3) ? F[C::zMom] : 0.0;
     Vec3d m = to_global(Vec3d{F[C::xMom], F[C::yMom], fz}, g);
     F[C::xMom] = m.x;
@@ -432,32 +450,34 @@ template <int DIM, int NSP = 1>
 __device__ __forceinline__ void hanel(const FaceStateT<NSP>& L, const FaceStateT<NSP>& R, double* F) {
     using C = CQ<DIM, NSP>;
     const double rL = L.rho, pL = L.p;
-    const double pLrL = pL / rL;
+    const double pLrL = quick_div(pL, rL);
     const double uL = L.vel.x, vL = L.vel.y, wL = L.vel.z;
     const double eL = L.u, aL = L.a;
     const double keL = 0.5 * (uL * uL + vL * vL + wL * wL);
     const double HL = eL + pLrL + keL;
     const double rR = R.rho, pR = R.p;
-    const double pRrR = pR / rR;
+    const double pRrR = quick_div(pR, rR);
     const double uR = R.vel.x, vR = R.vel.y, wR = R.vel.z;
     const double eR = R.u, aR = R.a;
     const double keR = 0.5 * (uR * uR + vR * vR + wR * wR);
     const double HR = eR + pRrR + keR;
     double pLplus, uLplus;
     if (fabs(uL) <= aL) {
-        uLplus = 1.0 / (4.0 * aL) * (uL + aL) * (uL + aL);
-        pLplus = pL * uLplus * (1.0 / aL * (2.0 - uL / aL));
+        const double r = quick_rcp(aL);
+        uLplus = 0.25 * r * (uL + aL) * (uL + aL);
+        pLplus = pL * uLplus * (r * (2.0 - div_by(uL, aL, r)));
     } else {
         uLplus = 0.5 * (uL + fabs(uL));
-        pLplus = pL * uLplus * (1.0 / uL);
+        pLplus = pL * uLplus * quick_rcp(uL);
     }
     double pRminus, uRminus;
     if (fabs(uR) <= aR) {
-        uRminus = -1.0 / (4.0 * aR) * (uR - aR) * (uR - aR);
-        pRminus = pR * uRminus * (1.0 / aR * (-2.0 - uR / aR));
+        const double r = quick_rcp(aR);
+        uRminus = -0.25 * r * (uR - aR) * (uR - aR);
+        pRminus = pR * uRminus * (r * (-2.0 - div_by(uR, aR, r)));
     } else {
         uRminus = 0.5 * (uR - fabs(uR));
-        pRminus = pR * uRminus * (1.0 / uR);
+        pRminus = pR * uRminus * quick_rcp(uR);
     }
     const double p_half = pLplus + pRminus;
     F[C::mass] += uLplus * rL + uRminus * rR;

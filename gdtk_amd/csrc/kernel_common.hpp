@@ -39,23 +39,26 @@ __device__ __forceinline__ StencilCell load_sc(const double* fs, int64_t np, int
 // Stage update and decode of one cell from its surface integrals si[] (fvcell.d:824-854,
 // simcore_gasdynamic_step.d:1225-1321, fvcell.d:586-821, fluidblock.d:607-676).
 template <int DIM, int STAGE>
-__device__ __forceinline__ void update_decode_store(const BlockDev& b, const IdealGasDev& gas, int64_t c,
+__device__ __forceinline__ void update_decode_store(const BlockDev& b, const IdealGasDev& gas, unsigned c,
                                                     const double* si, double dt, double low_T, double max_vel,
                                                     double min_T, double max_T) {
     using C = CQ<DIM>;
     const int64_t np = b.npad;
-    double vol_inv = 1.0 / b.vol[c];
+    const unsigned o = wave_origin(c);  // cells come in the lanes' order
+    c -= o;
+    const double vol_inv = quick_rcp(ld_plane(b.vol + o, c));
     double U[C::n];
+#pragma unroll
     for (int jq = 0; jq < C::n; ++jq) {
-        double dUdt = vol_inv * si[jq] + 0.0;
-        double u0 = b.U0[c + jq * np];
+        const double dUdt = vol_inv * si[jq] + 0.0;
+        const double u0 = ld_plane(b.U0 + jq * np + o, c);
         if (STAGE == 1) {
             const double gamma_1 = 1.0;
-            b.dUdt0[c + jq * np] = dUdt;
+            st_plane(b.dUdt0 + jq * np + o, c, dUdt);
             U[jq] = u0 + dt * gamma_1 * dUdt;
         } else {
             const double gamma_1 = 0.5, gamma_2 = 0.5;
-            U[jq] = u0 + dt * (gamma_1 * b.dUdt0[c + jq * np] + gamma_2 * dUdt);
+            U[jq] = u0 + dt * (gamma_1 * ld_plane(b.dUdt0 + jq * np + o, c) + gamma_2 * dUdt);
         }
     }
     double rho, u, p, T, a;
@@ -67,16 +70,17 @@ __device__ __forceinline__ void update_decode_store(const BlockDev& b, const Ide
         return;
     }
     if (STAGE == 2)
-        for (int jq = 0; jq < C::n; ++jq) b.Unew[c + jq * np] = U[jq];
-    double* fo = b.fs_out;
-    fo[c + FS_RHO * np] = rho;
-    fo[c + FS_VX * np] = vel.x;
-    fo[c + FS_VY * np] = vel.y;
-    fo[c + FS_VZ * np] = vel.z;
-    fo[c + FS_U * np] = u;
-    fo[c + FS_P * np] = p;
-    fo[c + FS_T * np] = T;
-    fo[c + FS_A * np] = a;
+#pragma unroll
+        for (int jq = 0; jq < C::n; ++jq) st_plane(b.Unew + jq * np + o, c, U[jq]);
+    double* fo = b.fs_out + o;
+    st_plane(fo + FS_RHO * np, c, rho);
+    st_plane(fo + FS_VX * np, c, vel.x);
+    st_plane(fo + FS_VY * np, c, vel.y);
+    st_plane(fo + FS_VZ * np, c, vel.z);
+    st_plane(fo + FS_U * np, c, u);
+    st_plane(fo + FS_P * np, c, p);
+    st_plane(fo + FS_T * np, c, T);
+    st_plane(fo + FS_A * np, c, a);
     if (!check_data(rho, p, T, a, vel, max_vel, min_T, max_T)) atomicAdd(&b.counters[1], 1);
 }
 

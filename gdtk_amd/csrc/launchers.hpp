@@ -31,6 +31,9 @@ hipError_t launch_decode(const BlockDev& b, const IdealGasDev& gas, double* U, d
 // (FaceBatch), then the cell update (dt read from device memory; start[q] = first launch
 // index of block q, a multiple of 256; total = launch size).  numerics: 0 Eilmer 4, 1 Eilmer 5
 // (lmr) limiter smoothing and AUSMDV sound speed.
+// Per block and direction (10 doubles each, 3 directions a block): the first face's frame, and a
+// flag (which must be 0 before) set where another face's differs.
+hipError_t launch_frame_check(const BlockDev* tab, const FaceBatch& fb, int nblocks, double* frames, hipStream_t s);
 hipError_t launch_face_flux_batch(const BlockDev* tab, const FaceBatch& fb, int nblocks, int dims, int flux_calc,
                                  int numerics, double eps, const IdealGasDev& gas, hipStream_t s);
 hipError_t launch_cell_update_batch(const BlockDev* tab, const int64_t* start, int nblocks, int64_t total, int dims,

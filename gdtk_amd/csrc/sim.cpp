@@ -382,6 +382,46 @@ struct Sim {
         }
     }
 
+    // The directions whose faces all have the same axis-aligned frame (BlockDev::axis).
+    void find_axis_frames() {
+        const size_t nb = blocks.size();
+        const int nd = (cfg.dimensions == 3) ? 3 : 2;
+        FaceBatch fb{};
+        for (int d = 0; d < 3; ++d) {
+            fb.start[d] = fstart[d].p;
+            fb.total[d] = (d < nd) ? ftotal[d] : 0;
+        }
+        DevArr<double> frames;  // per block and direction: 9 components, then whether any face differs
+        frames.alloc(nb * 30);
+        HIPCHK(launch_frame_check(tab(1, 0, 0), fb, (int)nb, frames.p, stream));
+        std::vector<double> h(nb * 30);
+        HIPCHK(hipMemcpyAsync(h.data(), frames.p, h.size() * sizeof(double), hipMemcpyDeviceToHost, stream));
+        HIPCHK(hipStreamSynchronize(stream));
+        bool any = false;
+        for (size_t q = 0; q < nb; ++q)
+            for (int d = 0; d < nd; ++d) {
+                const double* r = &h[(q * 3 + d) * 10];
+                int ax[3], used = 0;
+                bool ok = r[9] == 0.0;
+                for (int l = 0; l < 3; ++l) {
+                    ax[l] = -1;
+                    for (int k = 0; k < 3; ++k) {
+                        const double v = r[3 * l + k];
+                        if (v == 0.0) continue;
+                        if (std::fabs(v) != 1.0 || ax[l] >= 0) ok = false;
+                        ax[l] = k | (v < 0.0 ? 4 : 0);
+                        used |= 1 << k;
+                    }
+                    if (ax[l] < 0) ok = false;
+                }
+                // in 2-D the third local direction is the third axis (its momentum is not kept)
+                if (!ok || used != 7 || (nd == 2 && (ax[2] & 3) != 2)) continue;
+                for (int l = 0; l < 3; ++l) blocks[q]->dev.axis[d][l] = ax[l];
+                any = true;
+            }
+        if (any) build_tabs();
+    }
+
     // Sets up the batched launches once every block exists (the reference does the same
     // after building all blocks: set_up_cell_mapping, exchange_geometry).
     void finalize() {
@@ -424,6 +464,7 @@ struct Sim {
         for (auto& bp : blocks) refresh_dev(*bp);
         build_tabs();
         build_starts();
+        find_axis_frames();
         build_tiles(kchunk, tile_x);
         // Geometry exchange: ghost cells of exchange sides take their source cells' lengths.
         if (any_exchange) {
@@ -659,6 +700,11 @@ struct Sim {
                 HIPCHK(hipMemcpy(b->fgeom[q].p, geo.face[q].data(), geo.face[q].size() * sizeof(double),
                                  hipMemcpyHostToDevice));
             }
+            for (int e = 0; e < 2; ++e) {
+                d.fdiv[q][e] = FastDiv::of((unsigned)std::max(d.nf[q][e], 1));
+                d.cdiv[e] = FastDiv::of((unsigned)(e == 0 ? desc.nic : desc.njc));
+            }
+            for (int e = 0; e < 3; ++e) d.axis[q][e] = -1;
             d.fgeom[q] = b->fgeom[q].p;
             d.flux[q] = nullptr;  // face-flux arrays: allocated when the face-per-thread kernels run
         }
