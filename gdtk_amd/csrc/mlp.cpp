@@ -137,8 +137,9 @@ int gdtk_hip_mlp_forward(int h, int batch, const float* x, float* y) {
         m.ensure_batch(batch);
         hipStream_t s = m.stream;
         HIPCHK(hipMemcpyAsync(m.xb.p, x, (size_t)batch * m.n_in * sizeof(float), hipMemcpyHostToDevice, s));
-        m.forward(batch, m.xb.p, s);
-        HIPCHK(hipMemcpyAsync(y, m.A[m.nlayer - 1].p, (size_t)batch * m.n_out * sizeof(float), hipMemcpyDeviceToHost, s));
+        const MlpPass q = m.pass(batch, m.xb.p, 1, (size_t)m.n_in, nullptr, 0, 0, nullptr, s);
+        HIPCHK(launch_mlp_pass(m.H, m.NH, q, 0, s));
+        HIPCHK(hipMemcpyAsync(y, m.yout.p, (size_t)batch * m.n_out * sizeof(float), hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
         return GDTK_OK;
     });
@@ -152,7 +153,9 @@ int gdtk_hip_mlp_loss_grad(int h, int batch, const float* x, const float* y, flo
         hipStream_t s = m.stream;
         HIPCHK(hipMemcpyAsync(m.xb.p, x, (size_t)batch * m.n_in * sizeof(float), hipMemcpyHostToDevice, s));
         HIPCHK(hipMemcpyAsync(m.yb.p, y, (size_t)batch * m.n_out * sizeof(float), hipMemcpyHostToDevice, s));
-        m.loss_grad(batch, m.xb.p, m.yb.p, s);
+        const int nz = m.loss_grad(
+            m.pass(batch, m.xb.p, 1, (size_t)m.n_in, m.yb.p, 1, (size_t)m.n_out, nullptr, s), s);
+        HIPCHK(launch_mlp_sum_grads(m.nparam, nz, m.gparts.p, m.grads.p, s));
         const double L = m.read_loss(batch, s);
         if (loss) *loss = (float)L;
         if (grad) {
@@ -184,10 +187,7 @@ int gdtk_hip_mlp_train(int h, int n, const float* x, const float* y, int batch, 
             int nacc = 0;
             for (int b = 0; b < nb; ++b) {
                 const int* ib = m.idx.p + (size_t)b * batch;
-                HIPCHK(launch_gather_batch(batch, m.n_in, n, ib, x, m.xb.p, s));
-                HIPCHK(launch_gather_batch(batch, m.n_out, n, ib, y, m.yb.p, s));
-                m.loss_grad(batch, m.xb.p, m.yb.p, s);
-                m.adam(lr, s);
+                m.adam(lr, m.loss_grad(m.pass(batch, x, (size_t)n, 1, y, (size_t)n, 1, ib, s), s), s);
                 // the loss of every 16th batch is read back (a host sync), the rest run ahead
                 if ((b & 15) == 15 || b == nb - 1) {
                     acc += m.read_loss(batch, s);

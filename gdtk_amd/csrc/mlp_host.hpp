@@ -23,15 +23,17 @@ struct Mlp {
     // pass the roundings unchanged and update the FP32 masters.
     int bf16_train = 0;
     DevArr<float> wq;
-    bool wq_fresh = false;
+    // the inner layers' weights (wq's with bf16_train) in the operand order of the training passes
+    DevArr<float> packed_w;
+    bool wq_fresh = false;  // wq (with bf16_train) and packed_w follow params
     // BF16 inference fragments and the concatenated biases
     DevArr<unsigned short> frag;
     DevArr<float> bias_cat;
     bool packed = false;
-    // training batch buffers
+    // training batch buffers (the layouts of MlpPass)
     int bcap = 0;
-    std::vector<DevArr<float>> Z, A;
-    DevArr<float> xb, yb, dA, dZ, part, xh, yh, gparts, cparts;
+    std::vector<DevArr<float>> act, dz;
+    DevArr<float> xb, yb, yout, loss, gparts;
     DevArr<int> idx;
     hipStream_t stream = nullptr;
 
@@ -60,98 +62,97 @@ struct Mlp {
     void ensure_batch(int B) {
         if (B <= bcap) return;
         bcap = B;
-        Z.clear();
-        A.clear();
-        Z.resize(nlayer);
-        A.resize(nlayer);
+        const size_t cells = (size_t)mlp_blocks(B) * 16;
+        act.clear();
+        dz.clear();
+        act.resize(nlayer);
+        dz.resize(nlayer);
+        MlpPass q{};
         for (int l = 0; l < nlayer; ++l) {
-            Z[l].alloc((size_t)B * out_w[l]);
-            A[l].alloc((size_t)B * out_w[l]);
+            act[l].alloc(cells * ((in_w[l] + 15) / 16 * 16));
+            dz[l].alloc(cells * ((out_w[l] + 15) / 16 * 16));
+            q.in_w[l] = in_w[l];
+            q.out_w[l] = out_w[l];
         }
-        const size_t wmax = (size_t)std::max(std::max(H, n_in), n_out);
         xb.alloc((size_t)B * n_in);
         yb.alloc((size_t)B * n_out);
-        dA.alloc((size_t)B * wmax);
-        dZ.alloc((size_t)B * wmax);
-        part.alloc((size_t)mse_parts(B, n_out));
-        size_t gp = 0;
-        for (int l = 0; l < nlayer; ++l)
-            gp = std::max(gp, (size_t)gemm_split(out_w[l], in_w[l], B) * out_w[l] * in_w[l]);
-        gparts.alloc(gp);
-        cparts.alloc((size_t)colsum_parts(B) * wmax);
+        yout.alloc((size_t)B * n_out);
+        loss.alloc((size_t)mlp_blocks(B));
+        gparts.alloc((size_t)mlp_grad_splits(q, nlayer, B) * nparam);
     }
 
+    // The batch's inputs at x[k xk + row xc] (rows idx[b], or b), targets likewise.
+    MlpPass pass(int B, const float* x, size_t xk, size_t xc, const float* y, size_t yk, size_t yc, const int* rows,
+                 hipStream_t s) {
+        MlpPass q{};
+        q.B = B;
+        q.n_in = n_in;
+        q.n_out = n_out;
+        q.bf16 = bf16_train;
+        q.x = x;
+        q.y = y;
+        q.xk = xk;
+        q.xc = xc;
+        q.yk = yk;
+        q.yc = yc;
+        q.idx = rows;
+        q.y_out = yout.p;
+        q.loss = loss.p;
+        const float* Wm = weights(s);
+        for (int l = 0; l < nlayer; ++l) {
+            q.W[l] = Wm + woff[l];
+            const bool in = l > 0 && l < nlayer - 1;
+            q.Wf[l] = in ? packed_w.p + (size_t)(l - 1) * 2 * H * H : nullptr;
+            q.Wb[l] = in ? q.Wf[l] + H * H : nullptr;
+            q.b[l] = params.p + boff[l];  // the biases stay FP32 (as in inference)
+            q.act[l] = act[l].p;
+            q.dz[l] = dz[l].p;
+            q.in_w[l] = in_w[l];
+            q.out_w[l] = out_w[l];
+            q.woff[l] = woff[l];
+            q.boff[l] = boff[l];
+        }
+        return q;
+    }
+
+    size_t inner() const { return (size_t)(nlayer - 2); }
     const float* weights(hipStream_t s) {
-        if (!bf16_train) return params.p;
         if (!wq_fresh) {
-            wq.reserve(nparam);
-            HIPCHK(launch_round_bf16(nparam, params.p, wq.p, s));
+            if (bf16_train) {
+                wq.reserve(nparam);
+                HIPCHK(launch_round_bf16(nparam, params.p, wq.p, s));
+            }
+            packed_w.reserve(inner() * 2 * H * H);
+            HIPCHK(launch_mlp_operands(nparam, bf16_train ? wq.p : params.p, packed_w.p, H, woff[1], inner(), s));
             wq_fresh = true;
         }
-        return wq.p;
+        return bf16_train ? wq.p : params.p;
     }
 
-    // Forward pass of a cell-major batch X [B][n_in]; output A[last] = Z[last].
-    void forward(int B, const float* X, hipStream_t s) {
-        const float* in = X;
-        if (bf16_train) {
-            HIPCHK(launch_round_bf16((size_t)B * n_in, X, xq_buf(B), s));
-            in = xq.p;
-        }
-        const float* Wt = weights(s);
-        for (int l = 0; l < nlayer; ++l) {
-            const int ni = in_w[l], no = out_w[l];
-            // Z[b][o] = sum_k in[b][k] W[o][k]; the biases stay FP32 (as in inference)
-            HIPCHK(launch_gemm_f32(B, no, ni, in, ni, 1, Wt + woff[l], 1, ni, Z[l].p, no, 0, s));
-            HIPCHK(launch_bias_act(B, no, params.p + boff[l], Z[l].p, A[l].p, l < nlayer - 1 ? 1 : 0, bf16_train, s));
-            in = A[l].p;
-        }
-    }
-    DevArr<float> xq;
-    float* xq_buf(int B) {
-        xq.reserve((size_t)B * n_in);
-        return xq.p;
-    }
-
-    // Backward pass after forward(B, X) and the loss gradient in dZ (output layer).
-    void backward(int B, const float* X, hipStream_t s) {
-        const float* Wt = weights(s);
-        for (int l = nlayer - 1; l >= 0; --l) {
-            const int ni = in_w[l], no = out_w[l];
-            const float* in = (l == 0) ? (bf16_train ? xq.p : X) : A[l - 1].p;
-            // dW[o][k] = sum_b dZ[b][o] in[b][k]  (split over the batch)
-            HIPCHK(launch_gemm_f32_split(no, ni, B, dZ.p, 1, no, in, ni, 1, grads.p + woff[l], ni, gparts.p,
-                                         gemm_split(no, ni, B), s));
-            HIPCHK(launch_colsum(B, no, dZ.p, grads.p + boff[l], cparts.p, s));
-            if (l == 0) break;
-            // dA[b][k] = sum_o dZ[b][o] W[o][k]
-            HIPCHK(launch_gemm_f32(B, ni, no, dZ.p, no, 1, Wt + woff[l], ni, 1, dA.p, ni, 0, s));
-            HIPCHK(launch_gelu_back((size_t)B * ni, Z[l - 1].p, dA.p, dZ.p, s));
-        }
-    }
-
-    // Mean-squared-error loss of the batch (sum of part[] / (B n_out)) and its gradient.
-    void loss_grad(int B, const float* X, const float* Y, hipStream_t s) {
-        forward(B, X, s);
-        HIPCHK(launch_mse(B, n_out, A[nlayer - 1].p, Y, dZ.p, part.p, s));
-        backward(B, X, s);
+    // Loss and gradient shares of a batch; the number of shares in gparts.
+    int loss_grad(const MlpPass& q, hipStream_t s) {
+        const int nz = mlp_grad_splits(q, nlayer, q.B);
+        HIPCHK(launch_mlp_pass(H, NH, q, 1, s));
+        HIPCHK(launch_mlp_weight_grad(q, nlayer, nz, nparam, gparts.p, s));
+        return nz;
     }
 
     double read_loss(int B, hipStream_t s) {
-        const int np = mse_parts(B, n_out);
+        const int np = mlp_blocks(B);
         std::vector<float> h((size_t)np);
-        HIPCHK(hipMemcpyAsync(h.data(), part.p, np * sizeof(float), hipMemcpyDeviceToHost, s));
+        HIPCHK(hipMemcpyAsync(h.data(), loss.p, np * sizeof(float), hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
         double acc = 0.0;
         for (float v : h) acc += v;
         return acc / ((double)B * n_out);
     }
 
-    void adam(float lr, hipStream_t s) {
+    void adam(float lr, int nz, hipStream_t s) {
         ++adam_t;
-        HIPCHK(launch_adam(nparam, params.p, grads.p, am.p, av.p, lr, 0.9f, 0.999f, 1.0e-8f, adam_t, s));
+        HIPCHK(launch_mlp_adam(nparam, nz, gparts.p, params.p, am.p, av.p, bf16_train ? wq.p : nullptr, packed_w.p, H,
+                               woff[1], inner(), lr, 0.9f, 0.999f, 1.0e-8f, adam_t, s));
         packed = false;
-        wq_fresh = false;
+        wq_fresh = true;
     }
 
     void pack(hipStream_t s) {
