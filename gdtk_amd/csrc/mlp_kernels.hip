@@ -39,7 +39,7 @@ constexpr float GELU_C = 0.044715f;
 __device__ __forceinline__ float gelu_fast(float z) {
     constexpr float A = -2.0f * 1.4426950408889634f * 0.7978845608028654f;
     constexpr float B = 0.044715f * A;
-    const float w = z * (A + B * (z * z));
+    const float w = z * fmaf(B, z * z, A);
     return z * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(w));
 }
 
@@ -104,45 +104,56 @@ hipError_t launch_mlp_pack(const float* W, int n_out, int n_in, int chain, unsig
 // 32), NH hidden layers, n_in <= 32, n_out <= 16.  frag: packed layers in order; bias:
 // FP32 biases in order.
 //
-// A workgroup of 4 waves serves 128 cells, each wave two 16-cell column blocks (CB = 2), so
-// every weight fragment read feeds two MFMAs.  The H x H layers stream their fragments
-// through LDS one k-step at a time (NRB fragments = 16 KiB for H = 256), double-buffered:
-// the global loads of k-step s+1 are in flight while k-step s is multiplied.  The small
-// first and last layers read their fragments straight from global memory (L2).
-constexpr int INF_WAVES = 4, INF_CB = 2;
-constexpr int INF_CELLS = INF_WAVES * INF_CB * 16;
-
+// A workgroup of 8 waves (4 for H = 64) has 16 cells a wave.  The H x H layers stream their
+// fragments through LDS two k-steps at a time (32 KiB for H = 256), loaded straight to LDS and
+// double-buffered: one barrier a stage, the next stage's loads under this one's products.  The
+// small first and last layers read their fragments from global memory (L2).  The sums start
+// from the biases.
+//
+// GELU bounds it: per 16 x 16 block a third more vector cycles (two transcendental
+// instructions a value) than the matrix cores need, and each of them waits for the other
+// within a wave.  So the registers are held to 128 a wave (16 cells, not 32, and scalar
+// addresses), for four waves a SIMD that fill each other's gaps: 2^19 cells through the
+// 3 x 256 network in 239 us with the matrix cores busy for 60, against 432 us with one wave
+// a SIMD of 32 cells each and 275 with two.
 // count (may be null): the number of leading cells to evaluate, read from device memory (at
 // most n, the arrays' stride); workgroups past it exit at once.
-template <int H, int NH>
-__global__ __launch_bounds__(256, 1) void k_mlp_infer(const float* __restrict__ x, int n_in, int n,
+template <int H, int NH, int WAVES, int CB>
+__global__ __launch_bounds__(64 * WAVES, 4) void k_mlp_infer(const float* __restrict__ x, int n_in, int n,
                                                       const unsigned* __restrict__ count,
                                                       const unsigned short* __restrict__ frag,
                                                       const float* __restrict__ bias, int n_out, float* __restrict__ y) {
+    constexpr int CELLS = WAVES * CB * 16;
     const int stride = n;
     if (count) {
         const unsigned c = *count;
         n = (c < (unsigned)n) ? (int)c : n;
-        if ((int)(blockIdx.x * INF_CELLS) >= n) return;
+        if ((int64_t)blockIdx.x * CELLS >= n) return;
     }
     constexpr int NRB = H / 16, NKS = H / 32;
-    constexpr int FRAG_PER_STEP = NRB * 64;                 // 16-byte fragments per k-step
-    constexpr int LOADS = FRAG_PER_STEP / 256;               // per thread
-    static_assert(FRAG_PER_STEP % 256 == 0, "k-step fragments must split over the workgroup");
+    constexpr int KS = 2;                                   // k-steps per stage
+    constexpr int FRAG_PER_STEP = KS * NRB * 64;            // 16-byte fragments per stage
+    constexpr int LOADS = FRAG_PER_STEP / (64 * WAVES);      // per thread
+    static_assert(FRAG_PER_STEP % (64 * WAVES) == 0, "k-step fragments must split over the workgroup");
     __shared__ bf16x8 lds[2][FRAG_PER_STEP];
     __shared__ float bias_s[NH * H + 16];
-    for (int k = threadIdx.x; k < NH * H + n_out; k += 256) bias_s[k] = bias[k];
+    for (int k = threadIdx.x; k < NH * H + n_out; k += 64 * WAVES) bias_s[k] = bias[k];
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, g = lane >> 4;
-    const int cell0 = blockIdx.x * INF_CELLS + wave * (INF_CB * 16);
+    const int cell0 = blockIdx.x * CELLS + wave * (CB * 16);
     const bf16x8* F = reinterpret_cast<const bf16x8*>(frag);
+    const unsigned lane16 = 16 * lane;
+    auto frag_at = [lane16](const bf16x8* f) {  // scalar base, 32-bit lane offset
+        typedef const __attribute__((address_space(1))) char* gptr;
+        return *(const __attribute__((address_space(1))) bf16x8*)((gptr)f + lane16);
+    };
 
-    bf16x8 act[INF_CB][NKS];
-    f32x4 acc[INF_CB][NRB];
+    bf16x8 act[CB][NKS];
+    f32x4 acc[CB][NRB];
     // first layer: one k-step over the zero-padded inputs (slots k = 8 g + j)
 #pragma unroll
-    for (int cb = 0; cb < INF_CB; ++cb) {
+    for (int cb = 0; cb < CB; ++cb) {
         const int cell = cell0 + cb * 16 + r;
         u16x8 xb;
 #pragma unroll
@@ -152,83 +163,95 @@ __global__ __launch_bounds__(256, 1) void k_mlp_infer(const float* __restrict__ 
         }
         act[cb][0] = __builtin_bit_cast(bf16x8, xb);
     }
-#pragma unroll
-    for (int rb = 0; rb < NRB; ++rb) {
-        const bf16x8 a = F[rb * 64 + lane];
-#pragma unroll
-        for (int cb = 0; cb < INF_CB; ++cb)
-            acc[cb][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, act[cb][0], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-    }
-    const bf16x8* Fl = F + NRB * 64;
-    __syncthreads();  // biases in LDS
+    // the sums start from the biases: accumulator i of row block rb is row 16 rb + 4 g + i
     const float* bl = bias_s;
-    for (int layer = 0; layer < NH; ++layer) {
-        // bias + GELU + BF16 -> B fragments of the next layer
+    auto start = [&] {
 #pragma unroll
-        for (int s = 0; s < NKS; ++s) {
-            const float4 b0 = *reinterpret_cast<const float4*>(bl + 32 * s + 4 * g);
-            const float4 b1 = *reinterpret_cast<const float4*>(bl + 32 * s + 16 + 4 * g);
+        for (int rb = 0; rb < NRB; ++rb) {
+            const f32x4 b = *reinterpret_cast<const f32x4*>(bl + 16 * rb + 4 * g);
 #pragma unroll
-            for (int cb = 0; cb < INF_CB; ++cb) {
-                bf16x8 v;
-                v[0] = (__bf16)gelu_fast(acc[cb][2 * s][0] + b0.x);
-                v[1] = (__bf16)gelu_fast(acc[cb][2 * s][1] + b0.y);
-                v[2] = (__bf16)gelu_fast(acc[cb][2 * s][2] + b0.z);
-                v[3] = (__bf16)gelu_fast(acc[cb][2 * s][3] + b0.w);
-                v[4] = (__bf16)gelu_fast(acc[cb][2 * s + 1][0] + b1.x);
-                v[5] = (__bf16)gelu_fast(acc[cb][2 * s + 1][1] + b1.y);
-                v[6] = (__bf16)gelu_fast(acc[cb][2 * s + 1][2] + b1.z);
-                v[7] = (__bf16)gelu_fast(acc[cb][2 * s + 1][3] + b1.w);
-                act[cb][s] = v;
-            }
+            for (int cb = 0; cb < CB; ++cb) acc[cb][rb] = b;
         }
         bl += H;
-        if (layer == NH - 1) break;
-#pragma unroll
-        for (int cb = 0; cb < INF_CB; ++cb)
-#pragma unroll
-            for (int rb = 0; rb < NRB; ++rb) acc[cb][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        // k-step s of this layer: fragments Fl[(rb * NKS + s) * 64 + lane] for rb < NRB
-        bf16x8 pre[LOADS];
+    };
+    // k-step s of a layer: fragments Fl[(rb * NKS + s) * 64 + lane], rb < NRB, straight to LDS
+    const bf16x8* Fl = F + NRB * 64;
+    auto stage = [&](int s, int buf) {
 #pragma unroll
         for (int q = 0; q < LOADS; ++q) {
-            const int f = threadIdx.x + 256 * q;  // f = rb * 64 + lane'
-            pre[q] = Fl[((f >> 6) * NKS + 0) * 64 + (f & 63)];
+            const int f = WAVES * q + wave, rb = f / KS, k = f % KS;
+            const bf16x8* src = Fl + (rb * NKS + KS * s + k) * 64;
+            asm("" : "+s"(src));  // stays a scalar base: lane addresses kept over the loop spill
+            __builtin_amdgcn_global_load_lds(
+                (const __attribute__((address_space(1))) void*)(
+                    (const __attribute__((address_space(1))) char*)src + lane16),
+                (__attribute__((address_space(3))) void*)(&lds[buf][f * 64]), 16, 0, 0);
         }
-#pragma unroll
-        for (int q = 0; q < LOADS; ++q) lds[0][threadIdx.x + 256 * q] = pre[q];
+    };
+    // this wave's loads have landed (s_waitcnt vmcnt(0)), then everybody's
+    auto staged = [&] {
+        __builtin_amdgcn_s_waitcnt(0x0f70);
         __syncthreads();
+    };
+    if (NH > 1) stage(0, 0);
+    __syncthreads();  // biases in LDS
+    start();
 #pragma unroll
-        for (int s = 0; s < NKS; ++s) {
-            const int buf = s & 1;
-            if (s + 1 < NKS) {
+    for (int rb = 0; rb < NRB; ++rb) {
+        const bf16x8 a = frag_at(F + rb * 64);
 #pragma unroll
-                for (int q = 0; q < LOADS; ++q) {
-                    const int f = threadIdx.x + 256 * q;
-                    pre[q] = Fl[((f >> 6) * NKS + (s + 1)) * 64 + (f & 63)];
+        for (int cb = 0; cb < CB; ++cb)
+            acc[cb][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, act[cb][0], acc[cb][rb], 0, 0, 0);
+        if (rb % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll 1
+    for (int layer = 0; layer < NH; ++layer) {
+        // GELU + BF16 -> B fragments of the next layer
+#pragma unroll
+        for (int s = 0; s < NKS; ++s)
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+                bf16x8 v;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    v[i] = (__bf16)gelu_fast(acc[cb][2 * s][i]);
+                    v[4 + i] = (__bf16)gelu_fast(acc[cb][2 * s + 1][i]);
                 }
+                act[cb][s] = v;
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        if (layer == NH - 1) break;
+        start();
+#pragma unroll
+        for (int s = 0; s < NKS / KS; ++s) {
+            const int buf = (NKS / KS == 1) ? layer & 1 : s & 1;
+            staged();
+            if (s + 1 < NKS / KS) {
+                stage(s + 1, buf ^ 1);
+            } else {
+                Fl += NRB * NKS * 64;
+                if (layer + 2 < NH) stage(0, buf ^ 1);
             }
 #pragma unroll
             for (int rb = 0; rb < NRB; ++rb) {
-                const bf16x8 a = lds[buf][rb * 64 + lane];
 #pragma unroll
-                for (int cb = 0; cb < INF_CB; ++cb)
-                    acc[cb][rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, act[cb][s], acc[cb][rb], 0, 0, 0);
-            }
-            if (s + 1 < NKS) {
+                for (int k = 0; k < KS; ++k) {
+                    const bf16x8 a = lds[buf][(rb * KS + k) * 64 + lane];
 #pragma unroll
-                for (int q = 0; q < LOADS; ++q) lds[buf ^ 1][threadIdx.x + 256 * q] = pre[q];
+                    for (int cb = 0; cb < CB; ++cb)
+                        acc[cb][rb] =
+                            __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, act[cb][KS * s + k], acc[cb][rb], 0, 0, 0);
+                }
+                if (rb % 2 == 1) __builtin_amdgcn_sched_barrier(0);
             }
-            __syncthreads();
         }
-        Fl += NRB * NKS * 64;
     }
     // output layer: one 16-row block, fragments from global
 #pragma unroll
-    for (int cb = 0; cb < INF_CB; ++cb) {
+    for (int cb = 0; cb < CB; ++cb) {
         f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int s = 0; s < NKS; ++s) o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Fl[s * 64 + lane], act[cb][s], o, 0, 0, 0);
+        for (int s = 0; s < NKS; ++s) o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag_at(Fl + s * 64), act[cb][s], o, 0, 0, 0);
         const int cell = cell0 + cb * 16 + r;
         if (cell < n) {
 #pragma unroll
@@ -243,13 +266,13 @@ __global__ __launch_bounds__(256, 1) void k_mlp_infer(const float* __restrict__ 
 hipError_t launch_mlp_infer(int H, int NH, const float* x, int n_in, int n, const unsigned short* frag,
                             const float* bias, int n_out, float* y, hipStream_t s, const unsigned* count) {
     if (n <= 0) return hipSuccess;
-    const unsigned grid = (unsigned)((n + INF_CELLS - 1) / INF_CELLS);
+    auto grid = [n](int cells) { return dim3((unsigned)(((int64_t)n + cells - 1) / cells)); };
     if (H == 256 && NH == 3) {
-        hipLaunchKernelGGL((k_mlp_infer<256, 3>), dim3(grid), dim3(256), 0, s, x, n_in, n, count, frag, bias, n_out,
-                           y);
+        hipLaunchKernelGGL((k_mlp_infer<256, 3, 8, 1>), grid(128), dim3(512), 0, s, x, n_in, n, count, frag, bias,
+                           n_out, y);
     } else if (H == 64 && NH == 2) {
-        hipLaunchKernelGGL((k_mlp_infer<64, 2>), dim3(grid), dim3(256), 0, s, x, n_in, n, count, frag, bias, n_out,
-                           y);
+        hipLaunchKernelGGL((k_mlp_infer<64, 2, 4, 1>), grid(64), dim3(256), 0, s, x, n_in, n, count, frag, bias,
+                           n_out, y);
     } else {
         return hipErrorNotSupported;
     }
