@@ -118,6 +118,12 @@ struct Sim {
     DevArr<unsigned> ctr;  // the stages' counters, then the control words of queued steps
     StageCounters sc;
     unsigned* ctr_host = nullptr;  // pinned copy of ctr
+    // Interior cells of a plane on their way to the host: two pinned buffers of at most PACK_CELLS
+    // (4 MiB) each, which the packing kernel and the copy to the caller take in turn.
+    static constexpr int64_t PACK_CELLS = (int64_t)1 << 19;
+    double* pack_host = nullptr;
+    int64_t pack_cells = 0;
+    std::mutex pack_mu;
     // Events around the chemistry of each queued step.
     static constexpr int MAX_QUEUED = 16;
     std::vector<hipEvent_t> qev;
@@ -181,6 +187,7 @@ struct Sim {
         if (cev1) (void)hipEventDestroy(cev1);
         if (cfail_host) (void)hipHostFree(cfail_host);
         if (ctr_host) (void)hipHostFree(ctr_host);
+        if (pack_host) (void)hipHostFree(pack_host);
         if (dt_host) (void)hipHostFree(dt_host);
         for (auto& e : qev)
             if (e) (void)hipEventDestroy(e);
@@ -916,23 +923,24 @@ struct Sim {
         else if (field == GDTK_FIELD_VOLUME) src = b.vol.p;
         else if (field >= GDTK_FIELD_ILENGTH && field <= GDTK_FIELD_KLENGTH) src = b.len.p + (field - GDTK_FIELD_ILENGTH) * np;
         else if (field != GDTK_FIELD_SHOCK || !b.shock.p) throw Error(GDTK_ERR_ARG, "bad field");
-        std::vector<double> h(np);
-        HIPCHK(hipStreamSynchronize(stream));
-        if (src) {
-            HIPCHK(hipMemcpy(h.data(), src, np * sizeof(double), hipMemcpyDeviceToHost));
-        } else {
-            std::vector<unsigned char> hs(np);
-            HIPCHK(hipMemcpy(hs.data(), b.shock.p, np, hipMemcpyDeviceToHost));
-            for (size_t q = 0; q < np; ++q) h[q] = hs[q];
+        const int64_t ncell = b.ncell();
+        std::lock_guard<std::mutex> lk(pack_mu);
+        const int64_t cells = std::min(ncell, PACK_CELLS);
+        if (pack_cells < cells) {
+            if (pack_host) HIPCHK(hipHostFree(pack_host));
+            pack_host = nullptr;
+            pack_cells = 0;
+            HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&pack_host), 2 * (size_t)cells * sizeof(double)));
+            pack_cells = cells;
         }
-        const int kg = (cfg.dimensions == 3) ? NGHOST : 0;
-        for (int k = 0; k < b.nkc; ++k)
-            for (int j = 0; j < b.njc; ++j)
-                for (int i = 0; i < b.nic; ++i) {
-                    size_t c = ((size_t)k * b.njc + j) * b.nic + i;
-                    size_t pc = (size_t)(i + NGHOST) + (size_t)d.NI * ((size_t)(j + NGHOST) + (size_t)d.NJ * (size_t)(k + kg));
-                    out[c] = h[pc];
-                }
+        auto count = [&](int64_t c0) { return std::min(cells, ncell - c0); };
+        HIPCHK(launch_pack_plane(d, src, 0, cells, pack_host, stream));
+        for (int64_t c0 = 0, q = 0; c0 < ncell; c0 += cells, q ^= 1) {
+            HIPCHK(hipStreamSynchronize(stream));
+            if (c0 + cells < ncell)
+                HIPCHK(launch_pack_plane(d, src, c0 + cells, count(c0 + cells), pack_host + (q ^ 1) * cells, stream));
+            std::memcpy(out + c0, pack_host + q * cells, (size_t)count(c0) * sizeof(double));
+        }
     }
 
     // The fused stage kernel serves the single-species gas with the AUSMDV or EFM
