@@ -63,6 +63,9 @@ struct BlockDev {
     int64_t nface[3];
     int bc_kind[6];
     double inflow[6][FS_MAX_PLANES];  // an inflow face's flow state, plane order
+    // Per padded cell: the first of the ghost records that copy the cell, or -1; the others follow
+    // by GhostRec::next.
+    int* ghead;
     int* counters;                // [0] decode failures, [1] invalid cells
     // Shock indicator per padded cell (0 or 1; adaptive flux calculator only, else null):
     // interior cells hold the last detection, ghost cells the copy made by the ghost fill
@@ -136,7 +139,7 @@ struct alignas(64) GhostRec {
     unsigned char* sdst;
     const unsigned char* ssrc;  // null: indicator 0 (inflow)
     int npd, nps, nface;  // plane strides of the destination, the source and the frame
-    int pad_;
+    int next;             // another record with the same source cell, or -1 (BlockDev::ghead)
 };
 
 // The faces of every direction of every block in one launch: per direction d, the first

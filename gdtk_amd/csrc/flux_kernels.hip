@@ -28,7 +28,7 @@ __device__ __forceinline__ int64_t ghost_pidx(const BlockDev& b, int side, int a
 // The record of one ghost cell (layer `layer` at in-face position (a, bb) of side `side`) for the
 // boundary kinds that read the block's own cells: internal_copy_then_reflect.d:111-134,
 // flow_state_copy.d:92-107, extrapolate_copy.d:124-140 (xOrder 0).
-__device__ __forceinline__ GhostRec ghost_own(const BlockDev& b, int side, int a, int bb, int layer) {
+__device__ __forceinline__ GhostRec ghost_own(const BlockDev& b, int side, int a, int bb, int layer, int*& head) {
     const int d = side / 2;
     const bool lo = (side % 2) == 0;
     const int nd = (d == 0) ? b.nic : (d == 1) ? b.njc : b.nkc;
@@ -39,6 +39,7 @@ __device__ __forceinline__ GhostRec ghost_own(const BlockDev& b, int side, int a
     r.dst = fs + g;
     r.npd = r.nps = (int)b.npad;
     r.sdst = b.shock ? b.shock + g : nullptr;
+    r.next = -1;
     if (kind == BC_INFLOW_SUPERSONIC) {
         r.src = b.inflow[side];
         r.nps = 1;
@@ -47,6 +48,7 @@ __device__ __forceinline__ GhostRec ghost_own(const BlockDev& b, int side, int a
     const int from = (kind == BC_SLIP_WALL) ? layer : 0;  // cells inside the side
     const int64_t s = ghost_pidx(b, side, a, bb, -1 - from);
     r.src = fs + s;
+    head = b.ghead + s;
     r.ssrc = b.shock ? b.shock + s : nullptr;
     if (kind == BC_SLIP_WALL) {
         const int pos = lo ? 0 : nd;
@@ -60,9 +62,12 @@ __device__ __forceinline__ GhostRec ghost_own(const BlockDev& b, int side, int a
 
 // Ghost cells of every side of every block: the records of the fill for one flow-state copy
 // (the blocks' fs_in), made once, or (lengths) the geometry exchange of
-// full_face_copy.d:1576-1625, the cell lengths of exchange sides, done once too.
+// full_face_copy.d:1576-1625, the cell lengths of exchange sides, done once too.  The records of
+// one copy are chained by their source cell (BlockDev::ghead, GhostRec::next), and the other
+// copy's the same way (link: the first copy's records).
 __global__ void k_ghost_setup(const BlockDev* __restrict__ tab, const SideDev* __restrict__ sides, int nsides,
-                              int64_t total, GhostRec* __restrict__ rec, int lengths) {
+                              int64_t total, GhostRec* __restrict__ rec, const GhostRec* __restrict__ link,
+                              int lengths) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= total) return;
     int lo = 0, hi = nsides - 1;
@@ -78,7 +83,11 @@ __global__ void k_ghost_setup(const BlockDev* __restrict__ tab, const SideDev* _
     const int a = (int)(face % sd.na), bb = (int)(face / sd.na);
     const BlockDev& b = tab[sd.blk];
     if (sd.kind != BC_EXCHANGE) {
-        if (!lengths) rec[t] = ghost_own(b, sd.side, a, bb, layer);
+        if (lengths) return;
+        int* head = nullptr;  // an inflow's ghosts copy no cell
+        GhostRec g = ghost_own(b, sd.side, a, bb, layer, head);
+        if (head) g.next = link ? link[t].next : atomicExch(head, (int)t);
+        rec[t] = g;
         return;
     }
     const BlockDev& o = tab[sd.oblk];
@@ -98,6 +107,7 @@ __global__ void k_ghost_setup(const BlockDev* __restrict__ tab, const SideDev* _
     g.nps = (int)o.npad;
     g.sdst = b.shock ? b.shock + dst : nullptr;
     g.ssrc = o.shock ? o.shock + src : nullptr;
+    g.next = link ? link[t].next : atomicExch(o.ghead + src, (int)t);
     rec[t] = g;
 }
 
@@ -290,12 +300,15 @@ hipError_t launch_frame_check(const BlockDev* tab, const FaceBatch& fb, int nblo
 // invalid-cell check (fluidblock.d:607-676).
 template <int DIM, int STAGE>
 __device__ __forceinline__ void cell_update_one(const BlockDev& b, const IdealGasDev& gas, double dt, double low_T,
-                                                double max_vel, double min_T, double max_T, unsigned t) {
+                                                double max_vel, double min_T, double max_T, unsigned t,
+                                                const GhostRec* push) {
     using C = CQ<DIM>;
     unsigned i, j;
     const unsigned rest = b.cdiv[0].divmod(t, i);
     const unsigned k = b.cdiv[1].divmod(rest, j);
     const unsigned c = (i + NGHOST) + (unsigned)b.NI * ((j + NGHOST) + (unsigned)b.NJ * (k + (DIM == 3 ? NGHOST : 0)));
+    if (DIM == 3) push = nullptr;
+    const int head = push ? ghost_head(b, (int)i, (int)j, c) : -1;
     // Faces in the order W, E, S, N, B, T with outsigns -1, +1: per direction the low face and
     // the one `step` behind it.
     unsigned lo[3], step[3], org[3];
@@ -326,16 +339,20 @@ __device__ __forceinline__ void cell_update_one(const BlockDev& b, const IdealGa
         }
         si[jq] = s;
     }
-    update_decode_store<DIM, STAGE>(b, gas, c, si, dt, low_T, max_vel, min_T, max_T);
+    update_decode_store<DIM, STAGE>(b, gas, c, si, dt, low_T, max_vel, min_T, max_T, push, head);
 }
 
 // Cells of every block in one launch (block ranges aligned as in k_face_flux_batch); dt
-// is read from device memory.
+// is read from device memory.  push (may be null, always in 3-D): the ghost records of the copy
+// that is written; the threads then write the ghost cells that copy their cells too.  The values
+// are at hand there, where a fill of its own costs a launch, its gap and a chain of scattered
+// loads before each stage: a step of a 2-D block of 200 x 100 cells 36.8 -> 34.1 us.
 template <int DIM, int STAGE>
 __global__ __launch_bounds__(256) void k_cell_update_batch(const BlockDev* __restrict__ tab,
                                                            const int64_t* __restrict__ start, int nblocks,
                                                            const double* __restrict__ dtp, CellLimits lim,
-                                                           IdealGasDev gas, const unsigned* __restrict__ stop) {
+                                                           IdealGasDev gas, const unsigned* __restrict__ stop,
+                                                           const GhostRec* __restrict__ push) {
     if (*stop) return;  // StepControl: the run waits for the host
     const int64_t w0 = (int64_t)blockIdx.x * blockDim.x;
     int lo = 0, hi = nblocks - 1;
@@ -348,7 +365,7 @@ __global__ __launch_bounds__(256) void k_cell_update_batch(const BlockDev* __res
     const BlockDev& b = tab[q];
     const int64_t t = w0 - start[q] + threadIdx.x;
     if (t >= (int64_t)b.nic * b.njc * b.nkc) return;
-    cell_update_one<DIM, STAGE>(b, gas, *dtp, lim.low_T, lim.max_vel, lim.min_T, lim.max_T, (unsigned)t);
+    cell_update_one<DIM, STAGE>(b, gas, *dtp, lim.low_T, lim.max_vel, lim.min_T, lim.max_T, (unsigned)t, push);
 }
 
 // The block time-step estimates of many blocks in two launches (fluidblock.d:987-1084 per
@@ -556,24 +573,24 @@ hipError_t launch_shock_detect(const BlockDev* tab, const FaceBatch& fb, const i
 
 hipError_t launch_cell_update_batch(const BlockDev* tab, const int64_t* start, int nblocks, int64_t total, int dims,
                                    int stage, const double* dtp, const CellLimits& lim, const IdealGasDev& gas,
-                                   const unsigned* stop, hipStream_t s) {
+                                   const unsigned* stop, const GhostRec* push, hipStream_t s) {
     if (total <= 0) return hipSuccess;
     dim3 grid(nblk(total, 256)), blk(256);
     if (dims == 3) {
-        if (stage == 1) hipLaunchKernelGGL((k_cell_update_batch<3, 1>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas, stop);
-        else hipLaunchKernelGGL((k_cell_update_batch<3, 2>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas, stop);
+        if (stage == 1) hipLaunchKernelGGL((k_cell_update_batch<3, 1>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas, stop, push);
+        else hipLaunchKernelGGL((k_cell_update_batch<3, 2>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas, stop, push);
     } else {
-        if (stage == 1) hipLaunchKernelGGL((k_cell_update_batch<2, 1>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas, stop);
-        else hipLaunchKernelGGL((k_cell_update_batch<2, 2>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas, stop);
+        if (stage == 1) hipLaunchKernelGGL((k_cell_update_batch<2, 1>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas, stop, push);
+        else hipLaunchKernelGGL((k_cell_update_batch<2, 2>), grid, blk, 0, s, tab, start, nblocks, dtp, lim, gas, stop, push);
     }
     return hipGetLastError();
 }
 
 hipError_t launch_ghost_setup(const BlockDev* tab, const SideDev* sides, int nsides, int64_t total, GhostRec* rec,
-                              hipStream_t s) {
+                              const GhostRec* link, hipStream_t s) {
     if (total <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_ghost_setup, dim3(nblk(total, 256)), dim3(256), 0, s, tab, sides, nsides, total, rec,
-                       rec ? 0 : 1);
+                       link, rec ? 0 : 1);
     return hipGetLastError();
 }
 

@@ -14,7 +14,8 @@ __global__ __launch_bounds__(256) void k_cell_update_species(const BlockDev* __r
                                                              const int64_t* __restrict__ start, int nblocks,
                                                              const double* __restrict__ dtp, CellLimits lim,
                                                              const ChemDev* __restrict__ cdp,
-                                                             const unsigned* __restrict__ stop) {
+                                                             const unsigned* __restrict__ stop,
+                                                             const GhostRec* __restrict__ push) {
     if (*stop) return;  // StepControl: the run waits for the host
     const int64_t w0 = (int64_t)blockIdx.x * blockDim.x;
     int lo = 0, hi = nblocks - 1;
@@ -27,7 +28,7 @@ __global__ __launch_bounds__(256) void k_cell_update_species(const BlockDev* __r
     const BlockDev& b = tab[q];
     const int64_t t = w0 - start[q] + threadIdx.x;
     if (t >= (int64_t)b.nic * b.njc * b.nkc) return;
-    cell_update_species<DIM, STAGE, NSP>(b, *cdp, *dtp, lim.low_T, lim.max_vel, lim.min_T, lim.max_T, t);
+    cell_update_species<DIM, STAGE, NSP>(b, *cdp, *dtp, lim.low_T, lim.max_vel, lim.min_T, lim.max_T, t, push);
 }
 
 // encode_conserved (fvcell.d:511-583) of every active cell of one block.
@@ -88,14 +89,14 @@ bool species_supported(int nsp) { return nsp == 2 || nsp == 5; }
 template <int NSP>
 static void cell_species(const BlockDev* tab, const int64_t* start, int nb, int64_t total, int dims, int stage,
                          const double* dtp, const CellLimits& lim, const ChemDev* cd, const unsigned* stop,
-                         hipStream_t s) {
+                         const GhostRec* push, hipStream_t s) {
     dim3 g(nblk256(total)), blk(256);
     if (dims == 3) {
-        if (stage == 1) hipLaunchKernelGGL((k_cell_update_species<3, 1, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd, stop);
-        else hipLaunchKernelGGL((k_cell_update_species<3, 2, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd, stop);
+        if (stage == 1) hipLaunchKernelGGL((k_cell_update_species<3, 1, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd, stop, push);
+        else hipLaunchKernelGGL((k_cell_update_species<3, 2, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd, stop, push);
     } else {
-        if (stage == 1) hipLaunchKernelGGL((k_cell_update_species<2, 1, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd, stop);
-        else hipLaunchKernelGGL((k_cell_update_species<2, 2, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd, stop);
+        if (stage == 1) hipLaunchKernelGGL((k_cell_update_species<2, 1, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd, stop, push);
+        else hipLaunchKernelGGL((k_cell_update_species<2, 2, NSP>), g, blk, 0, s, tab, start, nb, dtp, lim, cd, stop, push);
     }
 }
 
@@ -112,10 +113,10 @@ hipError_t launch_face_flux_species(const BlockDev* tab, const FaceBatch& fb, in
 
 hipError_t launch_cell_update_species(const BlockDev* tab, const int64_t* start, int nblocks, int64_t total, int dims,
                                      int stage, const double* dtp, const CellLimits& lim, int nsp, const ChemDev* cd,
-                                     const unsigned* stop, hipStream_t s) {
+                                     const unsigned* stop, const GhostRec* push, hipStream_t s) {
     if (total <= 0) return hipSuccess;
-    if (nsp == 2) cell_species<2>(tab, start, nblocks, total, dims, stage, dtp, lim, cd, stop, s);
-    else if (nsp == 5) cell_species<5>(tab, start, nblocks, total, dims, stage, dtp, lim, cd, stop, s);
+    if (nsp == 2) cell_species<2>(tab, start, nblocks, total, dims, stage, dtp, lim, cd, stop, push, s);
+    else if (nsp == 5) cell_species<5>(tab, start, nblocks, total, dims, stage, dtp, lim, cd, stop, push, s);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }

@@ -317,7 +317,8 @@ __device__ __forceinline__ void store_species_state(double* fs, int64_t np, int6
 // the mass-fraction sum test of gas_state.d:226-268) of one cell.
 template <int DIM, int STAGE, int NSP>
 __device__ __forceinline__ void cell_update_species(const BlockDev& b, const ChemDev& cd, double dt, double low_T,
-                                                    double max_vel, double min_T, double max_T, int64_t t) {
+                                                    double max_vel, double min_T, double max_T, int64_t t,
+                                                    const GhostRec* push) {
     using C = CQ<DIM, NSP>;
     const int i = (int)(t % b.nic);
     const int64_t rest = t / b.nic;
@@ -325,6 +326,9 @@ __device__ __forceinline__ void cell_update_species(const BlockDev& b, const Che
     const int k = (int)(rest / b.njc);
     const int64_t c = pidx(b, i, j, k);
     const int64_t np = b.npad;
+    if (DIM == 3) push = nullptr;
+    const int head = push ? ghost_head(b, i, j, (unsigned)c) : -1;
+    constexpr int NFS = FS_BASE_PLANES + 2 * NSP;
     constexpr int nfaces = (DIM == 3) ? 6 : 4;
     int64_t fidx[6];
     int fdir[6];
@@ -366,12 +370,27 @@ __device__ __forceinline__ void cell_update_species(const BlockDev& b, const Che
     bool reenc;
     if (decode_species<DIM, NSP>(cd, U, low_T, rho, vel, u, p, T, a, massf, rho_s, reenc)) {
         atomicAdd(&b.counters[0], 1);
+        if (push) {  // the ghosts copy what the cell keeps
+            double v[NFS];
+#pragma unroll
+            for (int f = 0; f < NFS; ++f) v[f] = b.fs_out[c + f * np];
+            push_ghosts<NFS>(push, head, v);
+        }
         return;
     }
     if (STAGE == 2)
 #pragma unroll
         for (int jq = 0; jq < C::n; ++jq) b.Unew[c + jq * np] = U[jq];
     store_species_state<NSP>(b.fs_out, np, c, rho, vel, u, p, T, a, massf, rho_s);
+    if (push && head >= 0) {
+        double v[NFS] = {rho, vel.x, vel.y, vel.z, u, p, T, a};
+#pragma unroll
+        for (int q = 0; q < NSP; ++q) {
+            v[FS_BASE_PLANES + q] = massf[q];
+            v[FS_BASE_PLANES + NSP + q] = rho_s[q];
+        }
+        push_ghosts<NFS>(push, head, v);
+    }
     bool ok = check_data(rho, p, T, a, vel, max_vel, min_T, max_T);
     double f_sum = 0.0;
 #pragma unroll

@@ -41,7 +41,7 @@ hipError_t launch_face_flux_batch(const BlockDev* tab, const FaceBatch& fb, int 
                                  int numerics, double eps, const IdealGasDev& gas, hipStream_t s);
 hipError_t launch_cell_update_batch(const BlockDev* tab, const int64_t* start, int nblocks, int64_t total, int dims,
                                    int stage, const double* dtp, const CellLimits& lim, const IdealGasDev& gas,
-                                   const unsigned* stop, hipStream_t s);
+                                   const unsigned* stop, const GhostRec* push, hipStream_t s);
 // Multi-species thermally perfect gas (flux_species.hip), nsp = 2 or 5: the same batched
 // face and cell-update launches, and one block's encode/decode at start-up.
 struct ChemDev;
@@ -52,7 +52,7 @@ hipError_t launch_face_flux_species_lmr(const BlockDev* tab, const FaceBatch& fb
                                        double eps, int nsp, const ChemDev* cd, int64_t total, hipStream_t s);
 hipError_t launch_cell_update_species(const BlockDev* tab, const int64_t* start, int nblocks, int64_t total, int dims,
                                      int stage, const double* dtp, const CellLimits& lim, int nsp, const ChemDev* cd,
-                                     const unsigned* stop, hipStream_t s);
+                                     const unsigned* stop, const GhostRec* push, hipStream_t s);
 hipError_t launch_encode_species(const BlockDev& b, double* U, hipStream_t s);
 hipError_t launch_decode_species(const BlockDev& b, const ChemDev* cd, double* U, double* fs, double low_T,
                                  hipStream_t s);
@@ -71,7 +71,7 @@ hipError_t launch_fill_f64(double* p, int64_t n, double v, hipStream_t s);
 // with rec null the exchange of the cell lengths; and the fill itself (exchange and the other
 // ghost-cell effects), with the shock indicators where shock is set.
 hipError_t launch_ghost_setup(const BlockDev* tab, const SideDev* sides, int nsides, int64_t total, GhostRec* rec,
-                              hipStream_t s);
+                              const GhostRec* link, hipStream_t s);
 hipError_t launch_ghost_fill(const GhostRec* rec, int64_t total, int nfs, int shock, hipStream_t s);
 // Shock detection over all blocks' interior cells (PJ detector, strict rule applied by
 // the adaptive flux kernels), launched like the cell update.

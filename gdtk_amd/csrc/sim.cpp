@@ -113,6 +113,15 @@ struct Sim {
     int nsides = 0;
     int64_t nghost = 0;
     DevArr<GhostRec> ghosts[2];  // per flow-state copy
+    DevArr<int> gheads;          // BlockDev::ghead of every block
+    // The ghost cells of the copy that the next step starts from hold what the cells they copy do,
+    // and the inflows' are set in both copies (queued_steps).
+    bool ghosts_ready = false;
+    // 2-D only: a step of 20000 cells takes 34.1 us instead of 36.8, of 99 000 cells 52.9 instead of
+    // 55.9, of 350 000 cells 99 instead of 103.  In 3-D nearly every wave has cells at a side, so
+    // all of them pay for the scattered stores: no gain up to 64^3 cells, 173 instead of 170 us
+    // for 97 x 75 x 63, 820 instead of 790 us for 128^3.
+    bool push_ghost_cells() const { return !use_fused() && cfg.dimensions == 2; }
     DevArr<int> tile_start;
     int total_tiles = 0, kchunk = 16, tile_x = 64, tiles_kc = -1, tiles_tx = -1;
     DevArr<unsigned> ctr;  // the stages' counters, then the control words of queued steps
@@ -366,12 +375,18 @@ struct Sim {
     void build_tabs() {
         const size_t nb = blocks.size();
         std::vector<BlockDev> h(8 * nb);
+        size_t ncells = 0;
+        for (auto& bp : blocks) ncells += (size_t)bp->dev.npad;
+        gheads.reserve(ncells);
+        ghosts_ready = false;
         for (int st = 1; st <= 2; ++st)
             for (int c = 0; c < 2; ++c)
                 for (int u = 0; u < 2; ++u)
-                    for (size_t q = 0; q < nb; ++q) {
+                    for (size_t q = 0, off = 0; q < nb; ++q) {
                         Block& b = *blocks[q];
                         BlockDev d = b.dev;
+                        d.ghead = gheads.p + off;
+                        off += (size_t)d.npad;
                         d.fs_in = b.fs[c].p;
                         d.fs_out = b.fs[1 - c].p;
                         d.U0 = b.U[u].p;
@@ -383,9 +398,11 @@ struct Sim {
         tabs.alloc(h.size());
         HIPCHK(hipMemcpy(tabs.p, h.data(), h.size() * sizeof(BlockDev), hipMemcpyHostToDevice));
         // The ghost records of each copy (inflow rows are read from the block records).
+        HIPCHK(hipMemsetAsync(gheads.p, 0xff, ncells * sizeof(int), stream));
         for (int c = 0; c < 2; ++c) {
             ghosts[c].reserve((size_t)nghost);
-            HIPCHK(launch_ghost_setup(tab(1, c, 0), sides.p, nsides, nghost, ghosts[c].p, stream));
+            HIPCHK(launch_ghost_setup(tab(1, c, 0), sides.p, nsides, nghost, ghosts[c].p,
+                                      c == 0 ? nullptr : ghosts[0].p, stream));
         }
     }
 
@@ -475,7 +492,7 @@ struct Sim {
         build_tiles(kchunk, tile_x);
         // Geometry exchange: ghost cells of exchange sides take their source cells' lengths.
         if (any_exchange) {
-            HIPCHK(launch_ghost_setup(tab(1, 0, 0), sides.p, nsides, nghost, nullptr, stream));
+            HIPCHK(launch_ghost_setup(tab(1, 0, 0), sides.p, nsides, nghost, nullptr, nullptr, stream));
             HIPCHK(hipStreamSynchronize(stream));
         }
         finalized = true;
@@ -499,7 +516,15 @@ struct Sim {
     // Batched stage over all blocks: ghost cells (exchange + BCs), then the fused stage
     // kernel, or the face-per-thread kernels (one launch for the faces of every direction,
     // then the cell update); dt is read from dt_dev.  Counters of the stage must be clear.
-    void launch_batched_stage(int stage, int c, int u) {
+    //
+    // in_step (a stage of step_graph): where push_ghost_cells() says so the cell update writes the
+    // ghost cells of the copy it writes, and the stage that reads them has no fill of its own.
+    // Stage 1 of a step has one all the same where something changes the cells between the steps
+    // (the chemistry) or the fill does more (the shock indicators).
+    void launch_batched_stage(int stage, int c, int u, bool in_step = false) {
+        const bool pushes = in_step && push_ghost_cells();
+        const bool fill_first = chem_h >= 0 || adaptive();
+        const GhostRec* push = (pushes && (stage == 1 || !fill_first)) ? ghosts[1 - c].p : nullptr;
         const BlockDev* t = tab(stage, c, u);
         const double nc = (double)total_cells();
         const double eps = 1.0e-12;  // epsilon_van_albada, globalconfig.d:1079
@@ -515,8 +540,9 @@ struct Sim {
             fb.total[d] = (d < nd) ? ftotal[d] : 0;
             if (d < nd) nfaces += nfaces_total(d);
         }
-        timed(3, (double)nghost,
-              [&] { return launch_ghost_fill(ghosts[c].p, nghost, nfs(), detect ? 1 : 0, stream); });
+        if (!pushes || (stage == 1 && fill_first))
+            timed(3, (double)nghost,
+                  [&] { return launch_ghost_fill(ghosts[c].p, nghost, nfs(), detect ? 1 : 0, stream); });
         if (detect)
             timed(4, nc, [&] {
                 return launch_shock_detect(t, fb, cstart.p, nb, ctotal, cfg.dimensions, sdet.compression_tolerance,
@@ -533,9 +559,9 @@ struct Sim {
             timed(1, nc, [&] {
                 if (nsp > 1)
                     return launch_cell_update_species(t, cstart.p, nb, ctotal, cfg.dimensions, stage, dt_dev.p, lim,
-                                                      nsp, tpg_dev.p, ctl(), stream);
+                                                      nsp, tpg_dev.p, ctl(), push, stream);
                 return launch_cell_update_batch(t, cstart.p, nb, ctotal, cfg.dimensions, stage, dt_dev.p, lim, gas,
-                                                ctl(), stream);
+                                                ctl(), push, stream);
             });
             return;
         }
@@ -599,8 +625,8 @@ struct Sim {
         try {
             HIPCHK(launch_step_control(ctr.p, step_control(), STEP_BEGIN, stream));
             launch_save(0);
-            launch_batched_stage(1, 0, u);
-            launch_batched_stage(2, 1, u);
+            launch_batched_stage(1, 0, u, true);
+            launch_batched_stage(2, 1, u, true);
             if (chem_h >= 0) HIPCHK(launch_step_control(ctr.p, step_control(), STEP_FLUX_DONE, stream));
         } catch (...) {
             profile = saved;
@@ -1218,6 +1244,7 @@ struct Sim {
     // U[0] again would not return the same state bit for bit: the flow state the step
     // started from is kept in fs_save instead and copied back.
     void restore_from_U0() {
+        ghosts_ready = false;
         if (nsp > 1) {
             for (auto& bp : blocks) {
                 Block& b = *bp;
@@ -1286,6 +1313,11 @@ struct Sim {
         int attempt = 1;  // of the step at the head of the queue
         while (true) {
             HIPCHK(launch_window_begin(ctl(), dt_dev.p, dt_global, stream));
+            if (push_ghost_cells() && !ghosts_ready) {
+                // afterwards the steps' own cell updates keep them (launch_batched_stage)
+                for (int c = 0; c < 2; ++c) HIPCHK(launch_ghost_fill(ghosts[c].p, nghost, nfs(), 0, stream));
+                ghosts_ready = true;
+            }
             int u = u0;
             for (int w = 0; w < n; ++w) {
                 HIPCHK(hipGraphLaunch(step_graph(u), stream));
@@ -1339,6 +1371,7 @@ struct Sim {
     // simcore_gasdynamic_step.d:906-1575 for the pc scheme, stage by stage with the host's checks
     // between them (profiling, captured steps switched off, or single stages run before).
     void gasdynamic_step() {
+        ghosts_ready = false;
         double t0 = time;
         finalize();
         ensure_save();
@@ -1397,6 +1430,7 @@ struct Sim {
     }
 
     int run(int max_steps, double max_time) {
+        ghosts_ready = false;  // whatever has been done to the cells since
         int taken = 0;
         while (true) {
             determine_time_step_size();
@@ -1571,6 +1605,7 @@ int gdtk_hip_sim_step_fixed_dt(int sim, double dt, double* state) {
     int rc = guarded([&] {
         sp = &get_sim(sim);
         sp->dt_global = dt;
+        sp->ghosts_ready = false;
         sp->one_step();
         sp->check_chem();
         return GDTK_OK;
