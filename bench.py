@@ -365,7 +365,7 @@ def bench_surrogate(ncells, steps, seed=2024, dt=1.0e-7, n_train=1 << 22, tols=(
                      "final_loss": [float(h[-1]) for h in info["loss"]]},
         "roofline": {"bound": "mfma", "achieved": pick["mfma_tflops"], "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": pick["mfma_tflops"] / BF16_PEAK_TFLOPS, "traffic": None,
-                     "kernel": "k_mlp_infer<256,3> x2 + features", "avg_launch_ms": pick["kernels"]["ms_network"],
+                     "kernel": "k_mlp_infer<256,3,8,1> x2 + features", "avg_launch_ms": pick["kernels"]["ms_network"],
                      "flops_per_cell": 2 * MLP_FLOPS_PER_CELL},
     }
 
@@ -932,7 +932,7 @@ def bench_coupled_headline(steps, warmup, spinup, with_cpu=True, log=None):
     chem_flops = per_att * chs["attempts_total"] + per_it * chs["iters_total"]
     chem_ach = chem_flops / max(chs["ms_integrate"] * 1e-3, 1e-12) / 1e12
     roof_chem = {"bound": "fp64", "achieved": chem_ach, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
-                 "frac": chem_ach / FP64_PEAK_TFLOPS, "traffic": None, "kernel": "k_chem_integrate<5,5,0,false,true>",
+                 "frac": chem_ach / FP64_PEAK_TFLOPS, "traffic": None, "kernel": "k_chem_integrate<5,5,0,false,2>",
                  "avg_launch_ms": chs["ms_integrate"], "flops_per_launch": chem_flops,
                  "note": "latency bound: at a 2 ns flow step most cells take one substep and the launch lasts as "
                          "long as the slowest cell's serial attempts (VALU 14 % busy)"}
