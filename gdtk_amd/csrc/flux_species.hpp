@@ -24,31 +24,32 @@ struct SpeciesCell {
     double rho_s[NSP];
 };
 
+// fs: the planes from the wave's origin on (ld_plane), as in the functions below.
 template <int NSP>
-__device__ __forceinline__ SpeciesCell<NSP> load_species_cell(const double* fs, int64_t np, int64_t c) {
+__device__ __forceinline__ SpeciesCell<NSP> load_species_cell(const double* fs, int64_t np, unsigned c) {
     SpeciesCell<NSP> s;
-    s.u = fs[c + FS_U * np];
-    s.vel.x = fs[c + FS_VX * np];
-    s.vel.y = fs[c + FS_VY * np];
-    s.vel.z = fs[c + FS_VZ * np];
+    s.u = ld_plane(fs + FS_U * np, c);
+    s.vel.x = ld_plane(fs + FS_VX * np, c);
+    s.vel.y = ld_plane(fs + FS_VY * np, c);
+    s.vel.z = ld_plane(fs + FS_VZ * np, c);
 #pragma unroll
-    for (int i = 0; i < NSP; ++i) s.rho_s[i] = fs[c + (FS_BASE_PLANES + NSP + i) * np];
+    for (int i = 0; i < NSP; ++i) s.rho_s[i] = ld_plane(fs + (FS_BASE_PLANES + NSP + i) * np, c);
     return s;
 }
 
 // The whole flow state of a cell as a face state (the reference's Lft.copy_values_from of
 // the cell after a failed EOS call, onedinterp.d:45-55); velocity given separately.
 template <int NSP>
-__device__ __forceinline__ void copy_cell_state(const double* fs, int64_t np, int64_t c, Vec3d vel_local,
+__device__ __forceinline__ void copy_cell_state(const double* fs, int64_t np, unsigned c, Vec3d vel_local,
                                                 FaceStateT<NSP>& s) {
-    s.rho = fs[c + FS_RHO * np];
-    s.u = fs[c + FS_U * np];
-    s.p = fs[c + FS_P * np];
-    s.T = fs[c + FS_T * np];
-    s.a = fs[c + FS_A * np];
+    s.rho = ld_plane(fs + FS_RHO * np, c);
+    s.u = ld_plane(fs + FS_U * np, c);
+    s.p = ld_plane(fs + FS_P * np, c);
+    s.T = ld_plane(fs + FS_T * np, c);
+    s.a = ld_plane(fs + FS_A * np, c);
     s.vel = vel_local;
 #pragma unroll
-    for (int i = 0; i < NSP; ++i) s.massf[i] = fs[c + (FS_BASE_PLANES + i) * np];
+    for (int i = 0; i < NSP; ++i) s.massf[i] = ld_plane(fs + (FS_BASE_PLANES + i) * np, c);
 }
 
 // gas_model.d:373-407 with tolerance 0 and assert_error_tolerance 0.1 (the call of
@@ -64,8 +65,9 @@ __device__ __forceinline__ bool scale_mass_fractions(double* massf) {
     }
     if (fabs(s - 1.0) > 0.1) return false;
     if (fabs(s - 1.0) > 0.0) {
+        const double r = quick_rcp(s);
 #pragma unroll
-        for (int i = 0; i < NSP; ++i) massf[i] /= s;
+        for (int i = 0; i < NSP; ++i) massf[i] = div_by(massf[i], s, r);
     }
     return true;
 }
@@ -99,101 +101,117 @@ __device__ __forceinline__ double pair_swap(double v) { return __shfl_xor(v, 1);
 // LMR: Eilmer 5's reconstruction (lmr/onedinterp.d:137-169, 268-286, 314-315): the mass
 // fractions themselves are reconstructed and scaled, then the density, each with the
 // dimensionalised limiter epsilon; AUSMDV takes the smooth-maximum sound speed.
+//
+// Bound by its instructions (VALU 80 % busy) at the 3 waves a SIMD that its registers allow: as
+// two branches, one per side, the reconstruction of all variables ran twice for every wave;
+// mirrored (L2R2Side) both lanes run it once, and what the Newton iteration does not use waits in
+// LDS, without which the shorter code spilled 20 registers and gained nothing.  With scalar plane
+// addresses and shared reciprocals the launch over 8 blocks of 256 x 128 cells, 5 species, went
+// from 91 to 83 us, VALU instructions a wave from 1958 to ~1420.
 template <int DIM, int FC, int NSP, bool LMR = false>
 __device__ __forceinline__ bool face_flux_species_pair(const BlockDev& b, const ChemDev& cd, int d, double eps,
-                                                       int64_t f, int right) {
+                                                       unsigned f, int right, volatile double* frame,
+                                                       volatile double* own) {
     using C = CQ<DIM, NSP>;
-    const int fi = (int)(f % b.nf[d][0]);
-    const int64_t rest = f / b.nf[d][0];
-    const int fj = (int)(rest % b.nf[d][1]);
-    const int fk = (int)(rest / b.nf[d][1]);
-    const double* fs = b.fs_in;
+    unsigned fi, fj;
+    const unsigned rest = b.fdiv[d][0].divmod(f, fi);
+    const unsigned fk = b.fdiv[d][1].divmod(rest, fj);
     const int64_t np = b.npad;
-    const int pos = (d == 0) ? fi : (d == 1) ? fj : fk;
+    const int pos = (int)((d == 0) ? fi : (d == 1) ? fj : fk);
     const int nd = (d == 0) ? b.nic : (d == 1) ? b.njc : b.nkc;
-    auto at = [&](int s) -> int64_t {
-        if (d == 0) return pidx(b, s, fj, fk);
-        if (d == 1) return pidx(b, fi, s, fk);
-        return pidx(b, fi, fj, s);
-    };
-    const FaceGeom g = load_face(b.fgeom[d], b.nface[d], f);
-    double F[C::n];
-    int side = -1;
-    if (pos == 0) side = 2 * d;
-    else if (pos == nd) side = 2 * d + 1;
-    double* out = b.flux[d];
+    const unsigned stride = (d == 0) ? 1u : (d == 1) ? (unsigned)b.NI : (unsigned)(b.NI * b.NJ);
+    // the cell on the face's right, and the stencil around the face
+    const unsigned cabs =
+        (fi + NGHOST) + (unsigned)b.NI * ((fj + NGHOST) + (unsigned)b.NJ * (fk + (DIM == 3 ? NGHOST : 0)));
+    const unsigned oc = wave_origin(cabs - 2 * stride);
+    const unsigned cL1 = cabs - 2 * stride - oc, cL0 = cL1 + stride, cR0 = cL0 + stride, cR1 = cR0 + stride;
+    const double* fs = b.fs_in + oc;
     const int64_t nfc = b.nface[d];
+    const unsigned of = wave_origin(f);
+    f -= of;
+    const double* fg = b.fgeom[d] + of;
+    FaceGeom g;
+    g.n = Vec3d{ld_plane(fg, f), ld_plane(fg + nfc, f), ld_plane(fg + 2 * nfc, f)};
+    g.t1 = Vec3d{ld_plane(fg + 3 * nfc, f), ld_plane(fg + 4 * nfc, f), ld_plane(fg + 5 * nfc, f)};
+    g.t2 = Vec3d{ld_plane(fg + 6 * nfc, f), ld_plane(fg + 7 * nfc, f), ld_plane(fg + 8 * nfc, f)};
+    g.area = 0.0;  // not used by the flux
+    double F[C::n];
+    const int side = (pos == 0) ? 2 * d : (pos == nd) ? 2 * d + 1 : -1;
+    double* out = b.flux[d] + of;
     if (side >= 0 && b.bc_kind[side] == BC_OUTFLOW_SIMPLE_FLUX) {
         if (right) return true;
         const int outsign = (side % 2 == 0) ? -1 : 1;
-        const int64_t c = at(side % 2 == 0 ? 0 : nd - 1);
-        const Vec3d v{fs[c + FS_VX * np], fs[c + FS_VY * np], fs[c + FS_VZ * np]};
+        const unsigned c = (side % 2 == 0) ? cR0 : cL0;
+        const Vec3d v{ld_plane(fs + FS_VX * np, c), ld_plane(fs + FS_VY * np, c), ld_plane(fs + FS_VZ * np, c)};
         double mf[NSP];
 #pragma unroll
-        for (int i = 0; i < NSP; ++i) mf[i] = fs[c + (FS_BASE_PLANES + i) * np];
-        outflow_flux<DIM, NSP>(g, outsign, fs[c + FS_RHO * np], fs[c + FS_U * np], fs[c + FS_P * np], v, F, mf);
+        for (int i = 0; i < NSP; ++i) mf[i] = ld_plane(fs + (FS_BASE_PLANES + i) * np, c);
+        outflow_flux<DIM, NSP>(g, outsign, ld_plane(fs + FS_RHO * np, c), ld_plane(fs + FS_U * np, c),
+                               ld_plane(fs + FS_P * np, c), v, F, mf);
 #pragma unroll
-        for (int j = 0; j < C::n; ++j) out[f + j * nfc] = F[j];
+        for (int j = 0; j < C::n; ++j) st_plane(out + j * nfc, f, F[j]);
         return true;
     }
-    // This lane's three stencil cells: L1, L0, R0 (left) or L0, R0, R1 (right); c1 is the
-    // lane's own cell, the one the face state starts as a copy of (onedinterp.d:127-128).
-    const int64_t cL0 = at(pos - 1), cR0 = at(pos);
-    const int64_t c0 = right ? cL0 : at(pos - 2);
-    const int64_t c1 = right ? cR0 : cL0;
-    const int64_t c2 = right ? at(pos + 1) : cR0;
-    const double* len = b.len + d * np;
+    // This lane's three stencil cells, from the outside across the face: L1, L0, R0 (left) or
+    // R1, R0, L0 (right); c1 is the lane's own cell, the one the face state starts as a copy of
+    // (onedinterp.d:127-128).
+    const unsigned c0 = right ? cR1 : cL1, c1 = right ? cR0 : cL0, c2 = right ? cL0 : cR0;
+    const double* len = b.len + d * np + oc;
     const SpeciesCell<NSP> S0 = load_species_cell<NSP>(fs, np, c0), S1 = load_species_cell<NSP>(fs, np, c1),
                            S2 = load_species_cell<NSP>(fs, np, c2);
     const Vec3d v0 = to_local(S0.vel, g), v1 = to_local(S1.vel, g), v2 = to_local(S2.vel, g);
-    const double l0 = len[c0], l1 = len[c1], l2 = len[c2];
+    // What the Newton iteration does not use waits in LDS meanwhile (frame[128 e] of the pair's face,
+    // own[256 e] of the lane): in registers these 13 doubles are what spills at 3 waves a SIMD.
+    const double gv[9] = {g.n.x, g.n.y, g.n.z, g.t1.x, g.t1.y, g.t1.z, g.t2.x, g.t2.y, g.t2.z};
+#pragma unroll
+    for (int e = 0; e < 9; ++e) frame[128 * e] = gv[e];
+    L2R2Side c;
+    c.prepare(ld_plane(len, c0), ld_plane(len, c1), ld_plane(len, c2), right != 0);
     FaceStateT<NSP> st;
-    st.T = fs[c1 + FS_T * np];
-    st.a = fs[c1 + FS_A * np];
+    st.T = ld_plane(fs + FS_T * np, c1);
+    own[768] = ld_plane(fs + FS_A * np, c1);
     bool ok;
-    auto build = [&](const auto& c) {
-        st.vel.x = c.template value<LMR>(v0.x, v1.x, v2.x, eps);
-        st.vel.y = c.template value<LMR>(v0.y, v1.y, v2.y, eps);
-        st.vel.z = c.template value<LMR>(v0.z, v1.z, v2.z, eps);
-        if (LMR) {
+    own[0] = c.template value<LMR>(v0.x, v1.x, v2.x, eps);
+    own[256] = c.template value<LMR>(v0.y, v1.y, v2.y, eps);
+    own[512] = c.template value<LMR>(v0.z, v1.z, v2.z, eps);
+    if (LMR) {
 #pragma unroll
-            for (int i = 0; i < NSP; ++i) {
-                const int64_t pl = (FS_BASE_PLANES + i) * np;
-                st.massf[i] = c.template value<true>(fs[c0 + pl], fs[c1 + pl], fs[c2 + pl], eps);
-            }
-            ok = scale_mass_fractions<NSP>(st.massf);
-            st.rho = c.template value<true>(fs[c0 + FS_RHO * np], fs[c1 + FS_RHO * np], fs[c2 + FS_RHO * np], eps);
-        } else {
-            double rs[NSP];
-#pragma unroll
-            for (int i = 0; i < NSP; ++i) rs[i] = c.value(S0.rho_s[i], S1.rho_s[i], S2.rho_s[i], eps);
-            double rho = 0.0;
-#pragma unroll
-            for (int i = 0; i < NSP; ++i) rho += rs[i];
-            st.rho = rho;
-#pragma unroll
-            for (int i = 0; i < NSP; ++i) st.massf[i] = rs[i] / st.rho;
-            ok = scale_mass_fractions<NSP>(st.massf);
+        for (int i = 0; i < NSP; ++i) {
+            const double* pl = fs + (FS_BASE_PLANES + i) * np;
+            st.massf[i] = c.template value<true>(ld_plane(pl, c0), ld_plane(pl, c1), ld_plane(pl, c2), eps);
         }
-        st.u = c.template value<LMR>(S0.u, S1.u, S2.u, eps);
-    };
-    if (right) {
-        L2R2Side<true> c;
-        c.prepare(0.0, l0, l1, l2);
-        build(c);
+        ok = scale_mass_fractions<NSP>(st.massf);
+        const double* pl = fs + FS_RHO * np;
+        st.rho = c.template value<true>(ld_plane(pl, c0), ld_plane(pl, c1), ld_plane(pl, c2), eps);
     } else {
-        L2R2Side<false> c;
-        c.prepare(l0, l1, l2, 0.0);
-        build(c);
+        double rs[NSP];
+#pragma unroll
+        for (int i = 0; i < NSP; ++i) rs[i] = c.value(S0.rho_s[i], S1.rho_s[i], S2.rho_s[i], eps);
+        double rho = 0.0;
+#pragma unroll
+        for (int i = 0; i < NSP; ++i) rho += rs[i];
+        st.rho = rho;
+        const double r = quick_rcp(rho);
+#pragma unroll
+        for (int i = 0; i < NSP; ++i) st.massf[i] = div_by(rs[i], rho, r);
+        ok = scale_mass_fractions<NSP>(st.massf);
     }
+    st.u = c.template value<LMR>(S0.u, S1.u, S2.u, eps);
     TpgMix mix;
-    if (!tpg_update_rhou<NSP>(cd, st, mix)) {
-        copy_cell_state<NSP>(fs, np, c1, v1, st);
+    const bool solved = tpg_update_rhou<NSP>(cd, st, mix);
+    g.n = Vec3d{frame[0], frame[128], frame[256]};
+    g.t1 = Vec3d{frame[384], frame[512], frame[640]};
+    g.t2 = Vec3d{frame[768], frame[896], frame[1024]};
+    st.vel = Vec3d{own[0], own[256], own[512]};
+    st.a = own[768];
+    if (!solved) {
+        const Vec3d v{ld_plane(fs + FS_VX * np, c1), ld_plane(fs + FS_VY * np, c1), ld_plane(fs + FS_VZ * np, c1)};
+        copy_cell_state<NSP>(fs, np, c1, to_local(v, g), st);
         mix.clear();  // another composition
     }
     st.vel = to_local(to_global(st.vel, g), g);
     // EFM's specific heats, each at its own side.
-    const bool shocked = flux_is_adaptive(FC) && ((b.shock[cL0] | b.shock[cR0]) != 0);
+    const bool shocked = flux_is_adaptive(FC) && ((b.shock[oc + cL0] | b.shock[oc + cR0]) != 0);
     const bool efm = FC == 1 || (FC == 2 && shocked);
     const double Cv = efm ? tpg_Cv<NSP>(cd, st.massf, st.T, mix) : 0.0;
     // swap the two sides' states
@@ -224,7 +242,7 @@ __device__ __forceinline__ bool face_flux_species_pair(const BlockDev& b, const 
     if (DIM == 3) F[C::zMom] = m.z;
 #pragma unroll
     for (int j = 0; j < C::n; ++j)
-        if ((j & 1) == right) out[f + j * nfc] = F[j];
+        if ((j & 1) == right) st_plane(out + j * nfc, f, F[j]);
     return right ? true : (ok && ok_o);
 }
 
@@ -407,6 +425,7 @@ template <int DIM, int FC, int NSP, bool LMR>
 __global__ __launch_bounds__(256, 3) void k_face_flux_species_pair(const BlockDev* __restrict__ tab, FaceBatch fb,
                                                                 int nblocks, double eps,
                                                                 const ChemDev* __restrict__ cdp) {
+    __shared__ double frames[9 * 128], owns[4 * 256];
     int64_t w0 = (int64_t)blockIdx.x * (blockDim.x / 2);
     const int d = __builtin_amdgcn_readfirstlane(face_batch_dir(fb, w0));
     const int64_t* __restrict__ start = fb.start[d];
@@ -420,7 +439,8 @@ __global__ __launch_bounds__(256, 3) void k_face_flux_species_pair(const BlockDe
     const BlockDev& b = tab[q];
     const int64_t f = w0 - start[q] + (threadIdx.x >> 1);
     if (f >= b.nface[d]) return;
-    if (!face_flux_species_pair<DIM, FC, NSP, LMR>(b, *cdp, d, eps, f, (int)(threadIdx.x & 1)))
+    if (!face_flux_species_pair<DIM, FC, NSP, LMR>(b, *cdp, d, eps, (unsigned)f, (int)(threadIdx.x & 1),
+                                                       frames + (threadIdx.x >> 1), owns + threadIdx.x))
         atomicAdd(&b.counters[0], 1);
 }
 

@@ -108,52 +108,38 @@ struct L2R2 {
     }
 };
 
-// One side of the l2r2 reconstruction: the coefficients and operations of L2R2::prepare and
-// L2R2::scalar that the left value (from L1, L0, R0) or the right value (from L0, R0, R1)
-// needs, in the same order, so that each side equals scalar()'s bit for bit.
-template <bool RIGHT>
+// One side of the l2r2 reconstruction, the left value (from L1, L0, R0) or the right one (from
+// R1, R0, L0), from the cells outside, on and across the face from that side.  The right side
+// is the left one mirrored: both differences and with them the correction change sign, products
+// and squares of two of them do not, and the sums commute, so each side equals L2R2::scalar()'s
+// bit for bit and both run the same instructions; where the order of a sum or of the limits
+// matters, it is the reference's for the side.
 struct L2R2Side {
-    double a, len_other, tO, tD, two;  // left: aL0, lenR0, tL01, tR0L0, twoL0L1
-    __device__ __forceinline__ void prepare(double lenL1, double lL0, double lR0, double lenR1) {
-        if (!RIGHT) {
-            len_other = lR0;
-            a = quick_div(0.5 * lL0, lenL1 + 2.0 * lL0 + lR0);
-            tO = quick_div(2.0, lL0 + lenL1);
-            tD = quick_div(2.0, lR0 + lL0);
-            two = (2.0 * lL0 + lenL1);
-        } else {
-            len_other = lL0;
-            a = quick_div(0.5 * lR0, lL0 + 2.0 * lR0 + lenR1);
-            tD = quick_div(2.0, lR0 + lL0);
-            tO = quick_div(2.0, lenR1 + lR0);
-            two = (2.0 * lR0 + lenR1);
-        }
+    double a, len_across, tO, tD, two;
+    bool right;
+    __device__ __forceinline__ void prepare(double outer, double own, double across, bool right_side) {
+        right = right_side;
+        len_across = across;
+        a = quick_div(0.5 * own, (right ? across : outer) + 2.0 * own + (right ? outer : across));
+        tO = quick_div(2.0, own + outer);
+        tD = quick_div(2.0, across + own);
+        two = (2.0 * own + outer);
     }
-    // left: value(qL1, qL0, qR0); right: value(qL0, qR0, qR1).  LMR: Eilmer 5's epsilon,
-    // eps_va scaled by max(1e-12, |qL0|, |qR0|) and by 2 / (lenR0 + lenL0), as L2R2::scalar.
+    // LMR: Eilmer 5's epsilon, eps_va scaled by max(1e-12, |qL0|, |qR0|) and by
+    // 2 / (lenR0 + lenL0), as L2R2::scalar.
     template <bool LMR = false>
-    __device__ __forceinline__ double value(double q0, double q1, double q2, double eps_va) const {
+    __device__ __forceinline__ double value(double q_outer, double q_own, double q_across, double eps_va) const {
         const double beta = 1.0;
         double eps = eps_va;
         if (LMR) {
-            const double qL0 = RIGHT ? q0 : q1, qR0 = RIGHT ? q1 : q2;
-            const double qq = fmax(fmax(1e-12, fabs(qL0)), fmax(1e-12, fabs(qR0)));
+            const double qq = fmax(fmax(1e-12, fabs(q_own)), fmax(1e-12, fabs(q_across)));
             eps = qq * eps_va * tD;
         }
-        if (!RIGHT) {
-            const double delLminus = (q1 - q0) * tO;
-            const double del = (q2 - q1) * tD;
-            const double sL =
-                quick_div(delLminus * del + fabs(delLminus * del) + eps, delLminus * delLminus + del * del + eps);
-            const double qL = q1 + beta * sL * a * (del * two + delLminus * len_other);
-            return clip_to_limits(qL, q1, q2);
-        } else {
-            const double del = (q1 - q0) * tD;
-            const double delRplus = (q2 - q1) * tO;
-            const double sR = quick_div(del * delRplus + fabs(del * delRplus) + eps, del * del + delRplus * delRplus + eps);
-            const double qR = q1 - beta * sR * a * (delRplus * len_other + del * two);
-            return clip_to_limits(qR, q0, q1);
-        }
+        const double dO = (q_own - q_outer) * tO;
+        const double dA = (q_across - q_own) * tD;
+        const double s = quick_div(dO * dA + fabs(dO * dA) + eps, dO * dO + dA * dA + eps);
+        const double q = q_own + beta * s * a * (dA * two + dO * len_across);
+        return clip_to_limits(q, right ? q_across : q_own, right ? q_own : q_across);
     }
 };
 
