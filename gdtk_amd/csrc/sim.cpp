@@ -540,9 +540,10 @@ struct Sim {
             fb.total[d] = (d < nd) ? ftotal[d] : 0;
             if (d < nd) nfaces += nfaces_total(d);
         }
+        fb.stop = ctl();
         if (!pushes || (stage == 1 && fill_first))
             timed(3, (double)nghost,
-                  [&] { return launch_ghost_fill(ghosts[c].p, nghost, nfs(), detect ? 1 : 0, stream); });
+                  [&] { return launch_ghost_fill(ghosts[c].p, nghost, nfs(), detect ? 1 : 0, ctl(), stream); });
         if (detect)
             timed(4, nc, [&] {
                 return launch_shock_detect(t, fb, cstart.p, nb, ctotal, cfg.dimensions, sdet.compression_tolerance,
@@ -1315,7 +1316,7 @@ struct Sim {
             HIPCHK(launch_window_begin(ctl(), dt_dev.p, dt_global, stream));
             if (push_ghost_cells() && !ghosts_ready) {
                 // afterwards the steps' own cell updates keep them (launch_batched_stage)
-                for (int c = 0; c < 2; ++c) HIPCHK(launch_ghost_fill(ghosts[c].p, nghost, nfs(), 0, stream));
+                for (int c = 0; c < 2; ++c) HIPCHK(launch_ghost_fill(ghosts[c].p, nghost, nfs(), 0, ctl(), stream));
                 ghosts_ready = true;
             }
             int u = u0;
