@@ -1299,6 +1299,10 @@ struct Sim {
     // U[0].  A failed stage 1 makes stage 2's results irrelevant, so one look at both stages'
     // counters decides as the stage-by-stage checks would.  Returns the steps taken; time,
     // step and the U parity follow them.
+    // A call that is refused while the queue is filled (a reactor that has been closed, no memory
+    // for its work arrays) ends the queue there: what was queued before it is waited for and
+    // counted, the step without its chemistry in time and U alone, as the step by step path leaves
+    // it, and then the refusal is reported.
     // With one wait per 10 steps a step of the 2-D tube of 200 x 100 cells takes 43 us instead of
     // 66, one of the nitrogen cylinder 161 us instead of 188.
     int queued_steps(int want) {
@@ -1319,14 +1323,21 @@ struct Sim {
                 for (int c = 0; c < 2; ++c) HIPCHK(launch_ghost_fill(ghosts[c].p, nghost, nfs(), 0, ctl(), stream));
                 ghosts_ready = true;
             }
-            int u = u0;
-            for (int w = 0; w < n; ++w) {
-                HIPCHK(hipGraphLaunch(step_graph(u), stream));
-                u = 1 - u;  // swap(U[0], U[end]) (simcore_gasdynamic_step.d:1557-1562)
-                if (!chem) continue;
-                HIPCHK(hipEventRecord(qev[2 * w], stream));
-                launch_chemistry(0, u, dt_global);
-                HIPCHK(hipEventRecord(qev[2 * w + 1], stream));
+            int u = u0, whole = 0;  // steps queued with their chemistry
+            std::exception_ptr refused;
+            try {
+                for (int w = 0; w < n; ++w) {
+                    HIPCHK(hipGraphLaunch(step_graph(u), stream));
+                    u = 1 - u;  // swap(U[0], U[end]) (simcore_gasdynamic_step.d:1557-1562)
+                    if (chem) {
+                        HIPCHK(hipEventRecord(qev[2 * w], stream));
+                        launch_chemistry(0, u, dt_global);
+                        HIPCHK(hipEventRecord(qev[2 * w + 1], stream));
+                    }
+                    ++whole;
+                }
+            } catch (...) {
+                refused = std::current_exception();
             }
             HIPCHK(launch_step_control(ctr.p, step_control(), STEP_END, stream));
             int nf[3], ni[3];
@@ -1340,9 +1351,10 @@ struct Sim {
             for (int w = 0; w < done + (flux_ok ? 1 : 0); ++w) {
                 u0 = 1 - u0;
                 time += dt_global;
+                attempts_last = (w == 0) ? attempt : 1;
+                if (w >= whole) break;
                 step += 1;
                 ++taken;
-                attempts_last = (w == 0) ? attempt : 1;
                 if (!chem) continue;
                 float ms = 0.0f;
                 HIPCHK(hipEventElapsedTime(&ms, qev[2 * w], qev[2 * w + 1]));
@@ -1350,6 +1362,7 @@ struct Sim {
                 ++chem_calls;
             }
             for (auto& bp : blocks) refresh_dev(*bp);
+            if (!stopped && refused) std::rethrow_exception(refused);
             if (!stopped) return taken;
             if (flux_ok) throw Error(GDTK_ERR_STEP_FAILED, "The thermochemical_increment() failed.");
             if (done > 0) attempt = 1;

@@ -61,3 +61,48 @@ def test_failed_chemistry_with_steps_behind_it(numerics, steps):
     N2 = alone.get(0, 300)
     assert N2[3] < 1.0e-4 and abs(N2[2] - 0.5) < 1.0e-6  # the contrast is there
     _same(alone, queued, 1)
+
+
+def _cylinder(queue, cfl):
+    from gdtk_amd import Simulation
+    blocks, rec, _ = cases.cylinder_blocks(24, 10, 2)
+    s = Simulation(2, tpg=rec, dt_init=1e-9, dt_max=1e-6, cfl_count=40, max_attempts_for_step=5)
+    for b in blocks:
+        s.add_block(b)
+    s.set_graph(queue)
+    s.set_chemistry(_air_chemistry(rec))
+    s.run(7)
+    s.set_dt(cfl * min(s.block_dt(q, 1.0, 1.0, False)[0] for q in range(2)), s.state()["step"])
+    return s, rec
+
+
+def _air_chemistry(rec):
+    from gdtk_amd.chem import Chemistry, mech_record
+    return Chemistry(rec, mech_record(gdata.load("park-air-5sp-1T")))
+
+
+@pytest.mark.parametrize("cfl", [0.4, 100.0])
+def test_reactor_refused_inside_a_queue(cfl):
+    """The reactor is closed and the run goes on: the step's flux update is taken (after repeats
+    at a smaller dt where the Courant number is too large), its chemistry refused.  Queued or
+    step by step, the simulation is left in the same state and goes on from it the same way
+    once it has a reactor again."""
+    sims = []
+    for queue in (True, False):
+        s, rec = _cylinder(queue, cfl)
+        before = s.state()
+        s._chem[0].close()
+        with pytest.raises(Exception, match="handle"):
+            s.run(12)
+        after = s.state()
+        assert after["step"] == before["step"] and after["time"] == before["time"] + after["dt"]
+        assert (after["attempts"] > 1) == (cfl > 1.0)
+        sims.append((s, rec))
+    _same(sims[0][0], sims[1][0], 2)
+    for s, rec in sims:
+        s.set_chemistry(_air_chemistry(rec))
+        s.set_dt(1.0e-9, s.state()["step"])
+        s.run(20)
+    _same(sims[0][0], sims[1][0], 2)
+    for q in range(2):
+        assert np.array_equal(sims[0][0].get(q, "dt_chem"), sims[1][0].get(q, "dt_chem"))
