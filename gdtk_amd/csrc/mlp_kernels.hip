@@ -136,7 +136,8 @@ __global__ __launch_bounds__(64 * WAVES, 4) void k_mlp_infer(const float* __rest
     constexpr int LOADS = FRAG_PER_STEP / (64 * WAVES);      // per thread
     static_assert(FRAG_PER_STEP % (64 * WAVES) == 0, "k-step fragments must split over the workgroup");
     __shared__ bf16x8 lds[2][FRAG_PER_STEP];
-    __shared__ float bias_s[NH * H + 16];
+    __shared__ alignas(16) float bias_s[NH * H + 16];
+    static_assert(__alignof__(bias_s) >= sizeof(f32x4), "read four biases at a time");
     for (int k = threadIdx.x; k < NH * H + n_out; k += 64 * WAVES) bias_s[k] = bias[k];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
