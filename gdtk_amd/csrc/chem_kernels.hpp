@@ -537,7 +537,10 @@ struct TpgL {
 };
 
 // Runs a phase's launcher with the rate code of the mechanism's walk: a structure of its own
-// code, the rows with the reaction bound 8 or 32, or the lists with the bound 32.
+// code, the rows with the reaction bound 8 or 32 (5 species: also 5, for the air reactions in
+// another order than the structure's; 3001 cells over 1e-7 s take 1.91-1.98 ms with the bound 5 and
+// 1.95-1.97 with 8, with RKF 3.57-3.58 and 3.80-3.88, 131072 cells the same with either), or the
+// lists with the bound 32.
 template <int NSP, class L>
 hipError_t chem_walk_run(L& l, const ChemCall& c) {
     if constexpr (NSP == MechShape<WALK_AIR5_PARK>::nsp) {
@@ -547,6 +550,9 @@ hipError_t chem_walk_run(L& l, const ChemCall& c) {
         if (c.walk == WALK_N2_PAIR) return l.template run<NSP, MechShape<WALK_N2_PAIR>::nr, WALK_N2_PAIR>();
     }
     if (c.walk == WALK_LIST) return l.template run<NSP, 32, WALK_LIST>();
+    if constexpr (NSP == 5) {
+        if (c.nr <= 5) return l.template run<NSP, 5, WALK_ROWS>();
+    }
     if (c.nr <= 8) return l.template run<NSP, 8, WALK_ROWS>();
     return l.template run<NSP, 32, WALK_ROWS>();
 }

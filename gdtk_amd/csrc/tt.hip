@@ -191,8 +191,10 @@ int gdtk_hip_tt_step_device(int tt, int n, const double* rho, const double* T, c
     hipLaunchKernelGGL((k_tt_step<5, NR, WK>), grid, dim3(TT_BLOCK), 0, s, t.dev, t.tdev, n, dt, rho, T, Tv, u, uv, p, \
                        massf, dt_chem, T_out, Tv_out, u_out, uv_out, p_out, massf_out, dt_chem_out, status, t.nsub.p, \
                        t.natt.p)
-            // the structure of the shipped mechanism, or the row walk (at most 8 reactions)
+            // the structure of the shipped mechanism, or the row walk (at most 8 reactions; its six
+            // in another order: 64 cells 12.0 ms with the bound 6, 12.7 with 8; 32768 15.3 and 15.8)
             if (t.host.walk == WALK_AIR5_GUPTA) GDTK_TT(MechShape<WALK_AIR5_GUPTA>::nr, WALK_AIR5_GUPTA);
+            else if (t.host.nr <= 6) GDTK_TT(6, WALK_ROWS);
             else GDTK_TT(8, WALK_ROWS);
 #undef GDTK_TT
             HIPCHK(hipGetLastError());
