@@ -40,6 +40,17 @@ struct DevArr {
         HIPCHK(hipMemset(p, 0, std::max<size_t>(count, 1) * sizeof(T)));
         HIPCHK(hipDeviceSynchronize());
     }
+    // Without the fill and its wait, for contents that are written next.
+    void alloc_raw(size_t count) {
+        free();
+        HIPCHK(hipMalloc(&p, std::max<size_t>(count, 1) * sizeof(T)));
+        n = count;
+    }
+    // `count` elements from the host; later calls of the same size keep the address.
+    void upload(const T* src, size_t count) {
+        if (count != n || !p) alloc_raw(count);
+        HIPCHK(hipMemcpy(p, src, count * sizeof(T), hipMemcpyHostToDevice));
+    }
     // Grows (never shrinks) to at least `count` elements; contents are not kept.
     void reserve(size_t count) {
         if (count > n || !p) alloc(count);

@@ -32,19 +32,7 @@ namespace gdtk {
 
 thread_local std::string g_last_error;
 
-struct DevBuf {
-    double* p = nullptr;
-    size_t n = 0;
-    void alloc(size_t count) {
-        n = count;
-        HIPCHK(hipMalloc(&p, std::max<size_t>(count, 1) * sizeof(double)));
-        HIPCHK(hipMemset(p, 0, std::max<size_t>(count, 1) * sizeof(double)));
-        HIPCHK(hipDeviceSynchronize());  // the fill is on the null stream
-    }
-    ~DevBuf() {
-        if (p) (void)hipFree(p);
-    }
-};
+using DevBuf = DevArr<double>;
 
 struct Block {
     int id;
@@ -112,7 +100,8 @@ struct Sim {
     DevArr<SideDev> sides;
     int nsides = 0;
     int64_t nghost = 0;
-    DevArr<GhostRec> ghosts[2];  // per flow-state copy
+    DevArr<GhostRec> ghost_recs;
+    GhostRec* ghosts[2] = {nullptr, nullptr};  // per flow-state copy
     DevArr<int> gheads;          // BlockDev::ghead of every block
     // The ghost cells of the copy that the next step starts from hold what the cells they copy do,
     // and the inflows' are set in both copies (queued_steps).
@@ -126,7 +115,7 @@ struct Sim {
     int total_tiles = 0, kchunk = 16, tile_x = 64, tiles_kc = -1, tiles_tx = -1;
     DevArr<unsigned> ctr;  // the stages' counters, then the control words of queued steps
     StageCounters sc;
-    unsigned* ctr_host = nullptr;  // pinned copy of ctr
+    unsigned* ctr_host = nullptr;  // pinned copy of ctr, behind dt_host
     // Interior cells of a plane on their way to the host: two pinned buffers of at most PACK_CELLS
     // (4 MiB) each, which the packing kernel and the copy to the caller take in turn.
     static constexpr int64_t PACK_CELLS = (int64_t)1 << 19;
@@ -147,7 +136,8 @@ struct Sim {
     std::vector<int64_t> cstart_h;
     int64_t ftotal[3] = {0, 0, 0}, ctotal = 0;
     // Block time-step estimates: one partial per workgroup of the cell launch, each block's
-    // last signal, and the per-block results {dt, cfl, last signal}.
+    // last signal, and the per-block results {dt, cfl, last signal}; behind them the frames of
+    // find_axis_frames.
     DevArr<double> dt_part, dt_last, dt_out;
     double* dt_host = nullptr;  // pinned copy of dt_out
     // Step-start copy of every block's flow state (multi-species gas): segments per
@@ -195,7 +185,6 @@ struct Sim {
         if (cev0) (void)hipEventDestroy(cev0);
         if (cev1) (void)hipEventDestroy(cev1);
         if (cfail_host) (void)hipHostFree(cfail_host);
-        if (ctr_host) (void)hipHostFree(ctr_host);
         if (pack_host) (void)hipHostFree(pack_host);
         if (dt_host) (void)hipHostFree(dt_host);
         for (auto& e : qev)
@@ -281,38 +270,35 @@ struct Sim {
             if (d < nd)
                 for (size_t q = 0; q < nb; ++q) st[q + 1] = st[q] + aligned(blocks[q]->dev.nface[d]);
             ftotal[d] = st[nb];
-            fstart[d].alloc(st.size());
-            HIPCHK(hipMemcpy(fstart[d].p, st.data(), st.size() * sizeof(int64_t), hipMemcpyHostToDevice));
+            fstart[d].upload(st.data(), st.size());
         }
         std::vector<int64_t> st(nb + 1, 0);
         for (size_t q = 0; q < nb; ++q) st[q + 1] = st[q] + aligned(blocks[q]->ncell());
         ctotal = st[nb];
-        cstart.alloc(st.size());
-        HIPCHK(hipMemcpy(cstart.p, st.data(), st.size() * sizeof(int64_t), hipMemcpyHostToDevice));
+        cstart.upload(st.data(), st.size());
         cstart_h = st;
         dt_part.alloc(2 * (size_t)(ctotal / 256));
         dt_last.alloc(nb);
-        dt_out.alloc(3 * nb);
-        HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&dt_host), 3 * nb * sizeof(double)));
+        dt_out.alloc(33 * nb);
     }
 
     // Face-flux arrays of the face-per-thread kernels, allocated the first time they run.
+    bool flux_ready = false;
     void ensure_flux_all() {
-        bool grew = false;
+        if (flux_ready) return;
         for (auto& bp : blocks) {
             Block& b = *bp;
             const int nd = (b.dims == 3) ? 3 : 2;
             for (int q = 0; q < nd; ++q)
                 if (!b.flux[q].p) {
-                    b.flux[q].alloc((size_t)b.dev.nface[q] * b.ncq);
+                    b.flux[q].alloc_raw((size_t)b.dev.nface[q] * b.ncq);  // every face is written first
                     b.dev.flux[q] = b.flux[q].p;
-                    grew = true;
                 }
         }
-        if (grew) {
-            build_tabs();
-            drop_graphs();
-        }
+        find_axis_frames();
+        build_tabs();
+        drop_graphs();
+        flux_ready = true;
     }
 
     static int tab_index(int stage, int c, int u) { return ((stage - 1) * 2 + c) * 2 + u; }
@@ -359,8 +345,7 @@ struct Sim {
             ts[q + 1] = (int)t;
         }
         total_tiles = ts.back();
-        tile_start.alloc(ts.size());
-        HIPCHK(hipMemcpy(tile_start.p, ts.data(), ts.size() * sizeof(int), hipMemcpyHostToDevice));
+        tile_start.upload(ts.data(), ts.size());
         tiles_kc = kc;
         tiles_tx = tx;
         grid = fused_batch_grid(cfg.dimensions, cfg.flux_calculator, tx);
@@ -375,10 +360,6 @@ struct Sim {
     void build_tabs() {
         const size_t nb = blocks.size();
         std::vector<BlockDev> h(8 * nb);
-        size_t ncells = 0;
-        for (auto& bp : blocks) ncells += (size_t)bp->dev.npad;
-        gheads.reserve(ncells);
-        ghosts_ready = false;
         for (int st = 1; st <= 2; ++st)
             for (int c = 0; c < 2; ++c)
                 for (int u = 0; u < 2; ++u)
@@ -395,18 +376,23 @@ struct Sim {
                         d.counters = reinterpret_cast<int*>(ctr.p + sc.cells(st, (int)q));
                         h[(size_t)tab_index(st, c, u) * nb + q] = d;
                     }
-        tabs.alloc(h.size());
-        HIPCHK(hipMemcpy(tabs.p, h.data(), h.size() * sizeof(BlockDev), hipMemcpyHostToDevice));
-        // The ghost records of each copy (inflow rows are read from the block records).
-        HIPCHK(hipMemsetAsync(gheads.p, 0xff, ncells * sizeof(int), stream));
+        tabs.upload(h.data(), h.size());
+    }
+
+    // The ghost records of each copy, once: the block records that they read inflow rows from stay
+    // where they are (build_tabs).
+    void build_ghosts() {
+        HIPCHK(hipMemsetAsync(gheads.p, 0xff, gheads.n * sizeof(int), stream));
+        ghost_recs.alloc_raw(2 * (size_t)nghost);
         for (int c = 0; c < 2; ++c) {
-            ghosts[c].reserve((size_t)nghost);
-            HIPCHK(launch_ghost_setup(tab(1, c, 0), sides.p, nsides, nghost, ghosts[c].p,
-                                      c == 0 ? nullptr : ghosts[0].p, stream));
+            ghosts[c] = ghost_recs.p + c * nghost;
+            HIPCHK(launch_ghost_setup(tab(1, c, 0), sides.p, nsides, nghost, ghosts[c], c == 0 ? nullptr : ghosts[0],
+                                      stream));
         }
     }
 
-    // The directions whose faces all have the same axis-aligned frame (BlockDev::axis).
+    // The directions whose faces all have the same axis-aligned frame (BlockDev::axis), for the
+    // face-per-thread kernels.
     void find_axis_frames() {
         const size_t nb = blocks.size();
         const int nd = (cfg.dimensions == 3) ? 3 : 2;
@@ -415,16 +401,15 @@ struct Sim {
             fb.start[d] = fstart[d].p;
             fb.total[d] = (d < nd) ? ftotal[d] : 0;
         }
-        DevArr<double> frames;  // per block and direction: 9 components, then whether any face differs
-        frames.alloc(nb * 30);
-        HIPCHK(launch_frame_check(tab(1, 0, 0), fb, (int)nb, frames.p, stream));
-        std::vector<double> h(nb * 30);
-        HIPCHK(hipMemcpyAsync(h.data(), frames.p, h.size() * sizeof(double), hipMemcpyDeviceToHost, stream));
+        // per block and direction: 9 components, then whether any face differs (zero until then)
+        double* frames = dt_out.p + 3 * nb;
+        double* h = dt_host + 3 * nb;
+        HIPCHK(launch_frame_check(tab(1, 0, 0), fb, (int)nb, frames, stream));
+        HIPCHK(hipMemcpyAsync(h, frames, nb * 30 * sizeof(double), hipMemcpyDeviceToHost, stream));
         HIPCHK(hipStreamSynchronize(stream));
-        bool any = false;
         for (size_t q = 0; q < nb; ++q)
             for (int d = 0; d < nd; ++d) {
-                const double* r = &h[(q * 3 + d) * 10];
+                const double* r = h + (q * 3 + d) * 10;
                 int ax[3], used = 0;
                 bool ok = r[9] == 0.0;
                 for (int l = 0; l < 3; ++l) {
@@ -441,9 +426,7 @@ struct Sim {
                 // in 2-D the third local direction is the third axis (its momentum is not kept)
                 if (!ok || used != 7 || (nd == 2 && (ax[2] & 3) != 2)) continue;
                 for (int l = 0; l < 3; ++l) blocks[q]->dev.axis[d][l] = ax[l];
-                any = true;
             }
-        if (any) build_tabs();
     }
 
     // Sets up the batched launches once every block exists (the reference does the same
@@ -479,16 +462,24 @@ struct Sim {
         }
         nsides = (int)hs.size();
         nghost = start;
-        sides.alloc(hs.size());
-        HIPCHK(hipMemcpy(sides.p, hs.data(), hs.size() * sizeof(SideDev), hipMemcpyHostToDevice));
+        sides.upload(hs.data(), hs.size());
         sc.nblocks = (int)blocks.size();
         ctr.alloc(ctr_words());
-        HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&ctr_host), ctr_words() * sizeof(unsigned)));
+        const size_t nd = 33 * blocks.size();
+        if (!dt_host)
+            HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&dt_host),
+                                 nd * sizeof(double) + ctr_words() * sizeof(unsigned)));
+        ctr_host = reinterpret_cast<unsigned*>(dt_host + nd);
         dt_dev.alloc(1);
-        for (auto& bp : blocks) refresh_dev(*bp);
+        size_t ncells = 0;
+        for (auto& bp : blocks) {
+            refresh_dev(*bp);
+            ncells += (size_t)bp->dev.npad;
+        }
+        gheads.alloc_raw(ncells);
         build_tabs();
+        build_ghosts();
         build_starts();
-        find_axis_frames();
         build_tiles(kchunk, tile_x);
         // Geometry exchange: ghost cells of exchange sides take their source cells' lengths.
         if (any_exchange) {
@@ -524,7 +515,7 @@ struct Sim {
     void launch_batched_stage(int stage, int c, int u, bool in_step = false) {
         const bool pushes = in_step && push_ghost_cells();
         const bool fill_first = chem_h >= 0 || adaptive();
-        const GhostRec* push = (pushes && (stage == 1 || !fill_first)) ? ghosts[1 - c].p : nullptr;
+        const GhostRec* push = (pushes && (stage == 1 || !fill_first)) ? ghosts[1 - c] : nullptr;
         const BlockDev* t = tab(stage, c, u);
         const double nc = (double)total_cells();
         const double eps = 1.0e-12;  // epsilon_van_albada, globalconfig.d:1079
@@ -543,7 +534,7 @@ struct Sim {
         fb.stop = ctl();
         if (!pushes || (stage == 1 && fill_first))
             timed(3, (double)nghost,
-                  [&] { return launch_ghost_fill(ghosts[c].p, nghost, nfs(), detect ? 1 : 0, ctl(), stream); });
+                  [&] { return launch_ghost_fill(ghosts[c], nghost, nfs(), detect ? 1 : 0, ctl(), stream); });
         if (detect)
             timed(4, nc, [&] {
                 return launch_shock_detect(t, fb, cstart.p, nb, ctotal, cfg.dimensions, sdet.compression_tolerance,
@@ -719,20 +710,15 @@ struct Sim {
                         setlen(pad(i, j, -1 - n), cidx(i, j, n));
                         setlen(pad(i, j, nkc + n), cidx(i, j, nkc - 1 - n));
                     }
-        b->pos.alloc(geo.pos.size());
-        HIPCHK(hipMemcpy(b->pos.p, geo.pos.data(), geo.pos.size() * sizeof(double), hipMemcpyHostToDevice));
-        b->len.alloc(3 * np);
-        b->vol.alloc(np);
-        HIPCHK(hipMemcpy(b->len.p, hlen.data(), hlen.size() * sizeof(double), hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(b->vol.p, hvol.data(), hvol.size() * sizeof(double), hipMemcpyHostToDevice));
+        b->pos.upload(geo.pos.data(), geo.pos.size());
+        b->len.upload(hlen.data(), hlen.size());
+        b->vol.upload(hvol.data(), hvol.size());
         int nd = (cfg.dimensions == 3) ? 3 : 2;
         for (int q = 0; q < 3; ++q) {
             for (int e = 0; e < 3; ++e) d.nf[q][e] = geo.nf[q][e];
             d.nface[q] = (q < nd) ? (int64_t)geo.nf[q][0] * geo.nf[q][1] * geo.nf[q][2] : 0;
             if (q < nd) {
-                b->fgeom[q].alloc(geo.face[q].size());
-                HIPCHK(hipMemcpy(b->fgeom[q].p, geo.face[q].data(), geo.face[q].size() * sizeof(double),
-                                 hipMemcpyHostToDevice));
+                b->fgeom[q].upload(geo.face[q].data(), geo.face[q].size());
             }
             for (int e = 0; e < 2; ++e) {
                 d.fdiv[q][e] = FastDiv::of((unsigned)std::max(d.nf[q][e], 1));
@@ -1320,7 +1306,7 @@ struct Sim {
             HIPCHK(launch_window_begin(ctl(), dt_dev.p, dt_global, stream));
             if (push_ghost_cells() && !ghosts_ready) {
                 // afterwards the steps' own cell updates keep them (launch_batched_stage)
-                for (int c = 0; c < 2; ++c) HIPCHK(launch_ghost_fill(ghosts[c].p, nghost, nfs(), 0, ctl(), stream));
+                for (int c = 0; c < 2; ++c) HIPCHK(launch_ghost_fill(ghosts[c], nghost, nfs(), 0, ctl(), stream));
                 ghosts_ready = true;
             }
             int u = u0, whole = 0;  // steps queued with their chemistry
