@@ -31,8 +31,8 @@ hipError_t launch_decode(const BlockDev& b, const IdealGasDev& gas, double* U, d
 // (FaceBatch), then the cell update (dt read from device memory; start[q] = first launch
 // index of block q, a multiple of 256; total = launch size).  numerics: 0 Eilmer 4, 1 Eilmer 5
 // (lmr) limiter smoothing and AUSMDV sound speed.
-// out[c - c0] = the plane's value in interior cell c (i fastest) of a block, c0 <= c < c0 + n; the
-// shock indicator where plane is null.
+// out[c - c0] = the plane's value in interior cell c (i fastest) of a block, c0 <= c < c0 + n; where
+// plane is null the shock indicators, a byte each.
 hipError_t launch_pack_plane(const BlockDev& b, const double* plane, int64_t c0, int64_t n, double* out, hipStream_t s);
 // Per block and direction (10 doubles each, 3 directions a block): the first face's frame, and a
 // flag (which must be 0 before) set where another face's differs.

@@ -952,7 +952,12 @@ struct Sim {
             HIPCHK(hipStreamSynchronize(stream));
             if (c0 + cells < ncell)
                 HIPCHK(launch_pack_plane(d, src, c0 + cells, count(c0 + cells), pack_host + (q ^ 1) * cells, stream));
-            std::memcpy(out + c0, pack_host + q * cells, (size_t)count(c0) * sizeof(double));
+            if (src) {
+                std::memcpy(out + c0, pack_host + q * cells, (size_t)count(c0) * sizeof(double));
+                continue;
+            }
+            const unsigned char* flag = reinterpret_cast<const unsigned char*>(pack_host + q * cells);
+            for (int64_t c = 0; c < count(c0); ++c) out[c0 + c] = flag[c];
         }
     }
 
