@@ -48,8 +48,8 @@ def test_gradients_over_block_edges(hidden, n_hidden, batch, n_in, n_out):
 def test_training_steps_are_adam_on_the_batch_gradients(bf16, n, batch):
     """train() gathers rows by index and adds the batch shares inside the update; the same
     steps from loss_grad() with Adam in float64 on the host.  One batch is the whole set in
-    some order, so the gradient does not depend on the shuffle; with more, the losses of the
-    epoch bound what a wrong gather would change."""
+    some order, so the gradient does not depend on the shuffle; with more, no entry moves
+    further than Adam's steps allow (test_epochs_are_adam_in_float64 follows their values)."""
     import torch
     from gdtk_amd.surrogate import Mlp
     X, Y = _data(n, 8, 5, seed=3)
@@ -75,3 +75,51 @@ def test_training_steps_are_adam_on_the_batch_gradients(bf16, n, batch):
     ref.set_params(net.get_params())
     assert np.array_equal(net.forward(X[:64]), ref.forward(X[:64]))
     assert np.array_equal(net.loss_grad(X, Y)[1], ref.loss_grad(X, Y)[1])
+
+
+def _adam(p, grad, steps, lr):
+    """Adam (Kingma & Ba 2015) in float64 with the gradient function grad(p) -> (loss, g)."""
+    m, v, losses = np.zeros_like(p), np.zeros_like(p), []
+    for t in range(1, steps + 1):
+        loss, g = grad(p)
+        losses.append(loss)
+        m = 0.9 * m + 0.1 * g
+        v = 0.999 * v + 0.001 * g * g
+        p = p - lr * (m / (1.0 - 0.9 ** t)) / (np.sqrt(v / (1.0 - 0.999 ** t)) + 1.0e-8)
+    return p, losses
+
+
+@pytest.mark.parametrize("hidden,n_hidden", [(64, 2), (256, 3)])
+@pytest.mark.parametrize("copies,n,batch,epochs", [(False, 48, 48, 6), (False, 1009, 1009, 3),
+                                                   (True, 200, 33, 1), (True, 2100, 1000, 3)])
+def test_epochs_are_adam_in_float64(hidden, n_hidden, copies, n, batch, epochs):
+    """Several updates in a row against the float64 oracle's gradients: every row the same, so
+    that all batches are alike whatever the shuffle (a gather past the rows, stale packed weights
+    or shares of another batch in any but the first update move the result), or the whole set as
+    the batch.  Gradients agree to 1e-4 of the largest entry (above), so where the first gradient
+    is more than 1e-2 of the largest an update, which depends on the ratios of an entry's gradients
+    alone, is off by at most 1e-2 lr.  Smaller entries may move by up to lr either way; the loss
+    depends on them by their gradient times that, and is held to 1e-4."""
+    import torch
+    from gdtk_amd.surrogate import Mlp
+    lr = 1.0e-3
+    X, Y = _data(n, 8, 5, seed=6)
+    if copies:
+        X[:], Y[:] = X[0], Y[0]
+    dev = torch.device("cuda:0")
+    xs, ys = (torch.tensor(np.ascontiguousarray(a.T), device=dev) for a in (X, Y))
+    torch.cuda.synchronize()
+    net = Mlp(8, 5, hidden=hidden, n_hidden=n_hidden, seed=11)
+    lay, _ = MO.layout(8, hidden, n_hidden, 5)
+    p0 = net.get_params().astype(np.float64)
+    hist = net.train(n, xs.data_ptr(), ys.data_ptr(), batch=batch, epochs=epochs, lr=lr, seed=4)
+    rows = 1 if copies else n
+    grad = lambda p: MO.loss_grad(p, lay, X[:rows].astype(np.float64), Y[:rows].astype(np.float64))  # noqa: E731
+    per = n // batch
+    want, losses = _adam(p0, grad, per * epochs, lr)
+    losses = np.array(losses).reshape(epochs, per)
+    # the history holds the losses read back: the last of an epoch and every 16th before it
+    assert np.max(np.abs(hist - losses[:, -1]) / losses[:, -1]) <= 1e-4
+    g0 = np.abs(grad(p0)[1])
+    err = np.abs(net.get_params() - want)
+    assert np.max(err[g0 > 1e-2 * g0.max()]) <= 1e-2 * lr * per * epochs
