@@ -61,7 +61,7 @@ struct Mlp {
 
     void ensure_batch(int B) {
         if (B <= bcap) return;
-        bcap = B;
+        bcap = 0;  // until every buffer has been allocated
         const size_t cells = (size_t)mlp_blocks(B) * 16;
         act.clear();
         dz.clear();
@@ -79,6 +79,7 @@ struct Mlp {
         yout.alloc((size_t)B * n_out);
         loss.alloc((size_t)mlp_blocks(B));
         gparts.alloc((size_t)mlp_grad_splits(q, nlayer, B) * nparam);
+        bcap = B;
     }
 
     // The batch's inputs at x[k xk + row xc] (rows idx[b], or b), targets likewise.
