@@ -16,8 +16,8 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libgdtkhip.so")
 ARCH = os.environ.get("GDTK_OFFLOAD_ARCH", "gfx950")
 
-# -ffp-contract=off keeps every expression in the written (reference) order, no FMA
-# contraction.  The packed-fp32 feature is turned off for all device code.
+# -ffp-contract=off: no FMA but those that are written.  The packed-fp32 feature is turned off
+# for all device code.
 HIP_FLAGS = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

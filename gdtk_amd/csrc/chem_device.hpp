@@ -4,8 +4,11 @@
 // device buffer; every lane of a wave reads the same entries, so those loads are uniform
 // (scalar).  Per-cell state is held in registers: arrays are sized by the template
 // parameters NSP (species, exact) and NRM (an upper bound on the reactions, the actual
-// count cd->nr is uniform at run time).  FP64 throughout, built without FMA contraction;
-// the operation order of every expression follows the reference function cited beside it.
+// count cd->nr is uniform at run time).  FP64 throughout, built without FMA contraction (an
+// fma is one that is written).  The formulas are those of the reference functions cited beside
+// them.  The curves of a species and the controller's decisions keep the reference's operation
+// order; the summed curves (TpgMix), the rate constants (arrhenius), the alpha-QSS step and every
+// quick_div are rearranged, as their comments say, and agree with it to rounding.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -71,7 +74,6 @@ struct RateRow {
 // How the rate code walks a mechanism (chosen on the host, mechanism_walk): its species lists,
 // the rows above, or code in which the structure of the mechanism is known at compile time.
 enum ChemWalk : int { WALK_LIST = 0, WALK_ROWS = 1, WALK_AIR5_PARK = 2, WALK_AIR5_GUPTA = 3, WALK_N2_PAIR = 4 };
-constexpr int NUM_WALKS = 5;
 
 // A species' code word in a row: its exponent as reactant and product, and whether it is in the
 // third-body list.

@@ -5,8 +5,9 @@
 // Flow-state planes of a block: rho, vx, vy, vz, u, p, T, a (FS_*), then massf[NSP] at
 // FS_BASE_PLANES + s and rho_s[NSP] at FS_BASE_PLANES + NSP + s.  Conserved quantities:
 // mass, momentum, total energy, then the species densities (CQ<DIM, NSP>).  The gas is the
-// gas part of a ChemDev table (species gas constants and CEA curves).  Every expression
-// keeps the reference's operation order (cited per function); FP64, no FMA contraction.
+// gas part of a ChemDev table (species gas constants and CEA curves).  The formulas are the
+// reference's (cited per function) in its order, but for quotients by quick_div (within an ulp)
+// and the temperature from the summed curve (TpgMix); FP64, no FMA contraction.
 #pragma once
 #include <hip/hip_runtime.h>
 

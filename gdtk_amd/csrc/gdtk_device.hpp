@@ -2,7 +2,8 @@
 //
 // Everything here is FP64 and is compiled with -ffp-contract=off so that the operation
 // order of each expression is the one written, which is the order of the D reference
-// (cited per function).  The functions are written against plain values so that the
+// (cited per function), but for quotients by quick_div or by a shared reciprocal, which are
+// within an ulp of the division.  The functions are written against plain values so that the
 // same code serves the face-per-thread kernels and the LDS-tiled fused stage kernel.
 #pragma once
 #include <hip/hip_runtime.h>

@@ -27,16 +27,16 @@ hipError_t launch_dt_batch(const BlockDev* tab, const int64_t* start, int nblock
 hipError_t launch_encode(const BlockDev& b, double* U, hipStream_t s);
 hipError_t launch_decode(const BlockDev& b, const IdealGasDev& gas, double* U, double* fs, double low_T,
                          hipStream_t s);
-// Face-per-thread kernels over all blocks: the faces of every direction in one launch
-// (FaceBatch), then the cell update (dt read from device memory; start[q] = first launch
-// index of block q, a multiple of 256; total = launch size).  numerics: 0 Eilmer 4, 1 Eilmer 5
-// (lmr) limiter smoothing and AUSMDV sound speed.
 // out[c - c0] = the plane's value in interior cell c (i fastest) of a block, c0 <= c < c0 + n; where
 // plane is null the shock indicators, a byte each.
 hipError_t launch_pack_plane(const BlockDev& b, const double* plane, int64_t c0, int64_t n, double* out, hipStream_t s);
 // Per block and direction (10 doubles each, 3 directions a block): the first face's frame, and a
 // flag (which must be 0 before) set where another face's differs.
 hipError_t launch_frame_check(const BlockDev* tab, const FaceBatch& fb, int nblocks, double* frames, hipStream_t s);
+// Face-per-thread kernels over all blocks: the faces of every direction in one launch
+// (FaceBatch), then the cell update (dt read from device memory; start[q] = first launch
+// index of block q, a multiple of 256; total = launch size).  numerics: 0 Eilmer 4, 1 Eilmer 5
+// (lmr) limiter smoothing and AUSMDV sound speed.
 hipError_t launch_face_flux_batch(const BlockDev* tab, const FaceBatch& fb, int nblocks, int dims, int flux_calc,
                                  int numerics, double eps, const IdealGasDev& gas, hipStream_t s);
 hipError_t launch_cell_update_batch(const BlockDev* tab, const int64_t* start, int nblocks, int64_t total, int dims,

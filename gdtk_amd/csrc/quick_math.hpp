@@ -18,9 +18,10 @@ __host__ __device__ inline double div_by(double a, double b, double y) {
 }
 
 // a / b for normal operands: the hardware reciprocal refined by one cubic step (residual e:
-// y (1 + e + e^2), relative error e^3), the quotient and one remainder correction.  7
-// instructions, where the compiler's division takes 11 to scale operands that none of the
-// quotients here needs scaled.
+// y (1 + e + e^2), relative error e^3), the quotient and one remainder correction: a / b within
+// an ulp (the reciprocal is not always the rounded one).  A divisor of zero or infinity gives a
+// NaN, where the division's result may be 0 or an infinity.  7 instructions, where the compiler's
+// division takes 11 to scale operands that none of the quotients here needs scaled.
 __device__ __forceinline__ double quick_rcp(double b) {
     const double y = __builtin_amdgcn_rcp(b);
     const double e = fma(-b, y, 1.0);

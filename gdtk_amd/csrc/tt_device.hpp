@@ -1,8 +1,10 @@
 // tt_device.hpp -- two-temperature air on gfx950: the TwoTemperatureAir gas
 // (src/gas/two_temperature_air.d, neutral species) and the TwoTemperatureAirKinetics reactor
-// (src/kinetics/two_temperature_air_kinetics.d), one lane per cell.  FP64, no FMA
-// contraction; every expression keeps the reference's operation order.  The mechanism is in
-// dense form (ascending lists, as prep-chem writes them), with explicit backward rates.
+// (src/kinetics/two_temperature_air_kinetics.d), one lane per cell.  FP64, no FMA contraction.
+// The formulas and the order of the steps are the reference's; within an expression sums over
+// the species are taken first and quotients by quick_div, so results agree with the reference's
+// operation order to rounding.  The mechanism is in dense form (ascending lists, as prep-chem
+// writes them), with explicit backward rates.
 #pragma once
 #include <hip/hip_runtime.h>
 
