@@ -171,9 +171,10 @@ __host__ __device__ inline int face_batch_dir(const FaceBatch& fb, int64_t& w0) 
 // of each step and behind the last one judges the step before it by its counters (the
 // reference's stage-by-stage checks, simcore_gasdynamic_step.d:946-1000, and the failed cells
 // of its chemistry; a flux update also before its chemistry) and counts it as finished or sets
-// stop; from then on every kernel of a step returns at once (the chemistry's own run over cells
-// that it leaves as they are), so the host finds the failed step's counters and starting state as
-// if it had waited for that step.
+// stop; from then on the kernels that write what a repeated step starts from (U, the saved flow
+// state, the shock indicators, dt_chem) or the counters leave them alone, so the host finds the
+// failed step's counters and starting state as if it had waited for that step.  What the others
+// write (fluxes, ghost cells, the faces' shock decisions) the repeated step writes anew.
 enum StepPoint : int {
     STEP_BEGIN,      // judge and count the step before, clear the counters
     STEP_FLUX_DONE,  // before the chemistry: judge the flux update

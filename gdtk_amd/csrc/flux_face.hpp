@@ -110,7 +110,6 @@ __device__ __forceinline__ void face_flux_one(const BlockDev& b, const IdealGasD
 template <int DIM, int FC, bool LMR>
 __global__ __launch_bounds__(256, 4) void k_face_flux_batch(const BlockDev* __restrict__ tab, FaceBatch fb,
                                                          int nblocks, double eps, IdealGasDev gas) {
-    if (*fb.stop) return;  // StepControl: the run waits for the host
     int64_t w0 = (int64_t)blockIdx.x * blockDim.x;
     const int d = __builtin_amdgcn_readfirstlane(face_batch_dir(fb, w0));
     const int64_t* __restrict__ start = fb.start[d];

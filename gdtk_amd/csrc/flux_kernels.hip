@@ -124,9 +124,7 @@ __global__ void k_ghost_setup(const BlockDev* __restrict__ tab, const SideDev* _
 // the state, all planes at once: 13.3 -> 4.5 us a launch over the 960 ghost cells of the nitrogen
 // cylinder (its step 211 -> 188 us), a 2-D tube of 200 x 100 cells 70 -> 66 us a step.
 template <int NFS>
-__global__ __launch_bounds__(64) void k_ghost_fill(const GhostRec* __restrict__ rec, int64_t total, int shock,
-                                                   const unsigned* __restrict__ stop) {
-    if (*stop) return;  // StepControl: the run waits for the host
+__global__ __launch_bounds__(64) void k_ghost_fill(const GhostRec* __restrict__ rec, int64_t total, int shock) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= total) return;
     const GhostRec r = rec[t];
@@ -180,7 +178,6 @@ template <int DIM>
 __global__ __launch_bounds__(256) void k_shock_faces_batch(const BlockDev* __restrict__ tab, FaceBatch fb,
                                                            int nblocks, double comp_tol, double shear_tol,
                                                            int damped_outflow) {
-    if (*fb.stop) return;  // StepControl: the run waits for the host
     int64_t w0 = (int64_t)blockIdx.x * blockDim.x;
     const int d = __builtin_amdgcn_readfirstlane(face_batch_dir(fb, w0));
     const int64_t* __restrict__ start = fb.start[d];
@@ -599,13 +596,12 @@ hipError_t launch_ghost_setup(const BlockDev* tab, const SideDev* sides, int nsi
     return hipGetLastError();
 }
 
-hipError_t launch_ghost_fill(const GhostRec* rec, int64_t total, int nfs, int shock, const unsigned* stop,
-                             hipStream_t s) {
+hipError_t launch_ghost_fill(const GhostRec* rec, int64_t total, int nfs, int shock, hipStream_t s) {
     if (total <= 0) return hipSuccess;
     const dim3 g(nblk(total, 64)), blk(64);
-    if (nfs == FS_BASE_PLANES) hipLaunchKernelGGL(k_ghost_fill<FS_BASE_PLANES>, g, blk, 0, s, rec, total, shock, stop);
-    else if (nfs == FS_BASE_PLANES + 4) hipLaunchKernelGGL(k_ghost_fill<FS_BASE_PLANES + 4>, g, blk, 0, s, rec, total, shock, stop);
-    else if (nfs == FS_BASE_PLANES + 10) hipLaunchKernelGGL(k_ghost_fill<FS_BASE_PLANES + 10>, g, blk, 0, s, rec, total, shock, stop);
+    if (nfs == FS_BASE_PLANES) hipLaunchKernelGGL(k_ghost_fill<FS_BASE_PLANES>, g, blk, 0, s, rec, total, shock);
+    else if (nfs == FS_BASE_PLANES + 4) hipLaunchKernelGGL(k_ghost_fill<FS_BASE_PLANES + 4>, g, blk, 0, s, rec, total, shock);
+    else if (nfs == FS_BASE_PLANES + 10) hipLaunchKernelGGL(k_ghost_fill<FS_BASE_PLANES + 10>, g, blk, 0, s, rec, total, shock);
     else return hipErrorInvalidValue;  // 1, 2 or 5 species
     return hipGetLastError();
 }

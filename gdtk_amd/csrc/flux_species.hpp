@@ -426,9 +426,6 @@ template <int DIM, int FC, int NSP, bool LMR>
 __global__ __launch_bounds__(256, 3) void k_face_flux_species_pair(const BlockDev* __restrict__ tab, FaceBatch fb,
                                                                 int nblocks, double eps,
                                                                 const ChemDev* __restrict__ cdp) {
-    // StepControl: the run waits for the host (and reads the counters, which a face whose mass
-    // fractions are far from summing to one would raise)
-    if (*fb.stop) return;
     __shared__ double frames[9 * 128], owns[4 * 256];
     int64_t w0 = (int64_t)blockIdx.x * (blockDim.x / 2);
     const int d = __builtin_amdgcn_readfirstlane(face_batch_dir(fb, w0));
@@ -444,7 +441,8 @@ __global__ __launch_bounds__(256, 3) void k_face_flux_species_pair(const BlockDe
     const int64_t f = w0 - start[q] + (threadIdx.x >> 1);
     if (f >= b.nface[d]) return;
     if (!face_flux_species_pair<DIM, FC, NSP, LMR>(b, *cdp, d, eps, (unsigned)f, (int)(threadIdx.x & 1),
-                                                       frames + (threadIdx.x >> 1), owns + threadIdx.x))
+                                                       frames + (threadIdx.x >> 1), owns + threadIdx.x) &&
+        !*fb.stop)  // StepControl: the counters are those of the step that failed
         atomicAdd(&b.counters[0], 1);
 }
 

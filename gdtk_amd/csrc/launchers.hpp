@@ -72,8 +72,7 @@ hipError_t launch_fill_f64(double* p, int64_t n, double v, hipStream_t s);
 // ghost-cell effects), with the shock indicators where shock is set.
 hipError_t launch_ghost_setup(const BlockDev* tab, const SideDev* sides, int nsides, int64_t total, GhostRec* rec,
                               const GhostRec* link, hipStream_t s);
-hipError_t launch_ghost_fill(const GhostRec* rec, int64_t total, int nfs, int shock, const unsigned* stop,
-                             hipStream_t s);
+hipError_t launch_ghost_fill(const GhostRec* rec, int64_t total, int nfs, int shock, hipStream_t s);
 // Shock detection over all blocks' interior cells (PJ detector, strict rule applied by
 // the adaptive flux kernels), launched like the cell update.
 hipError_t launch_shock_detect(const BlockDev* tab, const FaceBatch& fb, const int64_t* cstart, int nblocks,

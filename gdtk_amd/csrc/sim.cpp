@@ -534,7 +534,7 @@ struct Sim {
         fb.stop = ctl();
         if (!pushes || (stage == 1 && fill_first))
             timed(3, (double)nghost,
-                  [&] { return launch_ghost_fill(ghosts[c], nghost, nfs(), detect ? 1 : 0, ctl(), stream); });
+                  [&] { return launch_ghost_fill(ghosts[c], nghost, nfs(), detect ? 1 : 0, stream); });
         if (detect)
             timed(4, nc, [&] {
                 return launch_shock_detect(t, fb, cstart.p, nb, ctotal, cfg.dimensions, sdet.compression_tolerance,
@@ -1311,7 +1311,7 @@ struct Sim {
             HIPCHK(launch_window_begin(ctl(), dt_dev.p, dt_global, stream));
             if (push_ghost_cells() && !ghosts_ready) {
                 // afterwards the steps' own cell updates keep them (launch_batched_stage)
-                for (int c = 0; c < 2; ++c) HIPCHK(launch_ghost_fill(ghosts[c], nghost, nfs(), 0, ctl(), stream));
+                for (int c = 0; c < 2; ++c) HIPCHK(launch_ghost_fill(ghosts[c], nghost, nfs(), 0, stream));
                 ghosts_ready = true;
             }
             int u = u0, whole = 0;  // steps queued with their chemistry
