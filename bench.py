@@ -925,8 +925,8 @@ def bench_coupled_headline(steps, warmup, spinup, with_cpu=True, log=None):
                  "frac": face_ach / HBM_PEAK_GBS, "traffic": measured_traffic(kname, face["items_per_launch"]),
                  "kernel": kname, "avg_launch_ms": face_avg, "bytes_per_face": bpf,
                  "items_per_launch": face["items_per_launch"],
-                 "note": "bound by instruction issue, not HBM: per face two Newton T(u) solves and two "
-                         "reconstructions of 9 variables at 3 waves a SIMD"}
+                 "note": "bound by instruction issue and latency, not HBM: per face two Newton T(u) solves and "
+                         "two reconstructions of 9 variables at 3 waves a SIMD (VALU 50 % busy)"}
     per_att, per_it = alpha_qss_flops(mech, 5)
     chem_flops = per_att * chs["attempts_total"] + per_it * chs["iters_total"]
     chem_ach = chem_flops / max(chs["ms_integrate"] * 1e-3, 1e-12) / 1e12

@@ -13,11 +13,12 @@ namespace gdtk {
 // One thread per face of index direction d: reconstruction + flux calculator, or the
 // simple-outflow boundary flux effect on faces whose BC computes the flux itself.  The block
 // and the direction are the same for the whole workgroup, so every plane is a scalar base and
-// the lane's index a 32-bit offset from that of the wave's first lane.  The kernel is bound by
-// its instructions and by the latency of its loads (4 waves a SIMD at 128 registers): scalar
-// bases, divisions through the refined hardware reciprocal and index divisions by
-// multiplication took the launch over a 2-D tube of 200 x 100 cells from 7.0 to 5.2 us, over
-// 97 x 75 x 63 curvilinear cells (EFM) from 64 to 59 us.
+// the lane's index a 32-bit offset from that of the wave's first lane.  Small launches are bound
+// by their instructions and by the latency of their loads (4 waves a SIMD at 128 registers),
+// large ones by the bytes too (256 x 128 x 128 cells along the axes: 152 B a face beyond L2 at
+// 4.97 TB/s, a copy's rate, with the VALU 57 % busy): scalar bases, divisions through the refined
+// hardware reciprocal and index divisions by multiplication took the launch over a 2-D tube of
+// 200 x 100 cells from 7.0 to 5.2 us, over 97 x 75 x 63 curvilinear cells (EFM) from 64 to 59 us.
 //
 // AXIS: a direction whose faces all have the same axis-aligned frame.  The velocity components
 // are loaded, and the momentum fluxes stored, in the frame's order, and the nine planes of

@@ -103,12 +103,13 @@ __device__ __forceinline__ double pair_swap(double v) { return __shfl_xor(v, 1);
 // fractions themselves are reconstructed and scaled, then the density, each with the
 // dimensionalised limiter epsilon; AUSMDV takes the smooth-maximum sound speed.
 //
-// Bound by its instructions (VALU 80 % busy) at the 3 waves a SIMD that its registers allow: as
-// two branches, one per side, the reconstruction of all variables ran twice for every wave;
-// mirrored (L2R2Side) both lanes run it once, and what the Newton iteration does not use waits in
-// LDS, without which the shorter code spilled 20 registers and gained nothing.  With scalar plane
-// addresses and shared reciprocals the launch over 8 blocks of 256 x 128 cells, 5 species, went
-// from 91 to 83 us, VALU instructions a wave from 1958 to ~1420.
+// Bound by issue and latency (VALU 50 % busy, waves waiting a third of their time) at the 3 waves
+// a SIMD that its registers allow: as two branches, one per side, the reconstruction of all
+// variables ran twice for every wave; mirrored (L2R2Side) both lanes run it once, and what the
+// Newton iteration does not use waits in LDS, without which the shorter code spilled 20
+// registers and gained nothing (11 still do for 5 species: 44 of the 83 MB a launch writes).  With
+// scalar plane addresses and shared reciprocals the launch over 8 blocks of 256 x 128 cells, 5
+// species, went from 91 to 84 us, VALU instructions a wave from 1958 to 1623.
 template <int DIM, int FC, int NSP, bool LMR = false>
 __device__ __forceinline__ bool face_flux_species_pair(const BlockDev& b, const ChemDev& cd, int d, double eps,
                                                        unsigned f, int right, volatile double* frame,
@@ -421,7 +422,7 @@ __device__ __forceinline__ void cell_update_species(const BlockDev& b, const Che
 // Two lanes per face (face_flux_species_pair): a workgroup of 256 lanes serves 128 faces of
 // one direction of one block (the FaceBatch ranges start at multiples of 256 faces).
 // LMR: Eilmer 5 reconstruction and AUSMDV (face_flux_species_pair).
-// 3 waves per SIMD (168 VGPRs): the compiler fits the kernel there without spilling.
+// 3 waves per SIMD (168 VGPRs), with 0 to 2 registers spilled for 2 species, 11 to 16 for 5.
 template <int DIM, int FC, int NSP, bool LMR>
 __global__ __launch_bounds__(256, 3) void k_face_flux_species_pair(const BlockDev* __restrict__ tab, FaceBatch fb,
                                                                 int nblocks, double eps,
