@@ -116,6 +116,9 @@ struct Sim {
     DevArr<unsigned> ctr;  // the stages' counters, then the control words of queued steps
     StageCounters sc;
     unsigned* ctr_host = nullptr;  // pinned copy of ctr, behind dt_host
+    // A queue of steps was begun and not brought to its end (an error of the runtime): its control
+    // words may still hold a stop.
+    bool queue_open = false;
     // Interior cells of a plane on their way to the host: two pinned buffers of at most PACK_CELLS
     // (4 MiB) each, which the packing kernel and the copy to the caller take in turn.
     static constexpr int64_t PACK_CELLS = (int64_t)1 << 19;
@@ -983,6 +986,8 @@ struct Sim {
     // synchronising.  dt is written to dt_dev first.
     void launch_stage(int stage, double dt) {
         prepare_launches();
+        if (queue_open) HIPCHK(launch_clear_u32(ctl(), 3, stream));
+        queue_open = false;
         HIPCHK(launch_set_f64(dt_dev.p, dt, stream));
         launch_batched_stage(stage, cur, u0);
     }
@@ -1308,6 +1313,7 @@ struct Sim {
         int n = std::min(want, MAX_QUEUED), taken = 0;
         int attempt = 1;  // of the step at the head of the queue
         while (true) {
+            queue_open = true;
             HIPCHK(launch_window_begin(ctl(), dt_dev.p, dt_global, stream));
             if (push_ghost_cells() && !ghosts_ready) {
                 // afterwards the steps' own cell updates keep them (launch_batched_stage)
@@ -1337,6 +1343,7 @@ struct Sim {
             const bool stopped = c[0] != 0;
             const int done = (int)c[1];
             if (stopped) HIPCHK(launch_clear_u32(ctl(), 3, stream));
+            queue_open = false;
             const bool flux_ok = stopped && nf[1] == 0 && nf[2] == 0 && ni[1] <= cfg.max_invalid_cells &&
                                  ni[2] <= cfg.max_invalid_cells;  // then its chemistry failed
             for (int w = 0; w < done + (flux_ok ? 1 : 0); ++w) {
